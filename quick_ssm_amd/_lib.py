@@ -7,12 +7,14 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
 import threading
 from pathlib import Path
 from typing import Optional
 
 LIB_NAME = "libquick_ssm_hip.so"
 LIB_PATH = Path(__file__).resolve().parent / LIB_NAME
+NATIVE_PATH = LIB_PATH.with_name("_qssm_torch.so")
 
 # The QSSM_VERSION of include/quick_ssm_hip.h this binding was written against (same minor version = same ABI).
 QSSM_VERSION = 200
@@ -198,7 +200,7 @@ def _declare(lib: ctypes.CDLL) -> None:
 
 
 def is_built() -> bool:
-    return LIB_PATH.exists()
+    return LIB_PATH.exists() and NATIVE_PATH.exists()
 
 
 def load() -> ctypes.CDLL:
@@ -223,6 +225,31 @@ def load() -> ctypes.CDLL:
             _declare(lib)
             _lib = lib
     return _lib
+
+
+def load_native(take_launch):
+    """The extension module that launches scans for torch tensors (csrc/torch_scan.cpp), set up with `take_launch`
+    (hip_scan._take_launch) and `check`.  Raises RuntimeError if it has not been built."""
+    import importlib.machinery
+    import importlib.util
+
+    load()
+    if not NATIVE_PATH.exists():
+        raise RuntimeError(f"{NATIVE_PATH} is missing: the native launch path is not built. "
+                           "Run `python -m quick_ssm_amd.build`. There is no other device path.")
+    with _lock:
+        name = "quick_ssm_amd._qssm_torch"
+        module = sys.modules.get(name)
+        if module is None:
+            loader = importlib.machinery.ExtensionFileLoader(name, os.fspath(NATIVE_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader(name, loader))
+            loader.exec_module(module)
+            if module.abi_version // 100 != QSSM_VERSION // 100:
+                raise RuntimeError(f"{NATIVE_PATH} was built for version {module.abi_version} of the C ABI, this package "
+                                   f"binds version {QSSM_VERSION}. Rebuild with `python -m quick_ssm_amd.build`.")
+            module.set_hooks(take_launch, check)
+            sys.modules[name] = module
+    return module
 
 
 class launch_stream:

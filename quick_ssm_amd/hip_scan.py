@@ -1,6 +1,6 @@
-"""Host side of the HIP scan: tensor checks, launch planning, workspace, and the two launches.
+"""Host side of the HIP scan: workspace, launch numbering, and the two launches.
 
-Everything here is plumbing around `qssm_scan_forward` / `qssm_scan_backward`
+Everything here and in csrc/torch_scan.cpp (output tensors, plans, the call itself) is plumbing around `qssm_scan_forward` / `qssm_scan_backward`
 (include/quick_ssm_hip.h).  It takes the place of the launch code in the reference's
 `block_scan_forward_3d` (quick_ssm/triton_forwards.py:134-172) and `block_scan_backward_3d`
 (quick_ssm/triton_backwards.py:168-209): no fp32 upcast copies, no N-sized scratch, one launch per
@@ -16,7 +16,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from ._lib import BackwardCall, ForwardCall, Plan, Strides
+from ._lib import Plan
 
 Tensor = torch.Tensor
 
@@ -135,45 +135,6 @@ def _align_elems(tensors: Sequence[Optional[Tensor]], D: int) -> int:
     return 8 if low == 0 or low > 8 else low
 
 
-_ELEM_BYTES = {torch.float32: 4, torch.float16: 2, torch.bfloat16: 2}
-
-
-def _describe(given: Sequence[Optional[Tensor]], fresh: Sequence[Optional[Tensor]], L: int, D: int):
-    """What a launch needs of its tensors, with as few calls into torch as possible (small launches are bound by
-    the host): the caller's tensors made contiguous in their last axis, then strides, base addresses and the
-    alignment in elements (see `_align_elems`) of those and of the freshly allocated, contiguous outputs."""
-    kept, strides, ptrs = [], [], []
-    bits = D
-    for t in given:
-        if t is None:
-            kept.append(None)
-            strides.append(_NO_STRIDE)
-            ptrs.append(None)
-            continue
-        st = t.stride()
-        if st[2] != 1:
-            t = t.contiguous()
-            st = t.stride()
-        ptr = t.data_ptr()
-        es = _ELEM_BYTES[t.dtype]
-        bits |= 1 if ptr % es else (ptr // es) | st[0] | st[1]
-        kept.append(t)
-        strides.append(st)
-        ptrs.append(ptr)
-    out_stride = (L * D, D, 1)
-    for t in fresh:
-        if t is None:
-            strides.append(_NO_STRIDE)
-            ptrs.append(None)
-            continue
-        ptr = t.data_ptr()
-        bits |= (ptr // _ELEM_BYTES[t.dtype]) | out_stride[0]
-        strides.append(out_stride)
-        ptrs.append(ptr)
-    low = bits & -bits
-    return kept, tuple(strides), ptrs, (8 if low == 0 or low > 8 else low)
-
-
 # (device index, stream handle) -> how many `device_counted_launches` contexts are open on it
 _device_counted: Dict[Tuple[int, int], int] = {}
 
@@ -262,8 +223,9 @@ def _recover(buf: _Buffers, stream: int) -> int:
     return status
 
 
-def _launch_buffers(device: torch.device, dev_index: int, stream: int, need_c: int, need_w: int) -> Tuple[_Buffers, int, bool]:
-    """Control block, workspace and epoch argument for the next launch on (device, stream).
+def _number_launch(device: torch.device, dev_index: int, stream: int, need_c: int, need_w: int):
+    """Buffers and number of the next launch on (device, stream): (entry, control, workspace, their addresses and
+    sizes, epoch argument, capturing).
 
     Both buffers are zero-filled when they are allocated (torch.zeros runs a fill kernel on the
     current stream, ahead of the launch that uses them) and grown on demand.  Every launch leaves
@@ -280,7 +242,8 @@ def _launch_buffers(device: torch.device, dev_index: int, stream: int, need_c: i
     key = (dev_index, stream, on_device)
     # Looking the buffers up and taking the next number is one step under the lock: the forward of the next step on
     # the caller's thread and a backward on autograd's thread may launch on one stream at the same time, and two
-    # launches with one number would read each other's words as their own.
+    # launches with one number would read each other's words as their own.  The addresses are read in the same step:
+    # a larger launch on the other thread replaces the tensors, and a number only means something to its own buffers.
     with _ws_lock:
         buf = _buffers.get(key)
         if buf is None or buf.ctl_size < need_c or buf.ws_size < need_w or buf.epoch >= _EPOCH_MAX:
@@ -293,22 +256,49 @@ def _launch_buffers(device: torch.device, dev_index: int, stream: int, need_c: i
             if not on_device:
                 buf.epoch += 1
                 epoch = buf.epoch
+        taken = (buf, buf.control, buf.workspace, buf.ctl_ptr, buf.ctl_size, buf.ws_ptr, buf.ws_size, epoch, capturing)
     if failed:
         raise ScanLaunchError(_recover(buf, stream), buf.where)
-    return buf, epoch, capturing
+    return taken
 
 
-def _after_launch(buf: _Buffers, stream: int, capturing: bool) -> None:
-    """Every `_check_every`-th launch: ask for the status word, to be looked at before a later launch."""
+def _launch_buffers(device: torch.device, dev_index: int, stream: int, need_c: int, need_w: int) -> Tuple[_Buffers, int, bool]:
+    """Entry, epoch argument and whether the stream is capturing, for the next launch on (device, stream)."""
+    taken = _number_launch(device, dev_index, stream, need_c, need_w)
+    return taken[0], taken[7], taken[8]
+
+
+def _status_check_due(buf: _Buffers, capturing: bool) -> bool:
+    """Counts a launch; True behind every `_check_every`-th."""
     if _check_every <= 0 or capturing:
-        return
+        return False
     with _ws_lock:
         buf.since_check += 1
         due = buf.since_check >= _check_every
         if due:
             buf.since_check = 0
-    if due:
+    return due
+
+
+def _after_launch(buf: _Buffers, stream: int, capturing: bool) -> None:
+    """Every `_check_every`-th launch: ask for the status word, to be looked at before a later launch."""
+    if _status_check_due(buf, capturing):
         _lib.check(_lib.load().qssm_control_status_async(buf.ctl_ptr, buf.pinned.data_ptr(), stream))
+
+
+_devices: Dict[int, torch.device] = {}
+
+
+def _take_launch(dev_index: int, stream: int, need_c: int, need_w: int) -> tuple:
+    """What the native launches (csrc/torch_scan.cpp) ask for, from whatever thread they run on: the addresses and
+    sizes of control block and workspace, the epoch argument, the pinned word the status is to be copied to behind this
+    launch (0: not this time), and the two tensors, which the caller holds until the launch is on its stream."""
+    device = _devices.get(dev_index)
+    if device is None:
+        device = _devices[dev_index] = torch.device("cuda", dev_index)
+    buf, control, workspace, cp, cs, wp, ws, epoch, capturing = _number_launch(device, dev_index, stream, need_c, need_w)
+    status_to = buf.pinned.data_ptr() if _status_check_due(buf, capturing) else 0
+    return cp, cs, wp, ws, epoch, status_to, control, workspace
 
 
 def workspace_status(device: Optional[torch.device] = None, all_streams: bool = False) -> int:
@@ -378,59 +368,14 @@ def make_plan(B: int, L: int, D: int, in_dtype: torch.dtype, out_dtype: torch.dt
     return plan
 
 
-class _Launch:
-    """A ready-made argument block for one (direction, shape, storage, alignment, geometry): the plan, what the
-    host needs from it as plain ints, and the ctypes block whose pointers a call patches."""
-
-    __slots__ = ("plan", "call", "call_ref", "need_c", "need_w", "n_ckpt", "ckpt_stride", "strides")
-
-    def __init__(self, plan: Plan, call):
-        self.plan = plan
-        self.call = call
-        self.call_ref = ctypes.byref(call)
-        call.plan = ctypes.pointer(plan)
-        self.need_c = int(plan.control_bytes)
-        self.need_w = int(plan.workspace_bytes)
-        self.n_ckpt = int(plan.n_ckpt)
-        self.ckpt_stride = int(plan.ckpt_stride)
-        self.strides = None   # the stride tuples the block's stride fields were last filled from
+_native = None
 
 
-_tls = threading.local()   # argument blocks are patched in place, so every thread keeps its own
-
-
-def _launch_entry(key: tuple, make) -> _Launch:
-    cache = getattr(_tls, "launches", None)
-    if cache is None:
-        cache = _tls.launches = {}
-    entry = cache.get(key)
-    if entry is None:
-        if len(cache) >= 1024:
-            cache.clear()
-        entry = cache[key] = make()
-    return entry
-
-
-def _require_gpu(*tensors: Tensor) -> torch.device:
-    dev = tensors[0].device
-    for t in tensors:
-        if t.device.type != "cuda":
-            raise RuntimeError("HIP scan backend requires GPU tensors.")
-        if t.device != dev:
-            raise RuntimeError("all scan operands must live on one GPU")
-    return dev
-
-
-def _check_state(t: Optional[Tensor], B: int, D: int, dev: torch.device, name: str) -> None:
-    """A carried state / its gradient: fp32 [B, D], contiguous, on the operands' device."""
-    if t is None:
-        return
-    if tuple(t.shape) != (B, D) or t.dtype != torch.float32 or not t.is_contiguous() or t.device != dev:
-        raise ValueError(f"{name} must be a contiguous float32 tensor of shape {(B, D)} on {dev}, "
-                         f"got {t.dtype} {tuple(t.shape)} on {t.device}")
-
-
-_NO_STRIDE = (0, 0, 0)
+def _load_native():
+    """csrc/torch_scan.cpp's module, with the two callables it works with."""
+    global _native
+    _native = _lib.load_native(_take_launch)
+    return _native
 
 
 def scan_forward(
@@ -451,68 +396,11 @@ def scan_forward(
     `want_ckpt` (what the backward rebuilds h from).  `h_init` (fp32 [B, D], contiguous) is the
     state before the first step instead of zero; `h_final` (same layout) receives h(L-1).
     """
-    dev = _require_gpu(x, a, b) if c is None else _require_gpu(x, a, b, c)
-    B, L, D = x.shape
-    in_dtype = x.dtype
-    y = torch.empty((B, L, D), dtype=out_dtype, device=dev) if want_y else None
-    h = torch.empty((B, L, D), dtype=torch.float32, device=dev) if want_h else None
-    if h_init is not None or h_final is not None:
-        _check_state(h_init, B, D, dev, "h_init")
-        _check_state(h_final, B, D, dev, "h_final")
-    if B == 0 or L == 0 or D == 0:
-        if h_final is not None:  # nothing happened to the state
-            h_final.copy_(h_init) if h_init is not None else h_final.zero_()
-        return y, h, (torch.empty((B, 0, D), dtype=torch.float32, device=dev) if want_ckpt else None), 0
-
-    (x, a, b, c), strides, ptrs, align = _describe((x, a, b, c), (y, h), L, D)
-
     # Operands are left in the caches only for a backward: a forward that saves no states has none coming.
     keep = _forward_keep if (want_ckpt or want_h) else False
-
-    def make() -> _Launch:
-        stride = 0
-        if want_ckpt:
-            # The backward decides how far apart the saved states may be; the forward follows.
-            stride = make_plan(B, L, D, in_dtype, out_dtype, _lib.QSSM_BACKWARD, align, 0, bwd_tune).seg_len
-        plan = make_plan(B, L, D, in_dtype, out_dtype, _lib.QSSM_FORWARD, align, stride, tune)
-        if keep is not True:
-            plan = Plan.from_buffer_copy(plan)   # cached plans are shared: change a copy
-            plan.keep_tiles = 0 if keep is False else min(int(plan.keep_tiles), int(keep))
-        return _Launch(plan, ForwardCall())
-
-    entry = _launch_entry((0, B, L, D, in_dtype, out_dtype, align, want_ckpt, tune, bwd_tune, keep), make)
-    ckpt = torch.empty((B, entry.n_ckpt, D), dtype=torch.float32, device=dev) if want_ckpt else None
-
-    k = entry.call
-    if entry.strides != strides:
-        k.sx, k.sa, k.sb, k.sc, k.sy, k.sh = (Strides(s[0], s[1]) for s in strides)
-        entry.strides = strides
-    k.x, k.a, k.b, k.c, k.y, k.h_out = ptrs
-    k.ckpt = None if ckpt is None else ckpt.data_ptr()
-    k.h_init = None if h_init is None else h_init.data_ptr()
-    k.h_final = None if h_final is None else h_final.data_ptr()
-
-    index = dev.index
-    if index == torch.cuda.current_device():
-        _launch_on(index, dev, entry, _lib.load().qssm_scan_forward_call)
-    else:
-        with torch.cuda.device(dev):
-            _launch_on(index, dev, entry, _lib.load().qssm_scan_forward_call)
-    return y, h, ckpt, entry.ckpt_stride
-
-
-def _launch_on(index: int, dev: torch.device, entry: _Launch, fn) -> None:
-    """Fill in stream, buffers and epoch of a ready argument block and make the call (device `index` is current)."""
-    stream = _raw_stream(index)
-    buf, epoch, capturing = _launch_buffers(dev, index, stream, entry.need_c, entry.need_w)
-    k = entry.call
-    k.control, k.control_size, k.workspace, k.workspace_bytes = buf.ctl_ptr, buf.ctl_size, buf.ws_ptr, buf.ws_size
-    k.epoch = epoch
-    k.stream = stream
-    rc = fn(entry.call_ref)
-    if rc != 0:
-        _lib.check(rc)
-    _after_launch(buf, stream, capturing)
+    native = _native or _load_native()
+    return native.scan_forward(x, a, b, c, _DTYPE_CODE[out_dtype], want_y | want_h << 1 | want_ckpt << 2,
+                               -1 if keep is True else int(keep), tune, bwd_tune, h_init, h_final)
 
 
 def scan_backward(
@@ -533,53 +421,19 @@ def scan_backward(
     `h_init` is the state the forward started from, `dh_final` the gradient arriving at h(L-1),
     `dh_init` receives the gradient of h(-1); all fp32 [B, D], contiguous, optional.
     """
-    dev = _require_gpu(x, a, b, c, dy)
-    B, L, D = x.shape
-    in_dtype = x.dtype
-    grads = [torch.empty((B, L, D), dtype=in_dtype, device=dev) if n else None for n in need]
-    if h_init is not None or dh_final is not None or dh_init is not None:
-        for name, t in (("h_init", h_init), ("dh_final", dh_final), ("dh_init", dh_init)):
-            _check_state(t, B, D, dev, name)
-    if B == 0 or L == 0 or D == 0:
-        if dh_init is not None:  # the state passed through untouched
-            dh_init.copy_(dh_final) if dh_final is not None else dh_init.zero_()
-        return tuple(grads)
-    if (h is None) == (ckpt is None):
-        raise ValueError("pass exactly one of h and ckpt")
+    native = _native or _load_native()
+    mask = sum(1 << i for i, n in enumerate(need) if n)
+    return native.scan_backward(x, a, b, c, dy, h, ckpt, ckpt_stride, mask, tune, h_init, dh_final, dh_init)
 
-    if h is not None:
-        if h.dtype != torch.float32:
-            h = h.float()
-    elif not ckpt.is_contiguous():
-        ckpt = ckpt.contiguous()
-    (x, a, b, c, dy, h), strides, ptrs, align = _describe((x, a, b, c, dy, h), grads, L, D)
-    stride_arg = ckpt_stride if h is None else 0
-    out_dtype = dy.dtype
 
-    def make() -> _Launch:
-        return _Launch(make_plan(B, L, D, in_dtype, out_dtype, _lib.QSSM_BACKWARD, align, stride_arg, tune), BackwardCall())
-
-    entry = _launch_entry((1, B, L, D, in_dtype, out_dtype, align, stride_arg, tune), make)
-    if ckpt is not None and tuple(ckpt.shape) != (B, entry.n_ckpt, D):
-        raise ValueError(f"ckpt has shape {tuple(ckpt.shape)}, expected {(B, entry.n_ckpt, D)}")
-
-    k = entry.call
-    if entry.strides != strides:
-        (k.sx, k.sa, k.sb, k.sc, k.sdy, k.sh, k.sdx, k.sda, k.sdb, k.sdc) = (Strides(s[0], s[1]) for s in strides)
-        entry.strides = strides
-    k.x, k.a, k.b, k.c, k.dy, k.h, k.dx, k.da, k.db, k.dc = ptrs
-    k.ckpt = None if ckpt is None else ckpt.data_ptr()
-    k.h_init = None if h_init is None else h_init.data_ptr()
-    k.dh_final = None if dh_final is None else dh_final.data_ptr()
-    k.dh_init = None if dh_init is None else dh_init.data_ptr()
-
-    index = dev.index
-    if index == torch.cuda.current_device():
-        _launch_on(index, dev, entry, _lib.load().qssm_scan_backward_call)
-    else:
-        with torch.cuda.device(dev):
-            _launch_on(index, dev, entry, _lib.load().qssm_scan_backward_call)
-    return tuple(grads)
+def attach(y: Tensor, h: Optional[Tensor], ckpt: Optional[Tensor], stride: int, x: Tensor, a: Tensor, b: Tensor,
+           c: Tensor, k_in: torch.dtype, k_out: torch.dtype, h_final: Optional[Tensor] = None,
+           state: Optional[Tensor] = None, h_init: Optional[Tensor] = None) -> None:
+    """Make `y` (and `h_final`) the outputs of an autograd node over the operands (and the incoming `state`): what
+    `scan_forward` computed and kept, with the operands as the caller gave them and the storage types of the launch.
+    `h_init` is the state the launch started from."""
+    native = _native or _load_native()
+    native.attach_scan(y, h, ckpt, stride, x, a, b, c, _DTYPE_CODE[k_in], _DTYPE_CODE[k_out], h_final, state, h_init)
 
 
 def block_scan_forward_3d(x: Tensor, a: Tensor, b: Tensor, BLOCK_L: int = 256) -> Tuple[Tensor, Tensor]:

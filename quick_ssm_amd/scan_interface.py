@@ -65,7 +65,8 @@ def _launch_tiles(shape, tile_b, tile_d) -> List[Tuple[slice, slice]]:
 
 
 class _HipScanFunction(torch.autograd.Function):
-    """Autograd node of the device scan: one HIP launch forward, one backward.
+    """Autograd node of the device scan that can loop over tiles (`honor_tiles`); without them `scan` takes
+    `_device_scan`, the same two launches behind a native node.
 
     Argument list, saved state and returned gradients follow the reference's
     `_TritonScanFunction` (quick_ssm/scan_interface.py:49-158): forward takes
@@ -168,75 +169,70 @@ def _torch_scan(x: Tensor, a: Tensor, b: Tensor, c: Tensor, out_dtype: torch.dty
     return (c * h).to(out_dtype)
 
 
-class _HipScanCarryFunction(torch.autograd.Function):
-    """Autograd node of the device scan with a carried state: (x, a, b, c, h_init) -> (y, h_final).
+def _check_operands(x: Tensor, a: Tensor, b: Tensor, c: Tensor) -> None:
+    shape = x.shape
+    if shape != a.shape or shape != b.shape or shape != c.shape:
+        raise ValueError("x, a, b, c must share the same shape [B, L, D].")
+    if len(shape) != 3:
+        raise ValueError("x, a, b, c must be 3-D tensors [B, L, D].")
+    if not x.is_cuda:
+        raise RuntimeError("HIP scan backend requires GPU tensors.")
 
-    One HIP launch forward, one backward, like `_HipScanFunction`; the backward also takes the
-    gradient arriving at h_final and returns the gradient of h_init, so pieces of a sequence
-    chain through autograd exactly as the whole sequence would.
-    """
 
-    @staticmethod
-    def forward(ctx, x: Tensor, a: Tensor, b: Tensor, c: Tensor, h_init: Optional[Tensor], checkpoint: bool,
-                out_dtype: torch.dtype):
-        if x.shape != a.shape or x.shape != b.shape or x.shape != c.shape:
-            raise ValueError("x, a, b, c must share the same shape [B, L, D].")
-        if x.dim() != 3:
-            raise ValueError("x, a, b, c must be 3-D tensors [B, L, D].")
-        if x.device.type != "cuda":
-            raise RuntimeError("HIP scan backend requires GPU tensors.")
-        B, L, D = x.shape
-        if h_init is not None and tuple(h_init.shape) != (B, D):
-            raise ValueError(f"state must have shape {(B, D)}, got {tuple(h_init.shape)}.")
-        k_in, k_out = hip_scan.kernel_dtypes([x.dtype, a.dtype, b.dtype, c.dtype], out_dtype)
-        xs, as_, bs, cs = (t if t.dtype == k_in else t.to(k_in) for t in (x, a, b, c))
-        h0 = None
-        if h_init is not None:
-            h0 = h_init.detach().to(torch.float32).contiguous()
-            if h0.data_ptr() % 16 != 0:
-                h0 = h0.clone()
-        h_final = torch.empty((B, D), dtype=torch.float32, device=x.device)
-        train = any(ctx.needs_input_grad[:5])   # generation mode saves no states and leaves nothing in the caches
-        y, h_full, ckpt, stride = hip_scan.scan_forward(
-            xs, as_, bs, cs, out_dtype=k_out, want_h=train and not checkpoint, want_ckpt=train and bool(checkpoint),
-            h_init=h0, h_final=h_final,
-        )
-        ctx.save_for_backward(x, a, b, c)
-        ctx.k_in, ctx.k_out = k_in, k_out
-        ctx.h0, ctx.h_saved, ctx.ckpt, ctx.stride = h0, h_full, ckpt, stride
-        ctx.state_dtype = None if h_init is None else h_init.dtype
-        return (y if y.dtype == out_dtype else y.to(out_dtype)), h_final
+def _kernel_operands(x: Tensor, a: Tensor, b: Tensor, c: Tensor, out_dtype: torch.dtype):
+    """The operands in the one storage type of the launch, and the storage types of the launch."""
+    k_in, k_out = hip_scan.kernel_dtypes((x.dtype, a.dtype, b.dtype, c.dtype), out_dtype)
+    if not (x.dtype == a.dtype == b.dtype == c.dtype == k_in):
+        with torch.no_grad():
+            x, a, b, c = (t if t.dtype == k_in else t.to(k_in) for t in (x, a, b, c))
+    return x, a, b, c, k_in, k_out
 
-    @staticmethod
-    def backward(ctx, grad_y: Optional[Tensor], grad_state: Optional[Tensor]):
-        x, a, b, c = ctx.saved_tensors
-        k_in, k_out = ctx.k_in, ctx.k_out
-        B, L, D = x.shape
-        xs, as_, bs, cs = (t if t.dtype == k_in else t.to(k_in) for t in (x, a, b, c))
-        if grad_y is None:
-            grad_y = torch.zeros((B, L, D), dtype=k_out, device=x.device)
-        dy = grad_y if grad_y.dtype == k_out else grad_y.to(k_out)
-        dh_final = None
-        if grad_state is not None:
-            dh_final = grad_state.to(torch.float32).contiguous()
-            if dh_final.data_ptr() % 16 != 0:
-                dh_final = dh_final.clone()
-        need = tuple(ctx.needs_input_grad[:4])
-        dh_init = None
-        if ctx.needs_input_grad[4]:
-            dh_init = torch.empty((B, D), dtype=torch.float32, device=x.device)
-        out = hip_scan.scan_backward(
-            xs, as_, bs, cs, dy, h=ctx.h_saved, ckpt=None if ctx.h_saved is not None else ctx.ckpt,
-            ckpt_stride=ctx.stride, need=need, h_init=ctx.h0, dh_final=dh_final, dh_init=dh_init,
-        )
 
-        def _as(g: Optional[Tensor], like_dtype) -> Optional[Tensor]:
-            if g is None:
-                return None
-            return g if g.dtype == like_dtype else g.to(like_dtype)
+def _device_scan(x: Tensor, a: Tensor, b: Tensor, c: Tensor, checkpoint: bool, out_dtype: torch.dtype) -> Tensor:
+    """One launch over the whole tensor; with gradients on, y is the output of a native autograd node that makes one
+    launch backward (csrc/torch_scan.cpp)."""
+    _check_operands(x, a, b, c)
+    # No operand wants a gradient (inference, torch.no_grad()): no backward will come, so no state is saved and
+    # the launch streams its operands past the caches.
+    train = torch.is_grad_enabled() and (x.requires_grad or a.requires_grad or b.requires_grad or c.requires_grad)
+    xs, as_, bs, cs, k_in, k_out = _kernel_operands(x, a, b, c, out_dtype)
+    y, h, ckpt, stride = hip_scan.scan_forward(xs, as_, bs, cs, out_dtype=k_out, want_h=train and not checkpoint,
+                                               want_ckpt=train and bool(checkpoint))
+    if k_out != out_dtype:
+        y = y.to(out_dtype)
+    if train:
+        hip_scan.attach(y, h, ckpt, stride, x, a, b, c, k_in, k_out)
+    return y
 
-        return (_as(out[0], x.dtype), _as(out[1], a.dtype), _as(out[2], b.dtype), _as(out[3], c.dtype),
-                _as(dh_init, ctx.state_dtype), None, None)
+
+def _device_scan_chunk(x: Tensor, a: Tensor, b: Tensor, c: Tensor, state: Optional[Tensor], checkpoint: bool,
+                       out_dtype: torch.dtype) -> Tuple[Tensor, Tensor]:
+    """`_device_scan` with a carried state: the backward also takes the gradient arriving at the final state and
+    returns the gradient of the incoming one, so pieces of a sequence chain through autograd exactly as the whole
+    sequence would."""
+    _check_operands(x, a, b, c)
+    B, _, D = x.shape
+    if state is not None and tuple(state.shape) != (B, D):
+        raise ValueError(f"state must have shape {(B, D)}, got {tuple(state.shape)}.")
+    train = torch.is_grad_enabled() and (x.requires_grad or a.requires_grad or b.requires_grad or c.requires_grad
+                                         or (state is not None and state.requires_grad))
+    xs, as_, bs, cs, k_in, k_out = _kernel_operands(x, a, b, c, out_dtype)
+    h0 = None
+    if state is not None:
+        h0 = state.detach()
+        if h0.dtype != torch.float32 or not h0.is_contiguous():
+            h0 = h0.to(torch.float32).contiguous()
+        if h0.data_ptr() % 16 != 0:
+            h0 = h0.clone()
+    h_final = torch.empty((B, D), dtype=torch.float32, device=x.device)
+    # generation mode saves no states and leaves nothing in the caches
+    y, h, ckpt, stride = hip_scan.scan_forward(xs, as_, bs, cs, out_dtype=k_out, want_h=train and not checkpoint,
+                                               want_ckpt=train and bool(checkpoint), h_init=h0, h_final=h_final)
+    if k_out != out_dtype:
+        y = y.to(out_dtype)
+    if train:
+        hip_scan.attach(y, h, ckpt, stride, x, a, b, c, k_in, k_out, h_final, state, h0)
+    return y, h_final
 
 
 def scan_chunk(
@@ -265,7 +261,7 @@ def scan_chunk(
     if backend == "auto":
         chosen = "hip" if x.device.type == "cuda" else "torch"
     if chosen in ("hip", "triton"):
-        return _HipScanCarryFunction.apply(x, a, b, c, state, checkpoint, out_dtype)
+        return _device_scan_chunk(x, a, b, c, state, checkpoint, out_dtype)
     if chosen == "torch":
         h, final = naive_forward_3d(x, a, b, h_init=state, return_final=True)
         return (c * h).to(out_dtype), final
@@ -301,7 +297,9 @@ def scan(
     if backend == "auto":
         chosen = "hip" if x.device.type == "cuda" else "torch"
     if chosen in ("hip", "triton"):
-        return _HipScanFunction.apply(x, a, b, c, block_l, checkpoint, tile_b, tile_d, out_dtype)
+        if _HONOR_TILES:
+            return _HipScanFunction.apply(x, a, b, c, block_l, checkpoint, tile_b, tile_d, out_dtype)
+        return _device_scan(x, a, b, c, checkpoint, out_dtype)
     if chosen == "torch":
         return _torch_scan(x, a, b, c, out_dtype)
     raise ValueError(f"Unsupported backend '{backend}'. Use 'auto', 'hip', 'triton', or 'torch'.")

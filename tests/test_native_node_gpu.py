@@ -1,0 +1,57 @@
+"""The native autograd node of scan() and scan_chunk(): what autograd promises beyond the values of the gradients."""
+import pytest
+import torch
+
+from helpers import TOL, assert_close, make_inputs, oracle_all
+from quick_ssm_amd import hip_scan, scan, scan_chunk
+
+pytestmark = pytest.mark.gpu
+
+
+def test_a_graph_is_walked_once_unless_kept_and_frees_what_it_saved(gpu):
+    x, a, b, c, dy = make_inputs((2, 300, 24), seed=5)
+    ref = oracle_all(x, a, b, c, dy)
+    leaves = [t.to(gpu).requires_grad_(True) for t in (x, a, b, c)]
+    y = scan(*leaves, checkpoint=False)
+    first = torch.autograd.grad(y, leaves, dy.to(gpu), retain_graph=True)
+    second = torch.autograd.grad(y, leaves, dy.to(gpu))
+    for name, g1, g2 in zip(("dx", "da", "db", "dc"), first, second):
+        assert torch.equal(g1, g2), name
+        assert_close(name, g1.cpu(), ref[name], TOL[torch.float32])
+    assert y.grad_fn.h_saved is None
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(y, leaves, dy.to(gpu))
+    y = scan(*leaves)
+    with torch.no_grad():
+        leaves[1].mul_(0.5)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward(dy.to(gpu))
+
+
+@pytest.mark.parametrize("used", ["y", "state", "both"])
+@pytest.mark.parametrize("dtypes", [(torch.float32,) * 4, (torch.float16, torch.float32, torch.bfloat16, torch.float64)],
+                         ids=["f32", "mixed"])
+def test_either_output_of_a_piece_may_go_unused(gpu, used, dtypes):
+    x, a, b, c, dy = make_inputs((3, 90, 20), seed=8)
+    st, dst = torch.randn(3, 20, generator=torch.Generator().manual_seed(1)), torch.ones(3, 20)
+    ops = [t.to(d) for t, d in zip((x, a, b, c), dtypes)] + [st.half() if dtypes[0] != torch.float32 else st]
+
+    def grads(backend, device):
+        leaves = [t.to(device).requires_grad_(True) for t in ops]
+        ins = leaves if backend == "hip" else [t.double() for t in leaves]
+        y, h = scan_chunk(*ins, out_dtype=torch.float32 if backend == "hip" else torch.float64, backend=backend)
+        loss = 0.0
+        if used != "state":
+            loss = loss + (y * dy.to(y)).sum()
+        if used != "y":
+            loss = loss + (h * dst.to(h)).sum()
+        return torch.autograd.grad(loss, leaves, allow_unused=True)
+
+    for name, got, want in zip(("dx", "da", "db", "dc", "dstate"), grads("hip", gpu), grads("torch", "cpu")):
+        if want is None:          # c when only the state is used
+            assert got is None or not bool(got.any()), name
+            continue
+        assert got.dtype == want.dtype, name
+        # float32 arithmetic, one rounding to the operand's own type
+        assert_close(name, got.cpu().float(), want.float().numpy(), max(1e-5, torch.finfo(got.dtype).eps))
+    assert hip_scan.workspace_status() == 0
