@@ -471,6 +471,49 @@ QSSM_API int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int
                          int32_t partial_rows, void* out, void* stream);
 
 /*
+ * fp32 products on the 16-bit matrix cores: C_i(m, n) = sum over k of A_i(m, k) B_i(n, k) (+ bias_i(n)) for up to
+ * QSSM_SPLIT_MANY products of one shape, or the sum of up to QSSM_SPLIT_MANY runs of K k's as one product
+ * (`batch` = 1, `segments` > 1; C, bias and the maxima are then entry 0's).  Every operand element is used as the sum
+ * of two fp16 values scaled by a power of two per row of A and of B, three products per pair of elements are
+ * accumulated in fp32, and the scales leave exactly; error against fp32 products: at or below theirs.  Infinities and
+ * NaN reach the result as in fp32 arithmetic.  Results repeat bit for bit.
+ *   a, lda   A_i(m, k) = a[m * lda + k], or a[k * lda + m] with `a_kstrided` (then b must be k-strided too)
+ *   b, ldb   B_i(n, k) = b[n * ldb + k], or b[k * ldb + n] with `b_kstrided`
+ *   amax_a   [M] words of qssm_split_amax over the rows of A_i (over all runs of k), amax_b [N] of B_i
+ * N and the leading dimensions are multiples of 4, K too unless both operands are k-strided; a, b and c are 16-byte
+ * aligned.  `partial` is fp32 scratch of splits * batch * M * N floats when splits > 1 (qssm_split_gemm_splits names
+ * the number of parts that suits the launch; 1 is always right).
+ * These are the layer's projections (quick_ssm/layers.py:76-80,106) and what autograd records for them when the
+ * parameters are fp32.
+ */
+#define QSSM_SPLIT_MANY 5
+typedef struct {
+  const float *a[QSSM_SPLIT_MANY], *b[QSSM_SPLIT_MANY];
+  float* c[QSSM_SPLIT_MANY];
+  const float* bias[QSSM_SPLIT_MANY];
+  const uint32_t *amax_a[QSSM_SPLIT_MANY], *amax_b[QSSM_SPLIT_MANY];
+  int64_t lda, ldb, ldc;
+  int32_t M, N, K, batch, segments, splits, a_kstrided, b_kstrided;
+  float* partial;
+  uint64_t partial_floats;
+} qssm_split_gemm_call;
+QSSM_API int qssm_split_gemm(const qssm_split_gemm_call* call, void* stream);
+QSSM_API int qssm_split_gemm_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments);
+
+/*
+ * Bits of the largest absolute value in every row and every column of `count` fp32 matrices of one shape (up to
+ * QSSM_SPLIT_MANY; row stride ld and cols multiples of 4, 16-byte aligned), for qssm_split_gemm.  row[i] ([rows]) and
+ * col[i] ([cols]) may be NULL and may be shared between matrices; they only grow, so the caller clears them first.
+ */
+typedef struct {
+  const float* x[QSSM_SPLIT_MANY];
+  uint32_t *row[QSSM_SPLIT_MANY], *col[QSSM_SPLIT_MANY];
+  int64_t rows, ld;
+  int32_t cols, count;
+} qssm_split_amax_call;
+QSSM_API int qssm_split_amax(const qssm_split_amax_call* call, void* stream);
+
+/*
  * Streaming copy of `bytes` bytes (16-byte aligned, multiple of 16) on `stream`.  Not part of
  * the scan: it is the known-size kernel against which rocprof's FETCH_SIZE / WRITE_SIZE
  * counters and the achievable-bandwidth ceiling are calibrated by the benchmark.

@@ -91,6 +91,9 @@ static const int kMaxLdsBytes = 64 * 1024;
 static const int kCUs = 256;
 static const uint64_t kKeepBytes = 224ull << 20;  // operand bytes a forward leaves in the caches for its backward
 
+static const double kSplitPartCost = 0.0125;       // stages of the split GEMM that one more MB of partial sums costs
+static const int kSplitStageK = 16;
+
 static bool threads_ok(int t) { return t == 256 || t == 512 || t == 1024; }
 
 static int check_plan(const qssm_plan* pl, int direction) {
@@ -927,6 +930,92 @@ int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int32_t dtyp
     return fail(QSSM_EINVAL, "column sum for storage type %d is not built", dtype);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : hip_fail(e, "colsum kernel launch");
+}
+
+int qssm_split_gemm_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments) {
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || segments <= 0) return 1;
+  // Two workgroups per compute unit run at once.  A launch takes whole rounds of them, each as long as its stages of
+  // 16 k's (plus about 24 stages' worth to fill and drain a workgroup); every further part writes and reads C once
+  // more, which costs about as much as 1 / 40 of a round per 2 MB.
+  const double tiles = (double)split_gemm_tiles(M, N, batch), stages = (double)split_gemm_stages(K, segments);
+  const double out_mb = (double)M * N * batch * 4e-6;
+  int best = 1;
+  double best_cost = 0.0;
+  for (int s = 1; s <= 32 && (s == 1 || stages / s >= 16.0); ++s) {
+    const double rounds = (double)(int64_t)((tiles * s + 2 * kCUs - 1) / (2 * kCUs));
+    const double cost = rounds * (stages / s + 24.0) + (s > 1 ? (s + 1) * out_mb * kSplitPartCost : 0.0);
+    if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
+  }
+  return best;
+}
+
+int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
+  if (k == nullptr) return fail(QSSM_EINVAL, "call is NULL");
+  if (k->M < 0 || k->N < 0 || k->K < 1) return fail(QSSM_EINVAL, "bad dimension");
+  if (k->batch < 1 || k->batch > QSSM_SPLIT_MANY || k->segments < 1 || k->segments > QSSM_SPLIT_MANY ||
+      (k->batch > 1 && k->segments > 1))
+    return fail(QSSM_EINVAL, "1 to %d products, or runs of k of one product", QSSM_SPLIT_MANY);
+  if (k->splits < 1 || k->splits > 64) return fail(QSSM_EINVAL, "splits must be 1 to 64");
+  if (k->a_kstrided && !k->b_kstrided) return fail(QSSM_EINVAL, "a k-strided A needs a k-strided B");
+  if (k->M == 0 || k->N == 0) return 0;
+  if (k->N % 4 != 0 || k->lda % 4 != 0 || k->ldb % 4 != 0 || k->ldc % 4 != 0 ||
+      (k->K % 4 != 0 && !(k->a_kstrided && k->b_kstrided)))
+    return fail(QSSM_EALIGN, "N, K and the leading dimensions must be multiples of 4");
+  if (k->lda < (k->a_kstrided ? k->M : k->K) || k->ldb < (k->b_kstrided ? k->N : k->K) || k->ldc < k->N)
+    return fail(QSSM_EINVAL, "a leading dimension is below its row");
+  if (k->lda >= (1 << 20) || k->ldb >= (1 << 20)) return fail(QSSM_EINVAL, "a leading dimension is too large for 32-bit tile offsets");
+  const uint64_t floats = k->splits > 1 ? (uint64_t)k->splits * k->batch * k->M * k->N : 0;
+  if (floats > 0 && (k->partial == nullptr || k->partial_floats < floats || ((uintptr_t)k->partial) % 16 != 0))
+    return fail(QSSM_EWORKSPACE, "partial needs %llu floats, 16-byte aligned", (unsigned long long)floats);
+  SplitGemmArgs p;
+  memset(&p, 0, sizeof(p));
+  const int pairs = k->batch > k->segments ? k->batch : k->segments;
+  for (int i = 0; i < pairs; ++i) {
+    if (k->a[i] == nullptr || k->b[i] == nullptr) return fail(QSSM_EINVAL, "NULL operand");
+    if (((uintptr_t)k->a[i]) % 16 != 0 || ((uintptr_t)k->b[i]) % 16 != 0) return fail(QSSM_EALIGN, "operands must be 16-byte aligned");
+    p.a[i] = k->a[i];
+    p.b[i] = k->b[i];
+  }
+  for (int i = 0; i < k->batch; ++i) {
+    if (k->c[i] == nullptr || k->amax_a[i] == nullptr || k->amax_b[i] == nullptr) return fail(QSSM_EINVAL, "NULL result or maxima");
+    if (((uintptr_t)k->c[i]) % 16 != 0) return fail(QSSM_EALIGN, "results must be 16-byte aligned");
+    p.c[i] = k->c[i];
+    p.bias[i] = k->bias[i];
+    p.amax_a[i] = k->amax_a[i];
+    p.amax_b[i] = k->amax_b[i];
+  }
+  p.lda = k->lda; p.ldb = k->ldb; p.ldc = k->ldc;
+  p.M = k->M; p.N = k->N; p.K = k->K;
+  p.batch = k->batch; p.segments = k->segments; p.splits = k->splits;
+  p.partial = k->partial;
+  if (split_gemm_tiles(p.M, p.N, p.batch) * p.splits > 0x7fffffffll || split_gemm_stages(p.K, p.segments) * kSplitStageK > 0x7fffffffll ||
+      (int64_t)p.M * p.N / 4 * p.batch > 0x7fffffffll * 128)
+    return fail(QSSM_EINVAL, "product too large for one launch");
+  if (!launch_split_gemm(p, k->a_kstrided != 0, k->b_kstrided != 0, (hipStream_t)stream))
+    return fail(QSSM_EINVAL, "operand layout is not built");
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : hip_fail(e, "split_gemm_kernel launch");
+}
+
+int qssm_split_amax(const qssm_split_amax_call* k, void* stream) {
+  if (k == nullptr) return fail(QSSM_EINVAL, "call is NULL");
+  if (k->rows < 0 || k->cols < 0) return fail(QSSM_EINVAL, "negative dimension");
+  if (k->count < 1 || k->count > QSSM_SPLIT_MANY) return fail(QSSM_EINVAL, "1 to %d matrices", QSSM_SPLIT_MANY);
+  if (k->rows == 0 || k->cols == 0) return 0;
+  if (k->cols % 4 != 0 || k->ld % 4 != 0 || k->ld < k->cols) return fail(QSSM_EALIGN, "cols and ld must be multiples of 4, ld >= cols");
+  if (k->rows > 0x7fffffffll || k->cols > 65535 * 1024ll) return fail(QSSM_EINVAL, "matrix too large for one launch");
+  AmaxArgs p;
+  memset(&p, 0, sizeof(p));
+  for (int i = 0; i < k->count; ++i) {
+    if (k->x[i] == nullptr || ((uintptr_t)k->x[i]) % 16 != 0) return fail(QSSM_EALIGN, "matrices must be there and 16-byte aligned");
+    p.x[i] = k->x[i];
+    p.row[i] = k->row[i];
+    p.col[i] = k->col[i];
+  }
+  p.rows = k->rows; p.ld = k->ld; p.cols = k->cols;
+  launch_amax(p, k->count, (hipStream_t)stream);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : hip_fail(e, "amax_kernel launch");
 }
 
 int qssm_launch_count_step(uint32_t count, int32_t static_scratch, uint32_t* flag, uint32_t* next, int32_t* wipes) {

@@ -559,4 +559,34 @@ bool launch_norm_any(int dtype, const NormFwdArgs* f, const NormBwdArgs* b, int 
 bool launch_colsum_any(int dtype, const void* x, int64_t ld, int64_t rows, int S, int vec, float* partial, int chunks,
                        void* out, hipStream_t stream);
 
+// ---- fp32 products on the 16-bit matrix cores (gemm_split.hip) -----------------------------------------------------
+constexpr int kSplitGemmMany = 5;   // products (or runs of k) of one launch
+
+struct SplitGemmArgs {
+  const float *a[kSplitGemmMany], *b[kSplitGemmMany];  // one pair per product, or per run of k
+  float* c[kSplitGemmMany];                             // [M, N], row stride ldc
+  const float* bias[kSplitGemmMany];                    // [N] or null
+  const unsigned *amax_a[kSplitGemmMany], *amax_b[kSplitGemmMany];  // [M] and [N]: bits of the rows' largest magnitudes
+  int64_t lda, ldb, ldc;
+  int M, N, K;
+  int batch;       // products
+  int segments;    // runs of K k's that make up one product (batch is 1 when there are several)
+  int splits;      // parts the k's are dealt to
+  float* partial;  // [splits][batch][M][N] when there are several
+};
+
+struct AmaxArgs {
+  const float* x[kSplitGemmMany];  // [rows, cols], row stride ld
+  unsigned* row[kSplitGemmMany];   // [rows] or null; several matrices may share one
+  unsigned* col[kSplitGemmMany];   // [cols] or null
+  int64_t rows, ld;
+  int cols;
+  int rows_per_block;              // set by the launch
+};
+
+int64_t split_gemm_tiles(int64_t M, int64_t N, int64_t batch);
+int64_t split_gemm_stages(int64_t K, int64_t segments);
+bool launch_split_gemm(const SplitGemmArgs& args, bool a_kstrided, bool b_kstrided, hipStream_t stream);
+void launch_amax(const AmaxArgs& args, int count, hipStream_t stream);
+
 }  // namespace qssm

@@ -1,7 +1,8 @@
 """`SSM` and `RMSNorm`: the layer that feeds the scan.
 
 Same constructor arguments, parameter names (so state dicts interchange) and forward keywords as
-the reference's quick_ssm/layers.py:9-107.  The projections stay on torch GEMMs; the gate
+the reference's quick_ssm/layers.py:9-107.  The projections are torch GEMMs, except over fp32
+parameters, where they are split products on the 16-bit matrix cores (quick_ssm_amd/split_linear.py); the gate
 activations and casts between them and the scan happen inside the scan's own launches when the
 projections are stored as the 16-bit compute dtype (quick_ssm_amd/gated_scan.py) and are one fused HIP
 pass otherwise (quick_ssm_amd/gates.py),
@@ -19,6 +20,7 @@ import torch.nn as nn
 from . import _lib
 from . import gated_scan as _gated
 from . import scan_interface as _scan_interface
+from . import split_linear
 from .gates import gate_prologue, gate_prologue_wide
 from .norm import rms_norm
 from .scan_interface import scan
@@ -57,21 +59,47 @@ def column_sum(g2: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _products(ctx, u: torch.Tensor, weights, biases):
+    """u w^T + bias for every weight, inside an autograd function's forward: split products where they apply (the
+    maxima the backward wants are saved in `ctx.maxima`), else torch's."""
+    u2 = u.reshape(-1, u.shape[-1])
+    if not split_linear.usable(u2, weights):
+        ctx.maxima = None
+        return [torch.nn.functional.linear(u, w, b) for w, b in zip(weights, biases)]
+    outs, ctx.maxima = split_linear.forward(u2, weights, biases, ctx.needs_input_grad[0], any(ctx.needs_input_grad[1:]))
+    return [t.view(*u.shape[:-1], t.shape[-1]) for t in outs]
+
+
+def _product_gradients(ctx, grads, u: torch.Tensor, weights, need_du: bool, need_dw: bool):
+    """Gradients of the input and of the weights from the outputs' gradients ([rows, N] each).  A backward that is
+    itself recorded (create_graph) takes torch's products, which autograd can follow."""
+    u2 = u.reshape(-1, u.shape[-1])
+    if ctx.maxima is not None and not torch.is_grad_enabled():
+        du, dws = split_linear.backward(grads, u2, weights, ctx.maxima, need_du, need_dw)
+        return (None if du is None else du.view_as(u)), dws
+    du = None
+    if need_du:
+        du = grads[0] @ weights[0]
+        for g, w in zip(grads[1:], weights[1:]):
+            du = du + g @ w
+        du = du.view_as(u)
+    return du, [g.t() @ u2 if need_dw else None for g in grads]
+
+
 class _LinearBias(torch.autograd.Function):
     """u @ weight^T + bias, as `torch.nn.functional.linear`, with the bias gradient from `column_sum`."""
 
     @staticmethod
     def forward(ctx, u, weight, bias):
         ctx.save_for_backward(u, weight)
-        return torch.nn.functional.linear(u, weight, bias)
+        return _products(ctx, u, [weight], [bias])[0]
 
     @staticmethod
     def backward(ctx, g):
         u, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
         g2 = g.reshape(-1, g.shape[-1])
-        du = (g2 @ weight).view_as(u) if need[0] else None
-        dw = g2.t() @ u.reshape(-1, u.shape[-1]) if need[1] else None
+        du, (dw,) = _product_gradients(ctx, [g2], u, [weight], need[0], need[1])
         db = column_sum(g2) if need[2] else None
         return du, dw, db
 
@@ -85,7 +113,7 @@ class _PackedProjection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, w_a, w_b, w_ca, w_cb, w_d, bias_a, wide_w, wide_b):
         ctx.save_for_backward(u, wide_w)
-        return torch.nn.functional.linear(u, wide_w, wide_b)
+        return _products(ctx, u, [wide_w], [wide_b])[0]
 
     @staticmethod
     def backward(ctx, g):
@@ -93,13 +121,36 @@ class _PackedProjection(torch.autograd.Function):
         need = ctx.needs_input_grad
         S = wide_w.shape[0] // 5
         g2 = g.reshape(-1, g.shape[-1])
-        du = (g2 @ wide_w).view_as(u) if need[0] else None
-        blocks = [None] * 5
-        if any(need[1:6]):
-            dw = g2.t() @ u.reshape(-1, u.shape[-1])                              # [5 S, H]
-            blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
+        du, (dw,) = _product_gradients(ctx, [g2], u, [wide_w], need[0], any(need[1:6]))      # dw: [5 S, H]
+        blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
         dbias = column_sum(g2[:, :S]) if need[6] else None
         return (du, *blocks, dbias, None, None)
+
+
+class _SplitProjections(torch.autograd.Function):
+    """The five projections of a layer with fp32 parameters as one launch: the outputs share the input's maxima, the
+    input's gradient is one product over 5 S k's instead of five products and four additions, and the five weight
+    gradients are one launch."""
+
+    @staticmethod
+    def forward(ctx, u, w_a, w_b, w_ca, w_cb, w_d, bias_a):
+        ctx.save_for_backward(u, w_a, w_b, w_ca, w_cb, w_d)
+        return tuple(_products(ctx, u, [w_a, w_b, w_ca, w_cb, w_d], [bias_a, None, None, None, None]))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        u, *weights = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        gs = [g.reshape(-1, g.shape[-1]) for g in grads]
+        du, dws = _product_gradients(ctx, gs, u, weights, need[0], any(need[1:6]))
+        dbias = column_sum(gs[0]) if need[6] else None
+        return (du, *(dw if need[1 + k] else None for k, dw in enumerate(dws)), dbias)
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """An `nn.Linear` whose call does nothing but the product: no hooks, no replaced class or forward."""
+    return (type(m) is nn.Linear and "forward" not in m.__dict__ and type(m.weight) is nn.Parameter
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
 
 
 class SSM(nn.Module):
@@ -182,6 +233,15 @@ class SSM(nn.Module):
         return _PackedProjection.apply(u, self.A_proj.weight, self.B_proj.weight, self.C_proj_a.weight,
                                        self.C_proj_b.weight, self.D_proj.weight, self.A_proj.bias, wide_w, wide_b)
 
+    def _five_projections(self, u: torch.Tensor):
+        """The five projection outputs of a large layer (blocks in A, B, C_a, C_b, D order)."""
+        mods = (self.A_proj, self.B_proj, self.C_proj_a, self.C_proj_b, self.D_proj)
+        if (all(_plain_linear(m) for m in mods) and not nn.modules.module._has_any_global_hook()
+                and split_linear.usable(u.reshape(-1, u.shape[-1]), [m.weight for m in mods])
+                and self.A_proj.bias is not None and all(m.bias is None for m in mods[1:])):
+            return _SplitProjections.apply(u, *(m.weight for m in mods), self.A_proj.bias)
+        return tuple(m(u) for m in mods)
+
     def gates(self, u: torch.Tensor):
         """The scan's four operands (x, a, b, c) from the normalised input, in `compute_dtype`."""
         forget, drive, out_gate, in_gate = gate_prologue(
@@ -219,7 +279,7 @@ class SSM(nn.Module):
                 S = self.state_size_dim
                 pre = tuple(wide[..., k * S:(k + 1) * S] for k in range(5))
             else:
-                pre = (self.A_proj(u), self.B_proj(u), self.C_proj_a(u), self.C_proj_b(u), self.D_proj(u))
+                pre = self._five_projections(u)
             if wide is not None and wide.dim() == 3 and _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
                 y = _gated.gated_scan_wide(wide, out_dtype=out_dtype, compute_dtype=self.compute_dtype)
             elif _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
