@@ -479,7 +479,7 @@ QSSM_API int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int
  * NaN reach the result as in fp32 arithmetic.  Results repeat bit for bit.
  *   a, lda   A_i(m, k) = a[m * lda + k], or a[k * lda + m] with `a_kstrided` (then b must be k-strided too)
  *   b, ldb   B_i(n, k) = b[n * ldb + k], or b[k * ldb + n] with `b_kstrided`
- *   amax_a   [M] words of qssm_split_amax over the rows of A_i (over all runs of k), amax_b [N] of B_i
+ *   amax_a   words of qssm_split_amax over the rows of A_i (over all runs of k), [parts_a][M]; amax_b of B_i, [parts_b][N]
  * N and the leading dimensions are multiples of 4, K too unless both operands are k-strided; a, b and c are 16-byte
  * aligned.  `partial` is fp32 scratch of splits * batch * M * N floats when splits > 1 (qssm_split_gemm_splits names
  * the number of parts that suits the launch; 1 is always right).
@@ -493,7 +493,7 @@ typedef struct {
   const float* bias[QSSM_SPLIT_MANY];
   const uint32_t *amax_a[QSSM_SPLIT_MANY], *amax_b[QSSM_SPLIT_MANY];
   int64_t lda, ldb, ldc;
-  int32_t M, N, K, batch, segments, splits, a_kstrided, b_kstrided;
+  int32_t M, N, K, batch, segments, splits, a_kstrided, b_kstrided, parts_a, parts_b;
   float* partial;
   uint64_t partial_floats;
 } qssm_split_gemm_call;
@@ -501,17 +501,20 @@ QSSM_API int qssm_split_gemm(const qssm_split_gemm_call* call, void* stream);
 QSSM_API int qssm_split_gemm_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments);
 
 /*
- * Bits of the largest absolute value in every row and every column of `count` fp32 matrices of one shape (up to
- * QSSM_SPLIT_MANY; row stride ld and cols multiples of 4, 16-byte aligned), for qssm_split_gemm.  row[i] ([rows]) and
- * col[i] ([cols]) may be NULL and may be shared between matrices; they only grow, so the caller clears them first.
+ * Bits of the largest absolute value in the rows and columns of `count` fp32 matrices (up to QSSM_SPLIT_MANY + 1; row
+ * strides and cols multiples of 4, 16-byte aligned), for qssm_split_gemm.  A matrix is taken in blocks, and each writes
+ * words of its own: row is [row_parts][rows] and col [col_parts][cols], or NULL, with the numbers of parts that
+ * qssm_split_amax_parts gives for the matrix's shape (a row's largest is the largest of its parts).  Parts of several
+ * matrices laid one behind the other make the maxima over all of them.
  */
 typedef struct {
-  const float* x[QSSM_SPLIT_MANY];
-  uint32_t *row[QSSM_SPLIT_MANY], *col[QSSM_SPLIT_MANY];
+  const float* x;
+  uint32_t *row, *col;
   int64_t rows, ld;
-  int32_t cols, count;
-} qssm_split_amax_call;
-QSSM_API int qssm_split_amax(const qssm_split_amax_call* call, void* stream);
+  int32_t cols, reserved;
+} qssm_split_amax_matrix;
+QSSM_API int qssm_split_amax(const qssm_split_amax_matrix* matrices, int32_t count, void* stream);
+QSSM_API int qssm_split_amax_parts(int64_t rows, int32_t cols, int32_t* row_parts, int32_t* col_parts);
 
 /*
  * Streaming copy of `bytes` bytes (16-byte aligned, multiple of 16) on `stream`.  Not part of

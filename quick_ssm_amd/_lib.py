@@ -51,6 +51,7 @@ EXPORTED_SYMBOLS = (
     "qssm_split_gemm",
     "qssm_split_gemm_splits",
     "qssm_split_amax",
+    "qssm_split_amax_parts",
     "qssm_copy_bytes",
     "qssm_launch_count_step",
 )
@@ -120,29 +121,6 @@ class BackwardCall(ctypes.Structure):
         + [("control", ctypes.c_void_p), ("control_size", ctypes.c_uint64), ("workspace", ctypes.c_void_p),
            ("workspace_bytes", ctypes.c_uint64), ("epoch", ctypes.c_uint32), ("reserved", ctypes.c_uint32),
            ("stream", ctypes.c_void_p)]
-    )
-
-
-SPLIT_MANY = 5
-
-
-class SplitGemmCall(ctypes.Structure):
-    """Mirror of `qssm_split_gemm_call`."""
-
-    _fields_ = (
-        [(n, ctypes.c_void_p * SPLIT_MANY) for n in ("a", "b", "c", "bias", "amax_a", "amax_b")]
-        + [(n, ctypes.c_int64) for n in ("lda", "ldb", "ldc")]
-        + [(n, ctypes.c_int32) for n in ("M", "N", "K", "batch", "segments", "splits", "a_kstrided", "b_kstrided")]
-        + [("partial", ctypes.c_void_p), ("partial_floats", ctypes.c_uint64)]
-    )
-
-
-class SplitAmaxCall(ctypes.Structure):
-    """Mirror of `qssm_split_amax_call`."""
-
-    _fields_ = (
-        [(n, ctypes.c_void_p * SPLIT_MANY) for n in ("x", "row", "col")]
-        + [("rows", ctypes.c_int64), ("ld", ctypes.c_int64), ("cols", ctypes.c_int32), ("count", ctypes.c_int32)]
     )
 
 
@@ -218,12 +196,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.qssm_rmsnorm_backward.argtypes = [vp, i64, vp, i64, vp, vp, vp, vp, vp, i32, i64, i32, ctypes.c_float, i32, vp]
     lib.qssm_colsum.restype = ctypes.c_int
     lib.qssm_colsum.argtypes = [vp, i64, i64, i32, i32, vp, i32, vp, vp]
-    lib.qssm_split_gemm.restype = ctypes.c_int
-    lib.qssm_split_gemm.argtypes = [ctypes.POINTER(SplitGemmCall), vp]
     lib.qssm_split_gemm_splits.restype = ctypes.c_int
     lib.qssm_split_gemm_splits.argtypes = [i32] * 5
-    lib.qssm_split_amax.restype = ctypes.c_int
-    lib.qssm_split_amax.argtypes = [ctypes.POINTER(SplitAmaxCall), vp]
     lib.qssm_copy_bytes.restype = ctypes.c_int
     lib.qssm_copy_bytes.argtypes = [vp, vp, u64, vp]
     lib.qssm_launch_count_step.restype = ctypes.c_int

@@ -54,7 +54,7 @@ struct Fetch {
   int slot[U];       // where its halves go in a plane
   int kh[U];         // first k of the unit inside the stage
 
-  __device__ __forceinline__ void place(int row0, int n_rows, int64_t ld, const unsigned* amax) {
+  __device__ __forceinline__ void place(int row0, int n_rows, int64_t ld, const int* exps) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int idx = (int)threadIdx.x + 256 * u;
@@ -63,7 +63,7 @@ struct Fetch {
       off[u] = KSTRIDED ? (uint32_t)((half * 8) * (int)ld + r) * 4u : (uint32_t)(r * (int)ld + half * 8) * 4u;
       slot[u] = lds_at(row, half);
       kh[u] = half * 8;
-      scale[u] = exp2_int(scale_exp(amax[row0 + r]));
+      scale[u] = exp2_int(exps[row]);
     }
   }
   // `base` points at (k0, row0); `left` = k's from k0 to the end.
@@ -137,9 +137,6 @@ __global__ void __launch_bounds__(256, 2) split_gemm_kernel(const SplitGemmArgs 
 
   const int stages_per = (p.K + kBK - 1) / kBK, stages = stages_per * p.segments;
   const int s_begin = (int)((int64_t)stages * split / p.splits), s_end = (int)((int64_t)stages * (split + 1) / p.splits);
-  const unsigned* amax_a = p.amax_a[prob];
-  const unsigned* amax_b = p.amax_b[prob];
-
   float16v acc[4][2];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -149,17 +146,35 @@ __global__ void __launch_bounds__(256, 2) split_gemm_kernel(const SplitGemmArgs 
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
   const int wm = (wave >> 1) * 128, wn = (wave & 1) * 64;
-  const int ma = m0 + tid < p.M ? m0 + tid : p.M - 1;
-  const int nb = n0 + (tid & 127) < p.N ? n0 + (tid & 127) : p.N - 1;
-  const bool special = __syncthreads_or(amax_a[ma] >= kInfBits || amax_b[nb] >= kInfBits) != 0;
+  // Exponents of the tile's 256 rows of A and 128 rows of B, from the parts of their maxima (rows past the end have the
+  // last one's).
+  __shared__ int exps[kBM + kBN];
+  auto largest = [](const unsigned* words, int parts, int64_t stride) {
+    unsigned m = 0;
+#pragma unroll 16
+    for (int k = 0; k < parts; ++k) {
+      const unsigned w = words[k * stride];
+      m = m > w ? m : w;
+    }
+    return m;
+  };
+  const unsigned amax_a = largest(p.amax_a[prob] + (m0 + tid < p.M ? m0 + tid : p.M - 1), p.parts_a, p.M);
+  exps[tid] = scale_exp(amax_a);
+  bool odd = amax_a >= kInfBits;
+  if (tid < kBN) {
+    const unsigned amax_b = largest(p.amax_b[prob] + (n0 + tid < p.N ? n0 + tid : p.N - 1), p.parts_b, p.N);
+    exps[kBM + tid] = scale_exp(amax_b);
+    odd = odd || amax_b >= kInfBits;
+  }
+  const bool special = __syncthreads_or(odd) != 0;
 
   // where the operands of a stage start
   int seg = s_begin / stages_per, k0 = (s_begin - seg * stages_per) * kBK;
   if (!special) {
     Fetch<AKS, kBM> fa;
     Fetch<BKS, kBN> fb;
-    fa.place(m0, p.M, p.lda, amax_a);
-    fb.place(n0, p.N, p.ldb, amax_b);
+    fa.place(m0, p.M, p.lda, exps);
+    fb.place(n0, p.N, p.ldb, exps + kBM);
     int next = s_begin;   // the stage the next load takes; after the last one it is taken again, and never used
     const int a_step = AKS ? kBK * (int)p.lda : kBK, b_step = BKS ? kBK * (int)p.ldb : kBK;   // elements
     const float *a, *b;
@@ -268,9 +283,6 @@ __global__ void __launch_bounds__(256, 2) split_gemm_kernel(const SplitGemmArgs 
   }
 
   // ---- take the scales off and store ---------------------------------------------------------------------------
-  int* sE = reinterpret_cast<int*>(lds);   // the last stage has been read: the loop ends on a barrier
-  sE[tid] = special ? 0 : -scale_exp(amax_a[ma]);
-  lds_barrier();
   float* c = p.splits > 1 ? p.partial + ((int64_t)split * p.batch + prob) * p.M * p.N : p.c[prob];
   const int64_t ldc = p.splits > 1 ? p.N : p.ldc;
   const float* bias = p.splits > 1 ? nullptr : p.bias[prob];
@@ -278,7 +290,7 @@ __global__ void __launch_bounds__(256, 2) split_gemm_kernel(const SplitGemmArgs 
   for (int j = 0; j < 2; ++j) {
     const int n = n0 + wn + j * 32 + (lane & 31);
     if (n >= p.N) continue;
-    const int eb = special ? 0 : -scale_exp(amax_b[n]);
+    const int eb = exps[kBM + wn + j * 32 + (lane & 31)];
     const float bn = bias != nullptr ? bias[n] : 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -288,7 +300,7 @@ __global__ void __launch_bounds__(256, 2) split_gemm_kernel(const SplitGemmArgs 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int m = m0 + row + r;
-          const float v = ldexpf(acc[i][j][q * 4 + r], sE[row + r] + eb);
+          const float v = special ? acc[i][j][q * 4 + r] : ldexpf(acc[i][j][q * 4 + r], -(exps[row + r] + eb));
           if (m < p.M) c[(int64_t)m * ldc + n] = bias != nullptr ? v + bn : v;
         }
       }
@@ -313,59 +325,76 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const SplitGemmArgs p
   *reinterpret_cast<float4v*>(p.c[prob] + m * p.ldc + n) = s;
 }
 
-// Largest magnitude (as the bits of its absolute value, which order like integers, NaN above infinity) of every row
-// and every column of up to five matrices.  A wavefront takes rows of 1024 columns, 16 to a lane; its columns' maxima
-// stay in registers over the workgroup's rows.  The words start from zero and only grow, so a word that already holds
-// as much needs no atomic (a stale look only costs one).
-__global__ void __launch_bounds__(256) amax_kernel(const AmaxArgs p) {
-  __shared__ unsigned cols_lds[4][1024];
+// Largest magnitude (as the bits of its absolute value, which order like integers, NaN above infinity) of the rows and
+// columns of a block of one of the matrices.  A workgroup takes `block_rows` rows of 256 * Q columns, a quarter of the
+// rows per wavefront; its columns' maxima stay in registers over the rows.  Every block writes words of its own, and the
+// product that reads them takes the largest: no atomics and nothing to clear beforehand.  Bound by memory: eight 16-byte
+// loads per lane are in flight.
+template <int Q>
+__device__ __forceinline__ void amax_block(const AmaxMatrix& x, int block, unsigned (*cols_lds)[1024]) {
+  constexpr int RU = 8 / Q;   // rows at a time
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c0 = blockIdx.y * 1024;
-  const int64_t r0 = (int64_t)blockIdx.x * p.rows_per_block;
-  const int64_t r1 = r0 + p.rows_per_block < p.rows ? r0 + p.rows_per_block : p.rows;
-  const float* x = p.x[blockIdx.z];
-  unsigned* row_out = p.row[blockIdx.z];
-  unsigned* col_out = p.col[blockIdx.z];
-  uint4v cm[4];
+  const int cb = block % x.col_blocks, rb = block / x.col_blocks;
+  const int c0 = cb * (256 * Q);
+  const int per_wave = x.block_rows / 4;   // a multiple of 8
+  const int64_t r0 = (int64_t)rb * x.block_rows + wave * per_wave;
+  uint4v cm[Q];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) cm[q] = (uint4v)(0u);
-#pragma unroll 2
-  for (int64_t r = r0 + wave; r < r1; r += 4) {
-    unsigned rm = 0;
+  for (int q = 0; q < Q; ++q) cm[q] = (uint4v)(0u);
+  for (int k = 0; k < per_wave; k += RU) {
+    if (r0 + k >= x.rows) break;
+    uint4v v[RU][Q];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c = c0 + q * 256 + lane * 4;
-      if (c < p.cols) {
-        const uint4v v = *reinterpret_cast<const uint4v*>(x + r * p.ld + c) & 0x7fffffffu;
+    for (int i = 0; i < RU; ++i) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          cm[q][i] = cm[q][i] > v[i] ? cm[q][i] : v[i];
-          rm = rm > v[i] ? rm : v[i];
+      for (int q = 0; q < Q; ++q) {
+        const int c = c0 + q * 256 + lane * 4;
+        v[i][q] = (uint4v)(0u);
+        if (c < x.cols && r0 + k + i < x.rows) v[i][q] = *reinterpret_cast<const uint4v*>(x.x + (r0 + k + i) * x.ld + c);
+      }
+    }
+    unsigned mine = 0;
+#pragma unroll
+    for (int i = 0; i < RU; ++i) {
+      unsigned rm = 0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned m = v[i][q][e] & 0x7fffffffu;
+          cm[q][e] = cm[q][e] > m ? cm[q][e] : m;
+          rm = rm > m ? rm : m;
         }
       }
-    }
-    if (row_out != nullptr) {
+      if (x.row != nullptr) {
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const unsigned other = (unsigned)__shfl_xor((int)rm, o, 64);
-        rm = rm > other ? rm : other;
+        for (int o = 32; o > 0; o >>= 1) {
+          const unsigned other = (unsigned)__shfl_xor((int)rm, o, 64);
+          rm = rm > other ? rm : other;
+        }
+        if (lane == i) mine = rm;
       }
-      if (lane == 0 && rm != 0)
-        __hip_atomic_fetch_max(row_out + r, rm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    if (x.row != nullptr && lane < RU && r0 + k + lane < x.rows) x.row[(int64_t)cb * x.rows + r0 + k + lane] = mine;
   }
-  if (col_out == nullptr) return;
+  if (x.col == nullptr) return;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) *reinterpret_cast<uint4v*>(&cols_lds[wave][q * 256 + lane * 4]) = cm[q];
+  for (int q = 0; q < Q; ++q) *reinterpret_cast<uint4v*>(&cols_lds[wave][q * 256 + lane * 4]) = cm[q];
   __syncthreads();
-  for (int c = threadIdx.x; c < 1024 && c0 + c < p.cols; c += 256) {
+  for (int c = threadIdx.x; c < 256 * Q && c0 + c < x.cols; c += 256) {
     unsigned m = cols_lds[0][c];
 #pragma unroll
     for (int w = 1; w < 4; ++w) m = m > cols_lds[w][c] ? m : cols_lds[w][c];
-    unsigned* out = col_out + c0 + c;
-    if (m > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      __hip_atomic_fetch_max(out, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    x.col[(int64_t)rb * x.cols + c0 + c] = m;
   }
+}
+
+__global__ void __launch_bounds__(256) amax_kernel(const AmaxArgs p) {
+  __shared__ __align__(16) unsigned cols_lds[4][1024];
+  int block = blockIdx.x, k = 0;
+  while (block >= p.m[k].blocks) block -= p.m[k++].blocks;   // the grid has as many workgroups as all matrices have blocks
+  if (p.m[k].wide) amax_block<4>(p.m[k], block, cols_lds);
+  else amax_block<1>(p.m[k], block, cols_lds);
 }
 
 }  // namespace
@@ -396,15 +425,23 @@ bool launch_split_gemm(const SplitGemmArgs& p, bool a_kstrided, bool b_kstrided,
   return true;
 }
 
-void launch_amax(const AmaxArgs& given, int count, hipStream_t stream) {
-  AmaxArgs p = given;
-  const int col_blocks = (p.cols + 1023) / 1024;
-  // about eight workgroups per compute unit, at least 16 rows each
-  int64_t rows = (p.rows * col_blocks * count + 2047) / 2048;
-  rows = rows < 16 ? 16 : (rows + 3) / 4 * 4;
-  p.rows_per_block = (int)(rows > 4096 ? 4096 : rows);
-  const dim3 grid((unsigned)((p.rows + p.rows_per_block - 1) / p.rows_per_block), (unsigned)col_blocks, (unsigned)count);
-  hipLaunchKernelGGL(amax_kernel, grid, dim3(256), 0, stream, p);
+// Blocks of 256 columns, or 1024 where that would make more than 32 of them, and of at least 128 rows, at most 64 of
+// those: few enough words for a product to look through before it starts, and a few hundred workgroups for every matrix
+// that is worth the launch.
+void amax_shape(int64_t rows, int cols, AmaxMatrix* m) {
+  m->wide = cols > 2048 && (cols > 8192 || rows >= 16384);
+  const int width = m->wide ? 1024 : 256;
+  m->col_blocks = (cols + width - 1) / width;
+  const int64_t per = rows < 128 * 64 ? 128 : (rows + 63) / 64;
+  m->block_rows = (int)((per + 31) / 32 * 32);
+  m->row_blocks = (int)((rows + m->block_rows - 1) / m->block_rows);
+  m->blocks = m->row_blocks * m->col_blocks;
+}
+
+void launch_amax(const AmaxArgs& p, int count, hipStream_t stream) {
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) blocks += p.m[i].blocks;
+  hipLaunchKernelGGL(amax_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, p);
 }
 
 }  // namespace qssm

@@ -988,6 +988,8 @@ int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
   p.M = k->M; p.N = k->N; p.K = k->K;
   p.batch = k->batch; p.segments = k->segments; p.splits = k->splits;
   p.partial = k->partial;
+  p.parts_a = k->parts_a; p.parts_b = k->parts_b;
+  if (p.parts_a < 1 || p.parts_b < 1) return fail(QSSM_EINVAL, "the maxima have at least one part");
   if (split_gemm_tiles(p.M, p.N, p.batch) * p.splits > 0x7fffffffll || split_gemm_stages(p.K, p.segments) * kSplitStageK > 0x7fffffffll ||
       (int64_t)p.M * p.N / 4 * p.batch > 0x7fffffffll * 128)
     return fail(QSSM_EINVAL, "product too large for one launch");
@@ -997,23 +999,32 @@ int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
   return e == hipSuccess ? 0 : hip_fail(e, "split_gemm_kernel launch");
 }
 
-int qssm_split_amax(const qssm_split_amax_call* k, void* stream) {
-  if (k == nullptr) return fail(QSSM_EINVAL, "call is NULL");
-  if (k->rows < 0 || k->cols < 0) return fail(QSSM_EINVAL, "negative dimension");
-  if (k->count < 1 || k->count > QSSM_SPLIT_MANY) return fail(QSSM_EINVAL, "1 to %d matrices", QSSM_SPLIT_MANY);
-  if (k->rows == 0 || k->cols == 0) return 0;
-  if (k->cols % 4 != 0 || k->ld % 4 != 0 || k->ld < k->cols) return fail(QSSM_EALIGN, "cols and ld must be multiples of 4, ld >= cols");
-  if (k->rows > 0x7fffffffll || k->cols > 65535 * 1024ll) return fail(QSSM_EINVAL, "matrix too large for one launch");
+int qssm_split_amax_parts(int64_t rows, int32_t cols, int32_t* row_parts, int32_t* col_parts) {
+  if (row_parts == nullptr || col_parts == nullptr) return fail(QSSM_EINVAL, "NULL argument");
+  if (rows < 1 || cols < 1 || rows > 0x7fffffffll || cols > (1 << 26)) return fail(QSSM_EINVAL, "bad dimension");
+  AmaxMatrix m;
+  amax_shape(rows, cols, &m);
+  *row_parts = m.col_blocks;
+  *col_parts = m.row_blocks;
+  return 0;
+}
+
+int qssm_split_amax(const qssm_split_amax_matrix* matrices, int32_t count, void* stream) {
+  if (matrices == nullptr) return fail(QSSM_EINVAL, "matrices is NULL");
+  if (count < 1 || count > QSSM_SPLIT_MANY + 1) return fail(QSSM_EINVAL, "1 to %d matrices", QSSM_SPLIT_MANY + 1);
   AmaxArgs p;
   memset(&p, 0, sizeof(p));
-  for (int i = 0; i < k->count; ++i) {
-    if (k->x[i] == nullptr || ((uintptr_t)k->x[i]) % 16 != 0) return fail(QSSM_EALIGN, "matrices must be there and 16-byte aligned");
-    p.x[i] = k->x[i];
-    p.row[i] = k->row[i];
-    p.col[i] = k->col[i];
+  for (int i = 0; i < count; ++i) {
+    const qssm_split_amax_matrix& g = matrices[i];
+    if (g.rows < 1 || g.cols < 1 || g.rows > 0x7fffffffll || g.cols > (1 << 26)) return fail(QSSM_EINVAL, "bad dimension");
+    if (g.cols % 4 != 0 || g.ld % 4 != 0 || g.ld < g.cols) return fail(QSSM_EALIGN, "cols and ld must be multiples of 4, ld >= cols");
+    if (g.x == nullptr || ((uintptr_t)g.x) % 16 != 0) return fail(QSSM_EALIGN, "matrices must be there and 16-byte aligned");
+    AmaxMatrix& m = p.m[i];
+    amax_shape(g.rows, g.cols, &m);
+    m.x = g.x; m.row = g.row; m.col = g.col;
+    m.rows = g.rows; m.ld = g.ld; m.cols = g.cols;
   }
-  p.rows = k->rows; p.ld = k->ld; p.cols = k->cols;
-  launch_amax(p, k->count, (hipStream_t)stream);
+  launch_amax(p, count, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : hip_fail(e, "amax_kernel launch");
 }

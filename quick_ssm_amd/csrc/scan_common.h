@@ -566,7 +566,9 @@ struct SplitGemmArgs {
   const float *a[kSplitGemmMany], *b[kSplitGemmMany];  // one pair per product, or per run of k
   float* c[kSplitGemmMany];                             // [M, N], row stride ldc
   const float* bias[kSplitGemmMany];                    // [N] or null
-  const unsigned *amax_a[kSplitGemmMany], *amax_b[kSplitGemmMany];  // [M] and [N]: bits of the rows' largest magnitudes
+  // bits of the rows' largest magnitudes, [parts_a][M] and [parts_b][N]: a row's is the largest of its parts
+  const unsigned *amax_a[kSplitGemmMany], *amax_b[kSplitGemmMany];
+  int parts_a, parts_b;
   int64_t lda, ldb, ldc;
   int M, N, K;
   int batch;       // products
@@ -575,18 +577,22 @@ struct SplitGemmArgs {
   float* partial;  // [splits][batch][M][N] when there are several
 };
 
-struct AmaxArgs {
-  const float* x[kSplitGemmMany];  // [rows, cols], row stride ld
-  unsigned* row[kSplitGemmMany];   // [rows] or null; several matrices may share one
-  unsigned* col[kSplitGemmMany];   // [cols] or null
+struct AmaxMatrix {
+  const float* x;          // [rows, cols], row stride ld
+  unsigned *row, *col;     // [col_blocks][rows], [row_blocks][cols], or null
   int64_t rows, ld;
   int cols;
-  int rows_per_block;              // set by the launch
+  int wide, col_blocks, row_blocks, block_rows, blocks;   // from amax_shape
+};
+
+struct AmaxArgs {
+  AmaxMatrix m[kSplitGemmMany + 1];
 };
 
 int64_t split_gemm_tiles(int64_t M, int64_t N, int64_t batch);
 int64_t split_gemm_stages(int64_t K, int64_t segments);
 bool launch_split_gemm(const SplitGemmArgs& args, bool a_kstrided, bool b_kstrided, hipStream_t stream);
+void amax_shape(int64_t rows, int cols, AmaxMatrix* m);
 void launch_amax(const AmaxArgs& args, int count, hipStream_t stream);
 
 }  // namespace qssm
