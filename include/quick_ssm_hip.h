@@ -90,6 +90,8 @@ typedef struct qssm_plan {
   int32_t compute_dtype;  /* gated scans: the type the layer rounds its gates' outputs to (its compute dtype): the
                              projections' storage type, or QSSM_F16 / QSSM_BF16 for fp32 projections.  Plain scans:
                              in_dtype. */
+  int32_t element_aligned; /* 1: addresses and strides need the alignment of one element only and D need not be a
+                              multiple of vec (qssm_plan_scan_loose); 0: both are multiples of vec elements */
   uint64_t control_bytes;   /* control block the launch needs (status word + ticket counters) */
   uint64_t workspace_bytes; /* workspace the launch needs (words exchanged between workgroups) */
   uint64_t ckpt_elems;      /* B * n_ckpt * D floats */
@@ -127,6 +129,15 @@ QSSM_API int qssm_plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, i
  * No counterpart in the reference.
  */
 QSSM_API int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype,
+                         int32_t direction, int32_t align_elems, int32_t ckpt_stride, int32_t tune,
+                         qssm_plan* plan);
+
+/*
+ * qssm_plan_scan_tuned for tensors whose rows are not all aligned to the lanes' width, or not divided by it: from 32
+ * columns on such plans keep 8 or 16 bytes per lane at element alignment (`element_aligned`), where the other planners
+ * narrow the lanes to `align_elems` columns.  The same plan as theirs for everything else.
+ */
+QSSM_API int qssm_plan_scan_loose(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype,
                          int32_t direction, int32_t align_elems, int32_t ckpt_stride, int32_t tune,
                          qssm_plan* plan);
 

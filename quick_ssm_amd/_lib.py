@@ -29,6 +29,7 @@ EXPORTED_SYMBOLS = (
     "qssm_error_string",
     "qssm_plan_scan",
     "qssm_plan_scan_tuned",
+    "qssm_plan_scan_loose",
     "qssm_zero_fill",
     "qssm_control_status",
     "qssm_control_status_async",
@@ -82,6 +83,7 @@ class Plan(ctypes.Structure):
         ("lds_bytes", ctypes.c_int32),
         ("keep_tiles", ctypes.c_int32),
         ("compute_dtype", ctypes.c_int32),
+        ("element_aligned", ctypes.c_int32),
         ("control_bytes", ctypes.c_uint64),
         ("workspace_bytes", ctypes.c_uint64),
         ("ckpt_elems", ctypes.c_uint64),
@@ -144,6 +146,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.qssm_plan_scan.argtypes = [i32] * 8 + [ctypes.POINTER(Plan)]
     lib.qssm_plan_scan_tuned.restype = ctypes.c_int
     lib.qssm_plan_scan_tuned.argtypes = [i32] * 9 + [ctypes.POINTER(Plan)]
+    lib.qssm_plan_scan_loose.restype = ctypes.c_int
+    lib.qssm_plan_scan_loose.argtypes = [i32] * 9 + [ctypes.POINTER(Plan)]
     lib.qssm_control_status_async.restype = ctypes.c_int
     lib.qssm_control_status_async.argtypes = [vp, vp, vp]
     lib.qssm_scan_forward_call.restype = ctypes.c_int

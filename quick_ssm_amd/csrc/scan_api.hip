@@ -94,6 +94,8 @@ static const uint64_t kKeepBytes = 224ull << 20;  // operand bytes a forward lea
 static const double kSplitPartCost = 0.0125;       // stages of the split GEMM that one more MB of partial sums costs
 static const int kSplitStageK = 16;
 
+static const int kLooseColumns = 32;
+
 static bool threads_ok(int t) { return t == 256 || t == 512 || t == 1024; }
 
 static int check_plan(const qssm_plan* pl, int direction) {
@@ -105,7 +107,9 @@ static int check_plan(const qssm_plan* pl, int direction) {
   if (pl->steps != 4 && pl->steps != 8) return fail(QSSM_EINVAL, "plan.steps must be 4 or 8");
   if (!threads_ok(pl->threads)) return fail(QSSM_EINVAL, "plan.threads must be 256, 512 or 1024");
   if (pl->g_log2 < 0 || (1 << pl->g_log2) > pl->threads) return fail(QSSM_EINVAL, "plan.g_log2 out of range");
-  if (pl->D % pl->vec != 0) return fail(QSSM_EALIGN, "D=%d is not a multiple of plan.vec=%d", pl->D, pl->vec);
+  if (pl->element_aligned != 0 && pl->element_aligned != 1) return fail(QSSM_EINVAL, "plan.element_aligned must be 0 or 1");
+  if (pl->element_aligned ? pl->D > 0 && pl->D < pl->vec : pl->D % pl->vec != 0)
+    return fail(QSSM_EALIGN, "D=%d is not a multiple of plan.vec=%d", pl->D, pl->vec);
   const int ng = pl->threads >> pl->g_log2;
   if (pl->strip_cols != (pl->vec << pl->g_log2) || pl->seg_len != pl->steps * ng)
     return fail(QSSM_EINVAL, "plan geometry is inconsistent");
@@ -205,6 +209,9 @@ static int backward_launch(const qssm_plan* plan, const void* x, qssm_strides sx
                            uint64_t control_size, void* workspace, uint64_t workspace_bytes, uint32_t epoch,
                            void* stream, const GateExtras* gate = nullptr);
 
+static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
+                     int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan);
+
 extern "C" {
 
 int qssm_version(void) { return QSSM_VERSION; }
@@ -259,6 +266,18 @@ int qssm_plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t
 
 int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
                          int32_t align_elems, int32_t ckpt_stride, int32_t tune, qssm_plan* plan) {
+  return plan_scan(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, false, plan);
+}
+
+int qssm_plan_scan_loose(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
+                         int32_t align_elems, int32_t ckpt_stride, int32_t tune, qssm_plan* plan) {
+  return plan_scan(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, true, plan);
+}
+
+}  // extern "C"
+
+static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
+                     int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan) {
   if (plan == nullptr) return fail(QSSM_EINVAL, "plan is NULL");
   if (B < 0 || L < 0 || D < 0) return fail(QSSM_EINVAL, "negative dimension");
   if (direction != QSSM_FORWARD && direction != QSSM_BACKWARD) return fail(QSSM_EINVAL, "bad direction");
@@ -297,7 +316,21 @@ int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int3
   const bool wide_auto = direction == QSSM_FORWARD && tune_vec == 0 && os == 2 && D >= 256 &&
                          wide_chains * ((L + 63) / 64) >= 12 * kCUs && !(wide_chains < 32 && L >= 256 * 64);
   if (wide_ok && (tune_vec == 8 || wide_auto)) vec = 8;
-  while (vec > 1 && (align_elems % vec != 0 || (D > 0 && D % vec != 0))) vec >>= 1;
+  int whole = vec;   // columns a lane can take of rows that are aligned and divided that way
+  while (whole > 1 && (align_elems % whole != 0 || (D > 0 && D % whole != 0))) whole >>= 1;
+  // Rows that are not: single elements per lane would leave the launch bound by its instructions (a lane's load moves 2
+  // bytes), so a loose plan keeps the wide lanes at element alignment, the last one sharing columns with its neighbour.
+  // Step (forward and backward), narrow lanes -> these: fp16 B=8 L=4096 D=1001 529 -> 244 us, bf16 B=5 L=1537 D=777 138 ->
+  // 77, B=1 L=20000 D=515 258 -> 125, fp32 B=4 L=4096 D=333 158 -> 92, and where two columns were aligned already bf16 B=8
+  // L=4096 D=2050 524 -> 458, fp32 B=4 L=2048 D=1026 158 -> 119.  From kLooseColumns columns on (D=33 and 47 gained as
+  // well), below which a shared lane is a large part of a row.
+  if (loose && whole < vec && tune_vec == 0 && D >= kLooseColumns) {
+    if (vec == 8) vec = 4;
+    plan->element_aligned = vec > whole ? 1 : 0;
+    if (vec < whole) vec = whole;
+  } else {
+    vec = whole;
+  }
   plan->vec = vec;
 
   // Steps per lane: 8.  Fewer steps mean more, shorter tiles, and every tile pays the same fixed
@@ -463,6 +496,8 @@ int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int3
   return 0;
 }
 
+extern "C" {
+
 int qssm_zero_fill(void* workspace, uint64_t bytes, void* stream) {
   if (workspace == nullptr || bytes == 0) return 0;
   if (((uintptr_t)workspace) % 16 != 0 || bytes % 16 != 0)
@@ -538,10 +573,11 @@ static int forward_launch(const qssm_plan* plan, const void* x, qssm_strides sx,
   fwd_launch_fn fn = find_fwd_launcher(plan->in_dtype, plan->out_dtype);
   if (fn == nullptr) return fail(QSSM_EINVAL, "dtype pair is not built");
   const int es = dtype_size(plan->in_dtype), os = dtype_size(plan->out_dtype), v = plan->vec;
-  if (!aligned_to(x, sx.b, sx.l, es, v) || !aligned_to(a, sa.b, sa.l, es, v) || !aligned_to(b, sb.b, sb.l, es, v) ||
-      !aligned_to(c, sc.b, sc.l, es, v) || !aligned_to(y, sy.b, sy.l, os, v) ||
-      !aligned_to(h_out, sh.b, sh.l, 4, v) || !aligned_to(ckpt, 0, 0, 4, v) || !aligned_to(h_init, 0, 0, 4, v) ||
-      !aligned_to(h_final, 0, 0, 4, v))
+  const int va = plan->element_aligned ? 1 : v;   // what addresses and strides are multiples of, in elements
+  if (!aligned_to(x, sx.b, sx.l, es, va) || !aligned_to(a, sa.b, sa.l, es, va) || !aligned_to(b, sb.b, sb.l, es, va) ||
+      !aligned_to(c, sc.b, sc.l, es, va) || !aligned_to(y, sy.b, sy.l, os, va) ||
+      !aligned_to(h_out, sh.b, sh.l, 4, va) || !aligned_to(ckpt, 0, 0, 4, va) || !aligned_to(h_init, 0, 0, 4, va) ||
+      !aligned_to(h_final, 0, 0, 4, va))
     return fail(QSSM_EALIGN, "a pointer or stride is not aligned to plan.vec=%d elements", v);
   if (control == nullptr || control_size < plan->control_bytes)
     return fail(QSSM_EWORKSPACE, "control block has %llu bytes, plan needs %llu", (unsigned long long)control_size,
@@ -572,7 +608,7 @@ static int forward_launch(const qssm_plan* plan, const void* x, qssm_strides sx,
   const bool narrow_rows = v * es == 8 && (es == 2 || gate != nullptr) && (plan->g_log2 == 6 || plan->g_log2 == 5) &&
                            (plan->threads == 256 || plan->threads == 512);
   const bool wide_rows = es == 2 && v == 8 && (plan->threads == 256 || plan->threads == 512);   // every lane fetches its own 16 bytes
-  bool c_in_lds = y != nullptr && c != nullptr && ((narrow_rows && plan->steps == 8) || wide_rows) &&
+  bool c_in_lds = !plan->element_aligned && y != nullptr && c != nullptr && ((narrow_rows && plan->steps == 8) || wide_rows) &&
                   ((uintptr_t)c) % 16 == 0 && (sc.b * es) % 16 == 0 && (sc.l * es) % 16 == 0 &&
                   lds + fwd_c_lds_bytes(plan->threads, plan->steps, v * es) <= (size_t)kMaxLdsBytes;
   if (c_in_lds) lds += fwd_c_lds_bytes(plan->threads, plan->steps, v * es);
@@ -638,12 +674,13 @@ static int backward_launch(const qssm_plan* plan, const void* x, qssm_strides sx
   bwd_launch_fn fn = find_bwd_launcher(plan->in_dtype, plan->out_dtype);
   if (fn == nullptr) return fail(QSSM_EINVAL, "dtype pair is not built");
   const int es = dtype_size(plan->in_dtype), os = dtype_size(plan->out_dtype), v = plan->vec;
-  if (!aligned_to(x, sx.b, sx.l, es, v) || !aligned_to(a, sa.b, sa.l, es, v) || !aligned_to(b, sb.b, sb.l, es, v) ||
-      !aligned_to(c, sc.b, sc.l, es, v) || !aligned_to(dy, sdy.b, sdy.l, os, v) ||
-      !aligned_to(h, sh.b, sh.l, 4, v) || !aligned_to(ckpt, 0, 0, 4, v) || !aligned_to(h_init, 0, 0, 4, v) ||
-      !aligned_to(dh_final, 0, 0, 4, v) || !aligned_to(dh_init, 0, 0, 4, v) || !aligned_to(dx, sdx.b, sdx.l, es, v) ||
-      !aligned_to(da, sda.b, sda.l, es, v) || !aligned_to(db, sdb.b, sdb.l, es, v) ||
-      !aligned_to(dc, sdc.b, sdc.l, es, v))
+  const int va = plan->element_aligned ? 1 : v;   // what addresses and strides are multiples of, in elements
+  if (!aligned_to(x, sx.b, sx.l, es, va) || !aligned_to(a, sa.b, sa.l, es, va) || !aligned_to(b, sb.b, sb.l, es, va) ||
+      !aligned_to(c, sc.b, sc.l, es, va) || !aligned_to(dy, sdy.b, sdy.l, os, va) ||
+      !aligned_to(h, sh.b, sh.l, 4, va) || !aligned_to(ckpt, 0, 0, 4, va) || !aligned_to(h_init, 0, 0, 4, va) ||
+      !aligned_to(dh_final, 0, 0, 4, va) || !aligned_to(dh_init, 0, 0, 4, va) || !aligned_to(dx, sdx.b, sdx.l, es, va) ||
+      !aligned_to(da, sda.b, sda.l, es, va) || !aligned_to(db, sdb.b, sdb.l, es, va) ||
+      !aligned_to(dc, sdc.b, sdc.l, es, va))
     return fail(QSSM_EALIGN, "a pointer or stride is not aligned to plan.vec=%d elements", v);
   if (control == nullptr || control_size < plan->control_bytes)
     return fail(QSSM_EWORKSPACE, "control block has %llu bytes, plan needs %llu", (unsigned long long)control_size,
@@ -676,7 +713,7 @@ static int backward_launch(const qssm_plan* plan, const void* x, qssm_strides sx
   // lanes in both and their rows can be fetched 16 bytes at a time.
   size_t lds = (size_t)plan->lds_bytes;
   // (8 bytes per lane: 4 columns of 16-bit storage; 2 columns of fp32, with fp32 dy, only in the gated scan's kernels)
-  bool cg_in_lds = ((es == 2 && (os == 2 || os == 4) && v == 4) || (gate != nullptr && es == 4 && os == 4 && v == 2)) &&
+  bool cg_in_lds = !plan->element_aligned && ((es == 2 && (os == 2 || os == 4) && v == 4) || (gate != nullptr && es == 4 && os == 4 && v == 2)) &&
                    (plan->g_log2 == 6 || plan->g_log2 == 5) && plan->steps == 8 && plan->threads == 256 &&
                    ((uintptr_t)c) % 16 == 0 && (sc.b * es) % 16 == 0 && (sc.l * es) % 16 == 0 &&
                    ((uintptr_t)dy) % 16 == 0 && (sdy.b * os) % 16 == 0 && (sdy.l * os) % 16 == 0 &&

@@ -55,6 +55,10 @@ __global__ void __launch_bounds__(NTH) scan_bwd_kernel(const BwdArgs p) {
   static_assert(!GATED || sizeof(Tout) * VEC == 8, "gated scan: dy at 8 bytes per lane");
   constexpr bool GW = CLDS && sizeof(Tout) * VEC == 16;   // dy alone in LDS, 16 bytes per lane
   constexpr bool CREG = !CLDS || GW;                       // c in registers
+  // Rows that D does not divide into whole lanes (plans with element_aligned): the last lane of a row ends with it and
+  // shares columns with the lane before.  Only the register-only kernels are launched with such a D; in the others the
+  // arithmetic would cost what decides how many workgroups a compute unit holds (4 % of the headline shape's step).
+  constexpr bool LOOSE = !CLDS && VEC > 1;
   extern __shared__ __align__(16) float lds[];
   const Geometry& g = p.g;
   const int G = 1 << g.g_log2;
@@ -102,13 +106,13 @@ __global__ void __launch_bounds__(NTH) scan_bwd_kernel(const BwdArgs p) {
       // nobody wrote, and reports it.
       if (tid == 0) raise_status(g.status, 2);
       const int pseg = blockIdx.x / g.n_chains, pbi = chain / g.n_strips, pstrip = chain - pbi * g.n_strips;
-      const int pd = pstrip * cols + (tid & (G - 1)) * VEC;
+      const int pd0 = pstrip * cols + (tid & (G - 1)) * VEC, pd = LOOSE && pd0 > g.D - VEC ? g.D - VEC : pd0;
       float nanv[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) nanv[v] = __uint_as_float(0x7fc00000u);
       for (int i = 0; i < T; ++i) {
         const int t = pseg * g.seg_len + (tid >> g.g_log2) * T + i;
-        if (pd < g.D && t < g.L) {
+        if (pd0 < g.D && t < g.L) {
           if (p.dx != nullptr)
             store_stream<Tin, VEC>((char*)p.dx + ((int64_t)pbi * p.dx_sb + (int64_t)t * p.dx_sl + pd) * (int64_t)sizeof(Tin), 0u, nanv);
           if (p.da != nullptr)
@@ -121,7 +125,7 @@ __global__ void __launch_bounds__(NTH) scan_bwd_kernel(const BwdArgs p) {
             store_stream<Tin, VEC>((char*)p.dc2 + ((int64_t)pbi * p.dc2_sb + (int64_t)t * p.dc2_sl + pd) * (int64_t)sizeof(Tin), 0u, nanv);
         }
       }
-      if (p.dh_init != nullptr && pseg == 0 && (tid >> g.g_log2) == 0 && pd < g.D)
+      if (p.dh_init != nullptr && pseg == 0 && (tid >> g.g_log2) == 0 && pd0 < g.D)
         store_stream<float, VEC>((char*)p.dh_init + ((int64_t)pbi * g.D + pd) * (int64_t)sizeof(float), 0u, nanv);
       return;
     }
@@ -132,25 +136,27 @@ __global__ void __launch_bounds__(NTH) scan_bwd_kernel(const BwdArgs p) {
   const int strip = chain - bi * g.n_strips;
   const int j = tid >> g.g_log2;
   const int dl = (tid & (G - 1)) * VEC;
-  const int d = strip * cols + dl;
-  const bool dok = d < g.D;
+  const int last_d = g.D - VEC;
+  const int d = LOOSE && strip * cols + dl > last_d ? last_d : strip * cols + dl;
+  const bool dok = strip * cols + dl < g.D;
   const int t_tile = seg * g.seg_len;
   const int t0 = t_tile + j * T;
   const bool have_h = p.h != nullptr;
 
-  const int64_t col0 = (int64_t)strip * cols;
+  const int64_t col0 = LOOSE && strip * cols > last_d ? last_d : (int64_t)strip * cols;
+  const int dc = LOOSE ? d - (int)col0 : dl;   // first column of this lane in the operands, from the tile's base
   const char* xb = (const char*)p.x + ((int64_t)bi * p.x_sb + (int64_t)t_tile * p.x_sl + col0) * (int64_t)sizeof(Tin);
   const char* ab = (const char*)p.a + ((int64_t)bi * p.a_sb + (int64_t)t_tile * p.a_sl + col0) * (int64_t)sizeof(Tin);
   const char* bb = (const char*)p.b + ((int64_t)bi * p.b_sb + (int64_t)t_tile * p.b_sl + col0) * (int64_t)sizeof(Tin);
   const char* cb = (const char*)p.c + ((int64_t)bi * p.c_sb + (int64_t)t_tile * p.c_sl + col0) * (int64_t)sizeof(Tin);
   const char* gb = (const char*)p.dy + ((int64_t)bi * p.dy_sb + (int64_t)t_tile * p.dy_sl + col0) * (int64_t)sizeof(Tout);
-  const uint32_t xo = (uint32_t)((j * T * (int)p.x_sl + dl) * (int)sizeof(Tin)), xs = (uint32_t)p.x_sl * sizeof(Tin);
-  const uint32_t ao = (uint32_t)((j * T * (int)p.a_sl + dl) * (int)sizeof(Tin)), as = (uint32_t)p.a_sl * sizeof(Tin);
-  const uint32_t bo = (uint32_t)((j * T * (int)p.b_sl + dl) * (int)sizeof(Tin)), bs = (uint32_t)p.b_sl * sizeof(Tin);
-  const uint32_t co = (uint32_t)((j * T * (int)p.c_sl + dl) * (int)sizeof(Tin)), cs = (uint32_t)p.c_sl * sizeof(Tin);
-  const uint32_t go = (uint32_t)((j * T * (int)p.dy_sl + dl) * (int)sizeof(Tout)), gs = (uint32_t)p.dy_sl * sizeof(Tout);
+  const uint32_t xo = (uint32_t)((j * T * (int)p.x_sl + dc) * (int)sizeof(Tin)), xs = (uint32_t)p.x_sl * sizeof(Tin);
+  const uint32_t ao = (uint32_t)((j * T * (int)p.a_sl + dc) * (int)sizeof(Tin)), as = (uint32_t)p.a_sl * sizeof(Tin);
+  const uint32_t bo = (uint32_t)((j * T * (int)p.b_sl + dc) * (int)sizeof(Tin)), bs = (uint32_t)p.b_sl * sizeof(Tin);
+  const uint32_t co = (uint32_t)((j * T * (int)p.c_sl + dc) * (int)sizeof(Tin)), cs = (uint32_t)p.c_sl * sizeof(Tin);
+  const uint32_t go = (uint32_t)((j * T * (int)p.dy_sl + dc) * (int)sizeof(Tout)), gs = (uint32_t)p.dy_sl * sizeof(Tout);
   const char* c2b = GATED ? (const char*)p.c2 + ((int64_t)bi * p.c2_sb + (int64_t)t_tile * p.c2_sl + col0) * (int64_t)sizeof(Tin) : nullptr;
-  const uint32_t c2o = GATED ? (uint32_t)((j * T * (int)p.c2_sl + dl) * (int)sizeof(Tin)) : 0u, c2s = GATED ? (uint32_t)p.c2_sl * sizeof(Tin) : 0u;
+  const uint32_t c2o = GATED ? (uint32_t)((j * T * (int)p.c2_sl + dc) * (int)sizeof(Tin)) : 0u, c2s = GATED ? (uint32_t)p.c2_sl * sizeof(Tin) : 0u;
   const float* hp = p.h + (int64_t)bi * p.h_sb + (int64_t)t0 * p.h_sl + d;
 
   // ---- ask for the neighbours' words first: they are looked at once the answers are back ------
@@ -619,12 +625,12 @@ __global__ void __launch_bounds__(NTH) scan_bwd_kernel(const BwdArgs p) {
   char* dab = (char*)p.da + ((int64_t)bi * p.da_sb + (int64_t)t_tile * p.da_sl + col0) * (int64_t)sizeof(Tin);
   char* dbb = (char*)p.db + ((int64_t)bi * p.db_sb + (int64_t)t_tile * p.db_sl + col0) * (int64_t)sizeof(Tin);
   char* dcb = (char*)p.dc + ((int64_t)bi * p.dc_sb + (int64_t)t_tile * p.dc_sl + col0) * (int64_t)sizeof(Tin);
-  const uint32_t dxo = (uint32_t)((j * T * (int)p.dx_sl + dl) * (int)sizeof(Tin)), dxs = (uint32_t)p.dx_sl * sizeof(Tin);
-  const uint32_t dao = (uint32_t)((j * T * (int)p.da_sl + dl) * (int)sizeof(Tin)), das = (uint32_t)p.da_sl * sizeof(Tin);
-  const uint32_t dbo = (uint32_t)((j * T * (int)p.db_sl + dl) * (int)sizeof(Tin)), dbs = (uint32_t)p.db_sl * sizeof(Tin);
-  const uint32_t dco = (uint32_t)((j * T * (int)p.dc_sl + dl) * (int)sizeof(Tin)), dcs = (uint32_t)p.dc_sl * sizeof(Tin);
+  const uint32_t dxo = (uint32_t)((j * T * (int)p.dx_sl + dc) * (int)sizeof(Tin)), dxs = (uint32_t)p.dx_sl * sizeof(Tin);
+  const uint32_t dao = (uint32_t)((j * T * (int)p.da_sl + dc) * (int)sizeof(Tin)), das = (uint32_t)p.da_sl * sizeof(Tin);
+  const uint32_t dbo = (uint32_t)((j * T * (int)p.db_sl + dc) * (int)sizeof(Tin)), dbs = (uint32_t)p.db_sl * sizeof(Tin);
+  const uint32_t dco = (uint32_t)((j * T * (int)p.dc_sl + dc) * (int)sizeof(Tin)), dcs = (uint32_t)p.dc_sl * sizeof(Tin);
   char* dc2b = GATED ? (char*)p.dc2 + ((int64_t)bi * p.dc2_sb + (int64_t)t_tile * p.dc2_sl + col0) * (int64_t)sizeof(Tin) : nullptr;
-  const uint32_t dc2o = GATED ? (uint32_t)((j * T * (int)p.dc2_sl + dl) * (int)sizeof(Tin)) : 0u, dc2s = GATED ? (uint32_t)p.dc2_sl * sizeof(Tin) : 0u;
+  const uint32_t dc2o = GATED ? (uint32_t)((j * T * (int)p.dc2_sl + dc) * (int)sizeof(Tin)) : 0u, dc2s = GATED ? (uint32_t)p.dc2_sl * sizeof(Tin) : 0u;
 #pragma unroll
   for (int i = T - 1; i >= 0; --i) {
     float vdx[VEC], vda[VEC], vdb[VEC], vdc[VEC], vdc2[VEC];

@@ -21,6 +21,9 @@
 //             is a serial dependency: one hop per cluster, not per tile.
 //   sweep 2   every lane re-runs its T steps from the true carry-in and stores the results
 //
+// Where D is no multiple of VEC (plans with element_aligned), the last lane of a row takes the row's last VEC columns,
+// some of which its neighbour has too: both compute the same bits from the same values, and both store them.
+//
 // Words exchanged between workgroups are {epoch:32 | fp32 bits:32}: flag and payload travel
 // in one 64-bit access, so no fence is needed between them, and a word left over from an
 // earlier launch (older epoch) reads as "not there yet".  Agent scope makes the accesses
@@ -151,7 +154,9 @@ __device__ __forceinline__ float elem(const Words<T, V>& p, int v) {
   return ElemBits<T>::template get<V>(p, v);
 }
 
-// One vector load / store of VEC elements at a byte offset from a workgroup-uniform base.
+// One vector load / store of VEC elements at a byte offset from a workgroup-uniform base.  The address needs the
+// alignment of one element only (one instruction all the same: the hardware takes global accesses at any address, and
+// pays for a misaligned one with the extra cache line it touches); the same holds for load_pack and store_pack.
 // Operands and results are touched exactly once by a launch, so they are marked non-temporal (streaming); KEEP
 // asks for an ordinary load instead, whose lines stay in the caches for a launch that follows.
 template <typename T, int V, bool KEEP = false>
@@ -164,9 +169,10 @@ __device__ __forceinline__ Words<T, V> load_stream(const char* base, uint32_t by
     return out;
   } else {
   typedef typename RawOf<sizeof(T) * V>::type raw_t;
+  typedef raw_t loose_t __attribute__((aligned(sizeof(T))));
   raw_t r;
-  if constexpr (KEEP) r = *reinterpret_cast<const raw_t*>(base + byte_off);
-  else r = __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(base + byte_off));
+  if constexpr (KEEP) r = *reinterpret_cast<const loose_t*>(base + byte_off);
+  else r = __builtin_nontemporal_load(reinterpret_cast<const loose_t*>(base + byte_off));
   Words<T, V> out;
   if constexpr (sizeof(T) * V <= 4) {
     out.w[0] = (uint32_t)r;
@@ -185,6 +191,7 @@ __device__ __forceinline__ void store_stream(char* base, uint32_t byte_off, cons
     store_stream<T, V / 2>(base, byte_off + 16u, f + V / 2);
   } else {
   typedef typename RawOf<sizeof(T) * V>::type raw_t;
+  typedef raw_t loose_t __attribute__((aligned(sizeof(T))));
   Words<T, V> p;
   ElemBits<T>::template set<V>(p, f);
   raw_t r;
@@ -194,7 +201,7 @@ __device__ __forceinline__ void store_stream(char* base, uint32_t byte_off, cons
 #pragma unroll
     for (int k = 0; k < Words<T, V>::N; ++k) r[k] = p.w[k];
   }
-  __builtin_nontemporal_store(r, reinterpret_cast<raw_t*>(base + byte_off));
+  __builtin_nontemporal_store(r, reinterpret_cast<loose_t*>(base + byte_off));
   }
 }
 
@@ -219,7 +226,8 @@ __device__ __forceinline__ Pack<T, V> load_pack(const T* p) {
     return out;
   } else {
     typedef typename RawOf<sizeof(T) * V>::type raw_t;
-    raw_t r = *reinterpret_cast<const raw_t*>(p);
+    typedef raw_t loose_t __attribute__((aligned(sizeof(T))));
+    raw_t r = *reinterpret_cast<const loose_t*>(p);
     return __builtin_bit_cast(Pack<T, V>, r);
   }
 }
@@ -234,7 +242,8 @@ __device__ __forceinline__ void store_pack(T* p, const Pack<T, V>& v) {
     store_pack<T, V / 2>(p + V / 2, hi);
   } else {
     typedef typename RawOf<sizeof(T) * V>::type raw_t;
-    *reinterpret_cast<raw_t*>(p) = __builtin_bit_cast(raw_t, v);
+    typedef raw_t loose_t __attribute__((aligned(sizeof(T))));
+    *reinterpret_cast<loose_t*>(p) = __builtin_bit_cast(raw_t, v);
   }
 }
 

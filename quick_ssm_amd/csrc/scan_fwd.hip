@@ -43,6 +43,10 @@ __global__ void __launch_bounds__(NTH) scan_fwd_kernel(const FwdArgs p) {
   // 16 bytes per lane: the load that deposits c in LDS gives every lane exactly its own columns of one step.
   constexpr bool WIDE = sizeof(Tin) * VEC == 16;
   constexpr int CROW = WIDE ? 1024 : 512;   // bytes of c one wavefront holds per step
+  // Rows that D does not divide into whole lanes (plans with element_aligned): the last lane of a row ends with it and
+  // shares columns with the lane before.  Only the register-only kernels are launched with such a D; in the others the
+  // arithmetic would cost what decides how many workgroups a compute unit holds (4 % of the headline shape's step).
+  constexpr bool LOOSE = !CLDS && VEC > 1;
   extern __shared__ __align__(16) float lds[];
   const Geometry& g = p.g;
   const int G = 1 << g.g_log2;
@@ -84,13 +88,13 @@ __global__ void __launch_bounds__(NTH) scan_fwd_kernel(const FwdArgs p) {
       // nobody wrote, and reports it.
       if (tid == 0) raise_status(g.status, 2);
       const int pseg = blockIdx.x / g.n_chains, pbi = chain / g.n_strips, pstrip = chain - pbi * g.n_strips;
-      const int pd = pstrip * cols + (tid & (G - 1)) * VEC;
+      const int pd0 = pstrip * cols + (tid & (G - 1)) * VEC, pd = LOOSE && pd0 > g.D - VEC ? g.D - VEC : pd0;
       float nanv[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) nanv[v] = __uint_as_float(0x7fc00000u);
       for (int i = 0; i < T; ++i) {
         const int t = pseg * g.seg_len + (tid >> g.g_log2) * T + i;
-        if (pd < g.D && t < g.L) {
+        if (pd0 < g.D && t < g.L) {
           if (p.y != nullptr)
             store_stream<Tout, VEC>((char*)p.y + ((int64_t)pbi * p.y_sb + (int64_t)t * p.y_sl + pd) * (int64_t)sizeof(Tout), 0u, nanv);
           if (p.h_out != nullptr)
@@ -99,7 +103,7 @@ __global__ void __launch_bounds__(NTH) scan_fwd_kernel(const FwdArgs p) {
             store_stream<float, VEC>((char*)p.ckpt + (((int64_t)pbi * g.n_ckpt + t / g.ckpt_stride) * g.D + pd) * (int64_t)sizeof(float), 0u, nanv);
         }
       }
-      if (p.h_final != nullptr && pseg == g.n_seg - 1 && (tid >> g.g_log2) == 0 && pd < g.D)
+      if (p.h_final != nullptr && pseg == g.n_seg - 1 && (tid >> g.g_log2) == 0 && pd0 < g.D)
         store_stream<float, VEC>((char*)p.h_final + ((int64_t)pbi * g.D + pd) * (int64_t)sizeof(float), 0u, nanv);
       return;
     }
@@ -109,23 +113,25 @@ __global__ void __launch_bounds__(NTH) scan_fwd_kernel(const FwdArgs p) {
   const int strip = chain - bi * g.n_strips;
   const int j = tid >> g.g_log2;         // lane group = time sub-segment
   const int dl = (tid & (G - 1)) * VEC;  // first column of this lane inside the strip
-  const int d = strip * cols + dl;
-  const bool dok = d < g.D;
+  const int last_d = g.D - VEC;
+  const int d = LOOSE && strip * cols + dl > last_d ? last_d : strip * cols + dl;
+  const bool dok = strip * cols + dl < g.D;
   const int t_tile = seg * g.seg_len;
   const int t0 = t_tile + j * T;
 
   // Workgroup-uniform base of the tile in every operand, plus a 32-bit per-lane byte offset.
-  const int64_t col0 = (int64_t)strip * cols;
+  const int64_t col0 = LOOSE && strip * cols > last_d ? last_d : (int64_t)strip * cols;
+  const int dc = LOOSE ? d - (int)col0 : dl;   // first column of this lane in the operands, from the tile's base
   const char* xb = (const char*)p.x + ((int64_t)bi * p.x_sb + (int64_t)t_tile * p.x_sl + col0) * (int64_t)sizeof(Tin);
   const char* ab = (const char*)p.a + ((int64_t)bi * p.a_sb + (int64_t)t_tile * p.a_sl + col0) * (int64_t)sizeof(Tin);
   const char* bb = (const char*)p.b + ((int64_t)bi * p.b_sb + (int64_t)t_tile * p.b_sl + col0) * (int64_t)sizeof(Tin);
   const char* cb = (const char*)p.c + ((int64_t)bi * p.c_sb + (int64_t)t_tile * p.c_sl + col0) * (int64_t)sizeof(Tin);
-  const uint32_t xo = (uint32_t)((j * T * (int)p.x_sl + dl) * (int)sizeof(Tin)), xs = (uint32_t)p.x_sl * sizeof(Tin);
-  const uint32_t ao = (uint32_t)((j * T * (int)p.a_sl + dl) * (int)sizeof(Tin)), as = (uint32_t)p.a_sl * sizeof(Tin);
-  const uint32_t bo = (uint32_t)((j * T * (int)p.b_sl + dl) * (int)sizeof(Tin)), bs = (uint32_t)p.b_sl * sizeof(Tin);
-  const uint32_t co = (uint32_t)((j * T * (int)p.c_sl + dl) * (int)sizeof(Tin)), cs = (uint32_t)p.c_sl * sizeof(Tin);
+  const uint32_t xo = (uint32_t)((j * T * (int)p.x_sl + dc) * (int)sizeof(Tin)), xs = (uint32_t)p.x_sl * sizeof(Tin);
+  const uint32_t ao = (uint32_t)((j * T * (int)p.a_sl + dc) * (int)sizeof(Tin)), as = (uint32_t)p.a_sl * sizeof(Tin);
+  const uint32_t bo = (uint32_t)((j * T * (int)p.b_sl + dc) * (int)sizeof(Tin)), bs = (uint32_t)p.b_sl * sizeof(Tin);
+  const uint32_t co = (uint32_t)((j * T * (int)p.c_sl + dc) * (int)sizeof(Tin)), cs = (uint32_t)p.c_sl * sizeof(Tin);
   const char* c2b = GATED ? (const char*)p.c2 + ((int64_t)bi * p.c2_sb + (int64_t)t_tile * p.c2_sl + col0) * (int64_t)sizeof(Tin) : nullptr;
-  const uint32_t c2o = GATED ? (uint32_t)((j * T * (int)p.c2_sl + dl) * (int)sizeof(Tin)) : 0u, c2s = GATED ? (uint32_t)p.c2_sl * sizeof(Tin) : 0u;
+  const uint32_t c2o = GATED ? (uint32_t)((j * T * (int)p.c2_sl + dc) * (int)sizeof(Tin)) : 0u, c2s = GATED ? (uint32_t)p.c2_sl * sizeof(Tin) : 0u;
   const bool want_y = p.y != nullptr;
   const bool has_c = want_y && p.c != nullptr;
 
@@ -481,8 +487,8 @@ __global__ void __launch_bounds__(NTH) scan_fwd_kernel(const FwdArgs p) {
   // ---- sweep 2: the recurrence proper, from the true carry-in -----------------------------------
   char* yb = (char*)p.y + ((int64_t)bi * p.y_sb + (int64_t)t_tile * p.y_sl + col0) * (int64_t)sizeof(Tout);
   char* hb = (char*)p.h_out + ((int64_t)bi * p.h_sb + (int64_t)t_tile * p.h_sl + col0) * (int64_t)sizeof(float);
-  const uint32_t yo = (uint32_t)((j * T * (int)p.y_sl + dl) * (int)sizeof(Tout)), ys = (uint32_t)p.y_sl * sizeof(Tout);
-  const uint32_t ho = (uint32_t)((j * T * (int)p.h_sl + dl) * (int)sizeof(float)), hs = (uint32_t)p.h_sl * sizeof(float);
+  const uint32_t yo = (uint32_t)((j * T * (int)p.y_sl + dc) * (int)sizeof(Tout)), ys = (uint32_t)p.y_sl * sizeof(Tout);
+  const uint32_t ho = (uint32_t)((j * T * (int)p.h_sl + dc) * (int)sizeof(float)), hs = (uint32_t)p.h_sl * sizeof(float);
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     float yv[VEC];

@@ -138,10 +138,10 @@ const qssm_plan& plan_for(const PlanKey& k) {
   qssm_plan p;
   int32_t stride = k.ckpt;
   if (k.direction == QSSM_FORWARD && k.ckpt != 0) {
-    check_rc(qssm_plan_scan_tuned(k.B, k.L, k.D, k.in, k.out, QSSM_BACKWARD, k.align, 0, k.bwd_tune, &p));
+    check_rc(qssm_plan_scan_loose(k.B, k.L, k.D, k.in, k.out, QSSM_BACKWARD, k.align, 0, k.bwd_tune, &p));
     stride = p.seg_len;
   }
-  check_rc(qssm_plan_scan_tuned(k.B, k.L, k.D, k.in, k.out, k.direction, k.align, stride, k.tune, &p));
+  check_rc(qssm_plan_scan_loose(k.B, k.L, k.D, k.in, k.out, k.direction, k.align, stride, k.tune, &p));
   if (k.direction == QSSM_FORWARD && k.keep >= 0 && p.keep_tiles > k.keep) p.keep_tiles = k.keep;
   if (plans.size() >= 1024) plans.clear();
   return plans.emplace(k, p).first->second;

@@ -1,0 +1,89 @@
+"""Plans for rows that are not aligned to, or not divided by, the lanes' width (qssm_plan_scan_loose)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import TOL, assert_close, make_inputs, oracle_all
+from quick_ssm_amd import _lib, hip_scan, scan, scan_chunk
+
+
+def _plan(B, L, D, dtype, out_dtype, direction, align, stride=0):
+    code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+    p = _lib.Plan()
+    lib = _lib.load()
+    _lib.check(lib.qssm_plan_scan_loose(B, L, D, code[dtype], code[out_dtype], direction, align, stride, 0, ctypes.byref(p)))
+    return p
+
+
+@pytest.mark.parametrize("D", [1, 3, 31, 32, 33, 34, 36, 63, 65, 127, 129, 255, 257, 258, 511, 513, 777, 1000, 1027, 4095])
+def test_every_column_is_covered_and_nothing_beyond_the_rows(D):
+    for dtype, out in ((torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)):
+        for align in (1, 2, 4, 8):
+            if align > 1 and D % align:
+                continue
+            for B, L in ((1, 1), (2, 300), (1, 5000), (4, 2048)):
+                back = _plan(B, L, D, dtype, out, _lib.QSSM_BACKWARD, align)
+                ahead = _plan(B, L, D, dtype, out, _lib.QSSM_FORWARD, align, back.seg_len)
+                assert ahead.n_ckpt == back.n_ckpt
+                for p, direction in ((back, _lib.QSSM_BACKWARD), (ahead, _lib.QSSM_FORWARD)):
+                    tight = hip_scan.make_plan(B, L, D, dtype, out, direction, align, p.ckpt_stride if p is ahead else 0)
+                    if not p.element_aligned:   # the same plan as without the freedom
+                        assert p.describe() == tight.describe()
+                        assert D % p.vec == 0 and align % p.vec == 0
+                        continue
+                    assert D >= 32 and p.vec > tight.vec and p.vec <= 4
+                    lanes = np.arange(p.n_strips * (1 << p.g_log2)) * p.vec
+                    first = np.minimum(lanes[lanes < D], D - p.vec)
+                    assert first.min() >= 0 and set((first[:, None] + np.arange(p.vec)).ravel()) == set(range(D))
+                    # a tile's base and a lane's offset from it are both non-negative
+                    strip = np.minimum(lanes[lanes < D] // p.strip_cols * p.strip_cols, D - p.vec)
+                    assert (first >= strip).all()
+
+
+SHAPES = [(2, 300, 33), (3, 100, 35), (2, 1100, 257), (1, 700, 258), (2, 513, 777), (1, 5000, 61), (64, 1, 1027)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
+                         ids=["f32", "bf16", "f16-f32"])
+@pytest.mark.parametrize("shift", [0, 1], ids=["dense", "shifted"])
+def test_scan_and_gradients_match_the_oracle(gpu, shape, dtypes, shift):
+    dtype, out = dtypes
+    x, a, b, c, dy = make_inputs(shape, dtype=dtype, seed=sum(shape), out_dtype=out)
+    ref = oracle_all(x, a, b, c, dy)
+
+    def place(t):
+        """On the GPU, its rows starting one element into wider ones when `shift`."""
+        if not shift:
+            return t.to(gpu)
+        wide = torch.full((*t.shape[:2], t.shape[2] + 3), float("nan"), dtype=t.dtype, device=gpu)
+        view = wide[..., 1:1 + t.shape[2]]
+        view.copy_(t)
+        return view
+
+    for checkpoint in (True, False):
+        leaves = [place(t).requires_grad_(True) for t in (x, a, b, c)]
+        y = scan(*leaves, checkpoint=checkpoint, out_dtype=out)
+        grads = torch.autograd.grad(y, leaves, place(dy))
+        assert hip_scan.workspace_status() == 0
+        assert_close("y", y.detach().cpu(), ref["y"], TOL[out])
+        for name, g in zip(("dx", "da", "db", "dc"), grads):
+            assert_close(name, g.cpu(), ref[name], TOL[dtype])
+
+
+@pytest.mark.gpu
+def test_states_cross_pieces_of_odd_rows(gpu):
+    x, a, b, c, dy = (t.to(gpu) for t in make_inputs((2, 900, 333), seed=4))
+    whole = [t.clone().requires_grad_(True) for t in (x, a, b, c)]
+    parts = [t.clone().requires_grad_(True) for t in (x, a, b, c)]
+    y = scan(*whole)
+    ys, state = [], torch.zeros(2, 333, device=gpu)
+    for lo, hi in ((0, 101), (101, 500), (500, 900)):
+        piece, state = scan_chunk(*(t[:, lo:hi] for t in parts), state)
+        ys.append(piece)
+    for got, want in zip((torch.cat(ys, 1), *torch.autograd.grad(torch.cat(ys, 1), parts, dy)),
+                         (y, *torch.autograd.grad(y, whole, dy))):
+        assert_close("piecewise", got.detach().cpu(), want.detach().cpu().numpy(), 1e-5)
