@@ -114,7 +114,8 @@ struct LaunchBuffers {
 
 // ---- launch plans ------------------------------------------------------------------------------------------------
 
-// Plans depend on nothing but these numbers, so they are kept (per thread, bounded).
+// Plans depend on nothing but these numbers, so they are kept (per thread, bounded) and handed out as copies: between
+// a plan and its launch the interpreter may run, and with it another scan on this thread.
 struct PlanKey {
   int32_t B, L, D, in, out, direction, align, ckpt, tune, bwd_tune, keep;
   bool operator==(const PlanKey& o) const { return std::memcmp(this, &o, sizeof(*this)) == 0; }
@@ -131,7 +132,7 @@ struct PlanHash {
 // A forward's `ckpt` says whether it saves states (1) or not (0); their spacing is the tile length of the backward
 // that `bwd_tune` asks for.  A backward's is the spacing the states were saved with.  `keep` < 0: the planner's cache
 // policy; otherwise the most tiles per chain that may leave their operands in the caches.
-const qssm_plan& plan_for(const PlanKey& k) {
+qssm_plan plan_for(const PlanKey& k) {
   static thread_local std::unordered_map<PlanKey, qssm_plan, PlanHash> plans;
   auto it = plans.find(k);
   if (it != plans.end()) return it->second;
@@ -245,7 +246,7 @@ ForwardOut scan_forward(const Tensor& x, const Tensor& a, const Tensor& b, const
   }
   TORCH_CHECK_VALUE(B <= INT32_MAX && L <= INT32_MAX && D <= INT32_MAX, "a dimension of the scan does not fit 32 bits");
   const Operand ox(x, bits), oa(a, bits), ob(b, bits), oc(c, bits);
-  const qssm_plan& plan = plan_for({(int32_t)B, (int32_t)L, (int32_t)D, code_of(x.scalar_type()), out_code, QSSM_FORWARD,
+  const qssm_plan plan = plan_for({(int32_t)B, (int32_t)L, (int32_t)D, code_of(x.scalar_type()), out_code, QSSM_FORWARD,
                                     align_of(bits), want_ckpt, tune, bwd_tune, keep});
   if (want_ckpt) out.ckpt = fresh(B, plan.n_ckpt, D, at::kFloat, x, nullptr);
   out.stride = plan.ckpt_stride;
@@ -293,7 +294,7 @@ Grads scan_backward(const Tensor& x, const Tensor& a, const Tensor& b, const Ten
   const Operand ox(x, bits), oa(a, bits), ob(b, bits), oc(c, bits), og(dy, bits);
   const Operand oh(h.defined() && h.scalar_type() != at::kFloat ? h.to(at::kFloat) : h, bits);
   const Tensor saved = ckpt.defined() ? ckpt.contiguous() : ckpt;
-  const qssm_plan& plan = plan_for({(int32_t)B, (int32_t)L, (int32_t)D, code_of(x.scalar_type()), code_of(dy.scalar_type()),
+  const qssm_plan plan = plan_for({(int32_t)B, (int32_t)L, (int32_t)D, code_of(x.scalar_type()), code_of(dy.scalar_type()),
                                     QSSM_BACKWARD, align_of(bits), (int32_t)(h.defined() ? 0 : ckpt_stride), tune, 0, -1});
   if (saved.defined())
     TORCH_CHECK_VALUE(saved.dim() == 3 && saved.size(0) == B && saved.size(1) == plan.n_ckpt && saved.size(2) == D &&

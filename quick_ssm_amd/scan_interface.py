@@ -65,8 +65,8 @@ def _launch_tiles(shape, tile_b, tile_d) -> List[Tuple[slice, slice]]:
 
 
 class _HipScanFunction(torch.autograd.Function):
-    """Autograd node of the device scan that can loop over tiles (`honor_tiles`); without them `scan` takes
-    `_device_scan`, the same two launches behind a native node.
+    """Autograd node of the device scan that can loop over tiles (`honor_tiles`) and that torch can follow
+    (`_followed_by_torch`); other calls of `scan` take `_device_scan`, the same two launches behind a native node.
 
     Argument list, saved state and returned gradients follow the reference's
     `_TritonScanFunction` (quick_ssm/scan_interface.py:49-158): forward takes
@@ -169,6 +169,86 @@ def _torch_scan(x: Tensor, a: Tensor, b: Tensor, c: Tensor, out_dtype: torch.dty
     return (c * h).to(out_dtype)
 
 
+class _HipScanCarryFunction(torch.autograd.Function):
+    """Autograd node of the device scan with a carried state: (x, a, b, c, h_init) -> (y, h_final), for calls that
+    torch itself follows (`_followed_by_torch`); the others take `_device_scan_chunk`.
+
+    One HIP launch forward, one backward, like `_HipScanFunction`; the backward also takes the
+    gradient arriving at h_final and returns the gradient of h_init, so pieces of a sequence
+    chain through autograd exactly as the whole sequence would.
+    """
+
+    @staticmethod
+    def forward(ctx, x: Tensor, a: Tensor, b: Tensor, c: Tensor, h_init: Optional[Tensor], checkpoint: bool,
+                out_dtype: torch.dtype):
+        if x.shape != a.shape or x.shape != b.shape or x.shape != c.shape:
+            raise ValueError("x, a, b, c must share the same shape [B, L, D].")
+        if x.dim() != 3:
+            raise ValueError("x, a, b, c must be 3-D tensors [B, L, D].")
+        if x.device.type != "cuda":
+            raise RuntimeError("HIP scan backend requires GPU tensors.")
+        B, L, D = x.shape
+        if h_init is not None and tuple(h_init.shape) != (B, D):
+            raise ValueError(f"state must have shape {(B, D)}, got {tuple(h_init.shape)}.")
+        k_in, k_out = hip_scan.kernel_dtypes([x.dtype, a.dtype, b.dtype, c.dtype], out_dtype)
+        xs, as_, bs, cs = (t if t.dtype == k_in else t.to(k_in) for t in (x, a, b, c))
+        h0 = None
+        if h_init is not None:
+            h0 = h_init.detach().to(torch.float32).contiguous()
+            if h0.data_ptr() % 16 != 0:
+                h0 = h0.clone()
+        h_final = torch.empty((B, D), dtype=torch.float32, device=x.device)
+        train = any(ctx.needs_input_grad[:5])   # generation mode saves no states and leaves nothing in the caches
+        y, h_full, ckpt, stride = hip_scan.scan_forward(
+            xs, as_, bs, cs, out_dtype=k_out, want_h=train and not checkpoint, want_ckpt=train and bool(checkpoint),
+            h_init=h0, h_final=h_final,
+        )
+        ctx.save_for_backward(x, a, b, c)
+        ctx.k_in, ctx.k_out = k_in, k_out
+        ctx.h0, ctx.h_saved, ctx.ckpt, ctx.stride = h0, h_full, ckpt, stride
+        ctx.state_dtype = None if h_init is None else h_init.dtype
+        return (y if y.dtype == out_dtype else y.to(out_dtype)), h_final
+
+    @staticmethod
+    def backward(ctx, grad_y: Optional[Tensor], grad_state: Optional[Tensor]):
+        x, a, b, c = ctx.saved_tensors
+        k_in, k_out = ctx.k_in, ctx.k_out
+        B, L, D = x.shape
+        xs, as_, bs, cs = (t if t.dtype == k_in else t.to(k_in) for t in (x, a, b, c))
+        if grad_y is None:
+            grad_y = torch.zeros((B, L, D), dtype=k_out, device=x.device)
+        dy = grad_y if grad_y.dtype == k_out else grad_y.to(k_out)
+        dh_final = None
+        if grad_state is not None:
+            dh_final = grad_state.to(torch.float32).contiguous()
+            if dh_final.data_ptr() % 16 != 0:
+                dh_final = dh_final.clone()
+        need = tuple(ctx.needs_input_grad[:4])
+        dh_init = None
+        if ctx.needs_input_grad[4]:
+            dh_init = torch.empty((B, D), dtype=torch.float32, device=x.device)
+        out = hip_scan.scan_backward(
+            xs, as_, bs, cs, dy, h=ctx.h_saved, ckpt=None if ctx.h_saved is not None else ctx.ckpt,
+            ckpt_stride=ctx.stride, need=need, h_init=ctx.h0, dh_final=dh_final, dh_init=dh_init,
+        )
+
+        def _as(g: Optional[Tensor], like_dtype) -> Optional[Tensor]:
+            if g is None:
+                return None
+            return g if g.dtype == like_dtype else g.to(like_dtype)
+
+        return (_as(out[0], x.dtype), _as(out[1], a.dtype), _as(out[2], b.dtype), _as(out[3], c.dtype),
+                _as(dh_init, ctx.state_dtype), None, None)
+
+
+def _followed_by_torch() -> bool:
+    """Whether a tracer, a functorch transform or forward-mode differentiation is at work: they know of a call only
+    what goes through `torch.autograd.Function` (a trace records it, the others refuse it), while the native node
+    would pass them by: a constant in the trace, a tangent lost without a word."""
+    return (torch._C._get_tracing_state() is not None or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _check_operands(x: Tensor, a: Tensor, b: Tensor, c: Tensor) -> None:
     shape = x.shape
     if shape != a.shape or shape != b.shape or shape != c.shape:
@@ -261,6 +341,8 @@ def scan_chunk(
     if backend == "auto":
         chosen = "hip" if x.device.type == "cuda" else "torch"
     if chosen in ("hip", "triton"):
+        if _followed_by_torch():
+            return _HipScanCarryFunction.apply(x, a, b, c, state, checkpoint, out_dtype)
         return _device_scan_chunk(x, a, b, c, state, checkpoint, out_dtype)
     if chosen == "torch":
         h, final = naive_forward_3d(x, a, b, h_init=state, return_final=True)
@@ -297,7 +379,7 @@ def scan(
     if backend == "auto":
         chosen = "hip" if x.device.type == "cuda" else "torch"
     if chosen in ("hip", "triton"):
-        if _HONOR_TILES:
+        if _HONOR_TILES or _followed_by_torch():
             return _HipScanFunction.apply(x, a, b, c, block_l, checkpoint, tile_b, tile_d, out_dtype)
         return _device_scan(x, a, b, c, checkpoint, out_dtype)
     if chosen == "torch":

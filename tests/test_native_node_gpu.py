@@ -55,3 +55,27 @@ def test_either_output_of_a_piece_may_go_unused(gpu, used, dtypes):
         # float32 arithmetic, one rounding to the operand's own type
         assert_close(name, got.cpu().float(), want.float().numpy(), max(1e-5, torch.finfo(got.dtype).eps))
     assert hip_scan.workspace_status() == 0
+
+
+def test_a_trace_records_the_scan_instead_of_its_result(gpu):
+    first, second = ([t.to(gpu) for t in make_inputs((2, 130, 24), seed=s)[:4]] for s in (1, 2))
+    state = torch.randn(2, 24, generator=torch.Generator().manual_seed(3)).to(gpu)
+    for fn, more in ((lambda x, a, b, c: scan(x, a, b, c), []),
+                     (lambda x, a, b, c, h: scan_chunk(x, a, b, c, h)[0], [state])):
+        traced = torch.jit.trace(fn, (*first, *more), check_trace=False)
+        assert torch.equal(traced(*second, *more), fn(*second, *more))
+
+
+def test_what_the_node_cannot_do_is_refused(gpu):
+    import torch.autograd.forward_ad as fwd
+
+    x, a, b, c = (t.to(gpu) for t in make_inputs((2, 30, 8), seed=1)[:4])
+    calls = (lambda x: scan(x, a, b, c), lambda x: scan_chunk(x, a, b, c)[0])
+    for fn in calls:
+        with fwd.dual_level(), pytest.raises(RuntimeError):
+            fn(fwd.make_dual(x, torch.ones_like(x)))
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda x: fn(x).sum())(x)
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(fn)(torch.stack([x, x]))
+        assert torch.isfinite(fn(x)).all()
