@@ -127,6 +127,46 @@ class _PackedProjection(torch.autograd.Function):
         return (du, *blocks, dbias, None, None)
 
 
+def _bias_gradient(g2: torch.Tensor) -> torch.Tensor:
+    """`column_sum`, or torch's sum where the backward is itself recorded."""
+    return g2.sum(0) if torch.is_grad_enabled() else column_sum(g2)
+
+
+class _WideProjections(torch.autograd.Function):
+    """The five projections of a 16-bit layer in training as one product over their concatenated weights, [.., 5 S] out.
+
+    What it is for is the backward: one product over 5 S k's for the input's gradient instead of five and four additions,
+    and one for all weights, whose five [S, H] products alone leave most of the GPU idle (K is the number of rows).  Unlike
+    `_PackedProjection` the parameters keep their own memory; concatenating them (42 MB at hidden 1024, state 4096) costs
+    a launch of about 20 us.  Layer step, five products -> one, bf16: B=8 L=2048 hidden 512 state 2048 1518 -> 1160 us,
+    B=16 L=1024 hidden 512 state 1024 1171 -> 772, B=2 hidden 1024 state 4096 955 -> 908, B=8 3013 -> 3000; at twice that
+    (B=16, 5718 against 5769) the five products are efficient by themselves (`SSM._WIDE_PRODUCT_LIMIT`)."""
+
+    @staticmethod
+    def forward(ctx, u, w_a, w_b, w_ca, w_cb, w_d, bias_a):
+        weights = (w_a, w_b, w_ca, w_cb, w_d)
+        S = w_a.shape[0]
+        wide_w = torch.cat(weights)                                                   # [5 S, H]
+        wide_b = torch.cat((bias_a, bias_a.new_zeros(4 * S)))
+        ctx.save_for_backward(u, wide_w, *weights)
+        return torch.nn.functional.linear(u, wide_w, wide_b)
+
+    @staticmethod
+    def backward(ctx, g):
+        u, wide_w, *weights = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        S = wide_w.shape[0] // 5
+        g2 = g.reshape(-1, 5 * S)
+        du = None
+        if need[0]:   # a recorded backward has to see the parameters themselves
+            du = (g2 @ (torch.cat(weights) if torch.is_grad_enabled() else wide_w)).view_as(u)
+        blocks = [None] * 5
+        if any(need[1:6]):
+            dw = g2.t() @ u.reshape(-1, u.shape[-1])                                  # [5 S, H]
+            blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
+        return (du, *blocks, _bias_gradient(g2[:, :S]) if need[6] else None)
+
+
 class _SplitProjections(torch.autograd.Function):
     """The five projections of a layer with fp32 parameters as one launch: the outputs share the input's maxima, the
     input's gradient is one product over 5 S k's instead of five products and four additions, and the five weight
@@ -143,7 +183,7 @@ class _SplitProjections(torch.autograd.Function):
         need = ctx.needs_input_grad
         gs = [g.reshape(-1, g.shape[-1]) for g in grads]
         du, dws = _product_gradients(ctx, gs, u, weights, need[0], any(need[1:6]))
-        dbias = column_sum(gs[0]) if need[6] else None
+        dbias = _bias_gradient(gs[0]) if need[6] else None
         return (du, *(dw if need[1 + k] else None for k, dw in enumerate(dws)), dbias)
 
 
@@ -189,6 +229,9 @@ class SSM(nn.Module):
     # Below this many elements per projection output a layer's step is bound by launches, not by their work.
     _BATCHED_PROJECTION_LIMIT = 1 << 23
 
+    # Up to this many, a 16-bit layer in training still takes one product for the five projections (`_WideProjections`).
+    _WIDE_PRODUCT_LIMIT = 1 << 26
+
     def _packed_parameters(self):
         """The five projection weights as one [5 S, H] tensor and a [5 S] bias (A_proj's, then zeros) that ARE the
         parameters' memory: each `nn.Linear.weight` is a row block of the wide tensor, `A_proj.bias` the head of the
@@ -233,13 +276,26 @@ class SSM(nn.Module):
         return _PackedProjection.apply(u, self.A_proj.weight, self.B_proj.weight, self.C_proj_a.weight,
                                        self.C_proj_b.weight, self.D_proj.weight, self.A_proj.bias, wide_w, wide_b)
 
-    def _five_projections(self, u: torch.Tensor):
-        """The five projection outputs of a large layer (blocks in A, B, C_a, C_b, D order)."""
+    def _projections(self):
+        """The five projections in A, B, C_a, C_b, D order, and whether their calls are nothing but products."""
         mods = (self.A_proj, self.B_proj, self.C_proj_a, self.C_proj_b, self.D_proj)
-        if (all(_plain_linear(m) for m in mods) and not nn.modules.module._has_any_global_hook()
-                and split_linear.usable(u.reshape(-1, u.shape[-1]), [m.weight for m in mods])
-                and self.A_proj.bias is not None and all(m.bias is None for m in mods[1:])):
-            return _SplitProjections.apply(u, *(m.weight for m in mods), self.A_proj.bias)
+        plain = (all(_plain_linear(m) for m in mods) and not nn.modules.module._has_any_global_hook()
+                 and self.A_proj.bias is not None and all(m.bias is None for m in mods[1:]))
+        return mods, plain
+
+    def _large_projections(self, u: torch.Tensor):
+        """The projection outputs of a layer above `_BATCHED_PROJECTION_LIMIT`: five tensors (blocks in A, B, C_a, C_b, D
+        order), or one [.., 5 S] tensor for a 16-bit layer in training."""
+        mods, plain = self._projections()
+        if plain and u.is_cuda:
+            weights, bias = [m.weight for m in mods], self.A_proj.bias
+            if split_linear.usable(u.reshape(-1, u.shape[-1]), weights):
+                return _SplitProjections.apply(u, *weights, bias)
+            if (u.dtype in (torch.float16, torch.bfloat16) and all(t.dtype == u.dtype for t in (*weights, bias))
+                    and 0 < u.numel() // self.hidden_size * self.state_size_dim <= self._WIDE_PRODUCT_LIMIT
+                    and torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
+                    and (u.requires_grad or any(t.requires_grad for t in (*weights, bias)))):
+                return _WideProjections.apply(u, *weights, bias)
         return tuple(m(u) for m in mods)
 
     def gates(self, u: torch.Tensor):
@@ -275,11 +331,12 @@ class SSM(nn.Module):
             # 16-bit projections stored as the compute dtype, or fp32 projections with fp32 y: the activations (and the
             # casts to the compute dtype) happen inside the scan's launches
             wide = self._wide_projection(u)
+            pre = () if wide is not None else self._large_projections(u)
+            if torch.is_tensor(pre):
+                wide = pre
             if wide is not None:
                 S = self.state_size_dim
                 pre = tuple(wide[..., k * S:(k + 1) * S] for k in range(5))
-            else:
-                pre = self._five_projections(u)
             if wide is not None and wide.dim() == 3 and _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
                 y = _gated.gated_scan_wide(wide, out_dtype=out_dtype, compute_dtype=self.compute_dtype)
             elif _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
