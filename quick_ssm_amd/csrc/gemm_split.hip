@@ -328,15 +328,15 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const SplitGemmArgs p
 // Largest magnitude (as the bits of its absolute value, which order like integers, NaN above infinity) of the rows and
 // columns of a block of one of the matrices.  A workgroup takes `block_rows` rows of 256 * Q columns, a quarter of the
 // rows per wavefront; its columns' maxima stay in registers over the rows.  Every block writes words of its own, and the
-// product that reads them takes the largest: no atomics and nothing to clear beforehand.  Bound by memory: eight 16-byte
+// product that reads them takes the largest: no atomics and nothing to clear beforehand.  Bound by memory: sixteen 16-byte
 // loads per lane are in flight.
 template <int Q>
 __device__ __forceinline__ void amax_block(const AmaxMatrix& x, int block, unsigned (*cols_lds)[1024]) {
-  constexpr int RU = 8 / Q;   // rows at a time
+  constexpr int RU = 16 / Q;   // rows at a time
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int cb = block % x.col_blocks, rb = block / x.col_blocks;
   const int c0 = cb * (256 * Q);
-  const int per_wave = x.block_rows / 4;   // a multiple of 8
+  const int per_wave = x.block_rows / 4;   // a multiple of 16
   const int64_t r0 = (int64_t)rb * x.block_rows + wave * per_wave;
   uint4v cm[Q];
 #pragma unroll
@@ -433,7 +433,7 @@ void amax_shape(int64_t rows, int cols, AmaxMatrix* m) {
   const int width = m->wide ? 1024 : 256;
   m->col_blocks = (cols + width - 1) / width;
   const int64_t per = rows < 128 * 64 ? 128 : (rows + 63) / 64;
-  m->block_rows = (int)((per + 31) / 32 * 32);
+  m->block_rows = (int)((per + 63) / 64 * 64);
   m->row_blocks = (int)((rows + m->block_rows - 1) / m->block_rows);
   m->blocks = m->row_blocks * m->col_blocks;
 }
