@@ -415,6 +415,10 @@ QSSM_API int qssm_gates_backward_strided(const void* g_a, const void* g_x, const
 QSSM_API int qssm_plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype,
                          int32_t out_dtype, int32_t direction, int32_t align_elems, int32_t ckpt_stride,
                          qssm_plan* plan);
+/* The same with clusters of up to eight tiles instead of two, for few chains over a long sequence. */
+QSSM_API int qssm_plan_scan_gated_long(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype,
+                         int32_t out_dtype, int32_t direction, int32_t align_elems, int32_t ckpt_stride,
+                         qssm_plan* plan);
 
 QSSM_API int qssm_scan_gated_forward(const qssm_plan* plan,
                             const void* A_pre, qssm_strides sA,

@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "qssm_scan_forward_call",
     "qssm_scan_backward_call",
     "qssm_plan_scan_gated",
+    "qssm_plan_scan_gated_long",
     "qssm_scan_gated_forward",
     "qssm_scan_gated_backward",
     "qssm_gates_forward",
@@ -179,6 +180,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     )
     lib.qssm_plan_scan_gated.restype = ctypes.c_int
     lib.qssm_plan_scan_gated.argtypes = [i32] * 9 + [ctypes.POINTER(Plan)]
+    lib.qssm_plan_scan_gated_long.restype = ctypes.c_int
+    lib.qssm_plan_scan_gated_long.argtypes = [i32] * 9 + [ctypes.POINTER(Plan)]
     lib.qssm_scan_gated_forward.restype = ctypes.c_int
     lib.qssm_scan_gated_forward.argtypes = (
         [ctypes.POINTER(Plan)] + [vp, Strides] * 6 + [vp] + [vp, u64, vp, u64, ctypes.c_uint32, vp]

@@ -88,6 +88,7 @@ static bool aligned_to(const void* p, int64_t sb, int64_t sl, int elem_bytes, in
 
 static const int kMaxThreads = 1024;
 static const int kMaxLdsBytes = 64 * 1024;
+static const int kGatedLdsBytes = 80 * 1024;   // the gated backward: half of a compute unit's LDS
 static const int kCUs = 256;
 static const uint64_t kKeepBytes = 224ull << 20;  // operand bytes a forward leaves in the caches for its backward
 
@@ -212,6 +213,9 @@ static int backward_launch(const qssm_plan* plan, const void* x, qssm_strides sx
 static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
                      int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan);
 
+static int plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype, int32_t out_dtype,
+                           int32_t direction, int32_t align_elems, int32_t ckpt_stride, int most, qssm_plan* plan);
+
 extern "C" {
 
 int qssm_version(void) { return QSSM_VERSION; }
@@ -223,11 +227,38 @@ int qssm_plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t ou
   return qssm_plan_scan_tuned(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, 0, plan);
 }
 
-// The gated kernels exist in one shape: 4 columns (8 bytes of 16-bit storage) and 8 steps per lane, 256 lanes,
-// rows of 64 or 32 lanes, clusters of at most two tiles (the backward's three LDS-resident operands leave LDS
-// for no more neighbour maps).
 int qssm_plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype, int32_t out_dtype,
                          int32_t direction, int32_t align_elems, int32_t ckpt_stride, qssm_plan* plan) {
+  return plan_scan_gated(B, L, D, dtype, compute_dtype, out_dtype, direction, align_elems, ckpt_stride, 1, plan);
+}
+
+// Clusters of up to eight tiles (75 KB of LDS for the backward, which still lets two workgroups share a compute unit, as
+// many as its registers do), where the planner's estimate asks for them: few chains over a long sequence, whose
+// hand-overs set the pace.  Clusters of two -> these, forward and backward: bf16 B=1 L=4096 S=1024 71 -> 32 and 79 -> 38 us,
+// B=1 L=2048 S=4096 41 -> 30 and 54 -> 51, fp32 projections B=1 L=4096 S=1024 67 -> 31 and 72 -> 45, B=2 L=2048 S=512 34 -> 19
+// and 40 -> 23; where the estimate asks for four (B=4 L=1024 S=2048, fp32 B=8 L=2048 S=1024) the same within 3 %.
+int qssm_plan_scan_gated_long(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype, int32_t out_dtype,
+                              int32_t direction, int32_t align_elems, int32_t ckpt_stride, qssm_plan* plan) {
+  return plan_scan_gated(B, L, D, dtype, compute_dtype, out_dtype, direction, align_elems, ckpt_stride, 3, plan);
+}
+
+int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
+                         int32_t align_elems, int32_t ckpt_stride, int32_t tune, qssm_plan* plan) {
+  return plan_scan(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, false, plan);
+}
+
+int qssm_plan_scan_loose(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
+                         int32_t align_elems, int32_t ckpt_stride, int32_t tune, qssm_plan* plan) {
+  return plan_scan(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, true, plan);
+}
+
+}  // extern "C"
+
+// The gated kernels exist in one shape: 4 columns (8 bytes of 16-bit storage) and 8 steps per lane, 256 lanes,
+// rows of 64 or 32 lanes, clusters of at most two tiles unless the caller takes more LDS than 64 KB.
+// `most` = log2 of the longest cluster.
+static int plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype, int32_t out_dtype,
+                           int32_t direction, int32_t align_elems, int32_t ckpt_stride, int most, qssm_plan* plan) {
   const int es = dtype_size(dtype);
   if (es == 0 || dtype_size(compute_dtype) == 0) return fail(QSSM_EINVAL, "unknown dtype code");
   if (es == 2 && compute_dtype != dtype)
@@ -253,28 +284,16 @@ int qssm_plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t
   if (g_log2 != plan->g_log2 || ckpt_stride != 0)
     rc = qssm_plan_scan_tuned(B, L, D, dtype, out_dtype, direction, align_elems, ckpt_stride,
                               kGatedTune | (g_log2 + 1), plan);
-  if (rc == 0 && plan->cluster > 2)   // same strips, more hand-overs, less LDS
+  if (rc == 0 && plan->cluster > (1 << most))   // same strips, more hand-overs, less LDS
     rc = qssm_plan_scan_tuned(B, L, D, dtype, out_dtype, direction, align_elems, ckpt_stride,
-                              kGatedTune | (g_log2 + 1) | (2 << 28), plan);
+                              kGatedTune | (g_log2 + 1) | ((most + 1) << 28), plan);
   if (rc != 0) return rc;
   plan->compute_dtype = compute_dtype;
   if (plan->vec != vec || plan->steps != 8 || plan->threads != 256 || (plan->g_log2 != 6 && plan->g_log2 != 5) ||
-      plan->cluster > 2)
+      plan->cluster > (1 << most))
     return fail(QSSM_EINVAL, "no gated geometry for this shape");
   return 0;
 }
-
-int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
-                         int32_t align_elems, int32_t ckpt_stride, int32_t tune, qssm_plan* plan) {
-  return plan_scan(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, false, plan);
-}
-
-int qssm_plan_scan_loose(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
-                         int32_t align_elems, int32_t ckpt_stride, int32_t tune, qssm_plan* plan) {
-  return plan_scan(B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, true, plan);
-}
-
-}  // extern "C"
 
 static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
                      int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan) {
@@ -727,7 +746,7 @@ static int backward_launch(const qssm_plan* plan, const void* x, qssm_strides sx
     if (!cg_in_lds || h != nullptr || gate->c2 == nullptr || ((uintptr_t)gate->c2) % 16 != 0 || (gate->sc2.b * es) % 16 != 0 ||
         (gate->sc2.l * es) % 16 != 0 || !tile_span_ok(plan, gate->c2, gate->sc2.b, gate->sc2.l, es) ||
         !aligned_to(gate->dc2, gate->sdc2.b, gate->sdc2.l, es, v) || !tile_span_ok(plan, gate->dc2, gate->sdc2.b, gate->sdc2.l, es) ||
-        lds + one > (size_t)kMaxLdsBytes)
+        lds + one > (size_t)kGatedLdsBytes)
       return fail(QSSM_EALIGN, "gated scan needs a plan of qssm_plan_scan_gated, dy stored as the projections are, saved "
                                "states, and Ca, Cb, dy with 16-byte aligned rows");
     lds += one;

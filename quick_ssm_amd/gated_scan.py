@@ -58,13 +58,14 @@ def supported(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype: torc
 
 
 def _plan(B: int, L: int, S: int, dtype: torch.dtype, compute_dtype: torch.dtype, out_dtype: torch.dtype,
-          direction: int, ckpt_stride: int) -> Plan:
-    key = (B, L, S, dtype, compute_dtype, out_dtype, direction, ckpt_stride)
+          direction: int, ckpt_stride: int, long: bool = False) -> Plan:
+    key = (B, L, S, dtype, compute_dtype, out_dtype, direction, ckpt_stride, long)
     plan = _plans.get(key)
     if plan is None:
         plan = Plan()
-        _lib.check(_lib.load().qssm_plan_scan_gated(B, L, S, _CODES[dtype], _CODES[compute_dtype], _CODES[out_dtype],
-                                                    direction, 8, ckpt_stride, ctypes.byref(plan)))
+        planner = _lib.load().qssm_plan_scan_gated_long if long else _lib.load().qssm_plan_scan_gated
+        _lib.check(planner(B, L, S, _CODES[dtype], _CODES[compute_dtype], _CODES[out_dtype], direction, 8, ckpt_stride,
+                           ctypes.byref(plan)))
         if len(_plans) >= 1024:
             _plans.clear()
         _plans[key] = plan
@@ -92,7 +93,7 @@ def _forward_launch(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype
     dev, dtype = A_pre.device, A_pre.dtype
     # the backward's tile length decides how far apart the saved states are; it takes dy stored as the projections are
     stride = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, 0).seg_len
-    plan = _plan(B, L, S, dtype, compute_dtype, out_dtype, _lib.QSSM_FORWARD, stride)
+    plan = _plan(B, L, S, dtype, compute_dtype, out_dtype, _lib.QSSM_FORWARD, stride, True)
     keep = hip_scan._forward_keep if train else False
     if keep is not True:
         plan = Plan.from_buffer_copy(plan)   # cached plans are shared: change a copy
@@ -118,7 +119,7 @@ def _backward_launch(pre: Sequence[Tensor], compute_dtype: torch.dtype, grad_y: 
     dA, dB, dCa, dCb, dD = grads
     B, L, S = A_pre.shape
     dtype = A_pre.dtype
-    plan = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, stride)
+    plan = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, stride, True)
     _launch(plan, A_pre.device, _lib.load().qssm_scan_gated_backward,
             A_pre.data_ptr(), _st(A_pre), B_in.data_ptr(), _st(B_in), Ca.data_ptr(), _st(Ca), Cb.data_ptr(), _st(Cb),
             D_pre.data_ptr(), _st(D_pre), grad_y.data_ptr(), _st(grad_y), ckpt.data_ptr(),
