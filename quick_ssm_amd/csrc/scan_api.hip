@@ -991,8 +991,8 @@ int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int32_t dtyp
 int qssm_split_gemm_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments) {
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || segments <= 0) return 1;
   // Two workgroups per compute unit run at once.  A launch takes whole rounds of them, each as long as its stages of
-  // 16 k's (plus about 24 stages' worth to fill and drain a workgroup); every further part writes and reads C once
-  // more, which costs about as much as 1 / 40 of a round per 2 MB.
+  // 16 k's, and about 24 stages' worth to fill and drain a workgroup (a round of 16 stages takes 36 us where a stage takes
+  // 1.5); every further part writes and reads C once more, at kSplitPartCost stages per MB.
   const double tiles = (double)split_gemm_tiles(M, N, batch), stages = (double)split_gemm_stages(K, segments);
   const double out_mb = (double)M * N * batch * 4e-6;
   int best = 1;

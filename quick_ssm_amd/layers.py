@@ -60,14 +60,21 @@ def column_sum(g2: torch.Tensor) -> torch.Tensor:
 
 
 def _products(ctx, u: torch.Tensor, weights, biases):
-    """u w^T + bias for every weight, inside an autograd function's forward: split products where they apply (the
-    maxima the backward wants are saved in `ctx.maxima`), else torch's."""
+    """u w^T + bias for every weight as split products, inside an autograd function's forward; the maxima the backward
+    wants are saved in `ctx.maxima`."""
     u2 = u.reshape(-1, u.shape[-1])
-    if not split_linear.usable(u2, weights):
-        ctx.maxima = None
-        return [torch.nn.functional.linear(u, w, b) for w, b in zip(weights, biases)]
     outs, ctx.maxima = split_linear.forward(u2, weights, biases, ctx.needs_input_grad[0], any(ctx.needs_input_grad[1:]))
     return [t.view(*u.shape[:-1], t.shape[-1]) for t in outs]
+
+
+def _product(ctx, u: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """One of them, as a split product where that applies, else torch's.  (Small layers are bound by the interpreter: a
+    16-bit one gets no further than its type.)"""
+    if (u.dtype is torch.float32 and u.numel() * weight.shape[0] >= split_linear.MIN_WORK
+            and split_linear.usable(u, (weight,))):
+        return _products(ctx, u, (weight,), (bias,))[0]
+    ctx.maxima = None
+    return torch.nn.functional.linear(u, weight, bias)
 
 
 def _product_gradients(ctx, grads, u: torch.Tensor, weights, need_du: bool, need_dw: bool):
@@ -92,14 +99,18 @@ class _LinearBias(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, weight, bias):
         ctx.save_for_backward(u, weight)
-        return _products(ctx, u, [weight], [bias])[0]
+        return _product(ctx, u, weight, bias)
 
     @staticmethod
     def backward(ctx, g):
         u, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
         g2 = g.reshape(-1, g.shape[-1])
-        du, (dw,) = _product_gradients(ctx, [g2], u, [weight], need[0], need[1])
+        if ctx.maxima is not None:
+            du, (dw,) = _product_gradients(ctx, [g2], u, [weight], need[0], need[1])
+        else:
+            du = (g2 @ weight).view_as(u) if need[0] else None
+            dw = g2.t() @ u.reshape(-1, u.shape[-1]) if need[1] else None
         db = column_sum(g2) if need[2] else None
         return du, dw, db
 
@@ -113,7 +124,7 @@ class _PackedProjection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, w_a, w_b, w_ca, w_cb, w_d, bias_a, wide_w, wide_b):
         ctx.save_for_backward(u, wide_w)
-        return _products(ctx, u, [wide_w], [wide_b])[0]
+        return _product(ctx, u, wide_w, wide_b)
 
     @staticmethod
     def backward(ctx, g):
@@ -121,8 +132,14 @@ class _PackedProjection(torch.autograd.Function):
         need = ctx.needs_input_grad
         S = wide_w.shape[0] // 5
         g2 = g.reshape(-1, g.shape[-1])
-        du, (dw,) = _product_gradients(ctx, [g2], u, [wide_w], need[0], any(need[1:6]))      # dw: [5 S, H]
-        blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
+        blocks = [None] * 5
+        if ctx.maxima is not None:
+            du, (dw,) = _product_gradients(ctx, [g2], u, [wide_w], need[0], any(need[1:6]))
+        else:
+            du = (g2 @ wide_w).view_as(u) if need[0] else None
+            dw = g2.t() @ u.reshape(-1, u.shape[-1]) if any(need[1:6]) else None              # [5 S, H]
+        if dw is not None:
+            blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
         dbias = column_sum(g2[:, :S]) if need[6] else None
         return (du, *blocks, dbias, None, None)
 
@@ -284,19 +301,19 @@ class SSM(nn.Module):
         return mods, plain
 
     def _large_projections(self, u: torch.Tensor):
-        """The projection outputs of a layer above `_BATCHED_PROJECTION_LIMIT`: five tensors (blocks in A, B, C_a, C_b, D
-        order), or one [.., 5 S] tensor for a 16-bit layer in training."""
+        """The projection outputs of a layer above `_BATCHED_PROJECTION_LIMIT`: one [.., 5 S] tensor for a 16-bit layer in
+        training, or None and the five tensors (blocks in A, B, C_a, C_b, D order)."""
         mods, plain = self._projections()
         if plain and u.is_cuda:
             weights, bias = [m.weight for m in mods], self.A_proj.bias
-            if split_linear.usable(u.reshape(-1, u.shape[-1]), weights):
-                return _SplitProjections.apply(u, *weights, bias)
+            if split_linear.usable(u, weights):
+                return None, _SplitProjections.apply(u, *weights, bias)
             if (u.dtype in (torch.float16, torch.bfloat16) and all(t.dtype == u.dtype for t in (*weights, bias))
                     and 0 < u.numel() // self.hidden_size * self.state_size_dim <= self._WIDE_PRODUCT_LIMIT
                     and torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
                     and (u.requires_grad or any(t.requires_grad for t in (*weights, bias)))):
-                return _WideProjections.apply(u, *weights, bias)
-        return tuple(m(u) for m in mods)
+                return _WideProjections.apply(u, *weights, bias), None
+        return None, tuple(m(u) for m in mods)
 
     def gates(self, u: torch.Tensor):
         """The scan's four operands (x, a, b, c) from the normalised input, in `compute_dtype`."""
@@ -331,9 +348,8 @@ class SSM(nn.Module):
             # 16-bit projections stored as the compute dtype, or fp32 projections with fp32 y: the activations (and the
             # casts to the compute dtype) happen inside the scan's launches
             wide = self._wide_projection(u)
-            pre = () if wide is not None else self._large_projections(u)
-            if torch.is_tensor(pre):
-                wide = pre
+            if wide is None:
+                wide, pre = self._large_projections(u)
             if wide is not None:
                 S = self.state_size_dim
                 pre = tuple(wide[..., k * S:(k + 1) * S] for k in range(5))

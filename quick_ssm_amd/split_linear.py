@@ -17,10 +17,11 @@ from . import hip_scan
 Tensor = torch.Tensor
 
 # Multiply-adds (over all weights of a launch) below which the library's product stays, because the fixed costs of the
-# maxima, the prologue and the sums over parts exceed the gain.  us for output, input gradient and weight gradient
-# together, library against these: 4096 rows, 1024 x 256 (1.1e9) 79 against 129; 4096 rows, 256 x 5120 (5.4e9) 335
-# against 250; 8192 rows, 512 x 5 * 1024 (2.1e10) 1042 against 588.
-MIN_WORK = 1 << 32
+# maxima, the prologue, the sums over parts and their launches exceed the gain.  us for output, input gradient and weight
+# gradient together, library against these: 4096 rows, 1024 x 256 (1.1e9) 79 against 129; 4096 rows, 256 x 5120 (5.4e9)
+# 335 against 250 on the GPU, but twice the launches, and a layer of that size is bound by its host (617 us a step against
+# 660); 2048 rows, 512 x 10240 (1.1e10) a layer step of 705 against 625; 8192 rows, 512 x 5 * 1024 (2.1e10) 1042 against 588.
+MIN_WORK = 1 << 33
 
 
 class Maxima(NamedTuple):
@@ -37,12 +38,13 @@ def _matrix_ok(t: Tensor) -> bool:
 
 
 def usable(u: Tensor, weights: Sequence[Tensor]) -> bool:
-    """Whether u [rows, K] times the transposes of the weights [N, K] may take the split products."""
-    if u.dtype is not torch.float32 or not u.is_cuda or torch.is_autocast_enabled("cuda"):
-        return False
+    """Whether u [.., K] times the transposes of the weights [N, K] may take the split products."""
     n, k = weights[0].shape
-    rows = u.shape[0]
-    if n % 4 or k % 4 or rows * n * k * len(weights) < MIN_WORK or rows >= 1 << 31 or not _matrix_ok(u):
+    if u.dtype is not torch.float32 or u.numel() * n * len(weights) < MIN_WORK:
+        return False
+    if not u.is_cuda or torch.is_autocast_enabled("cuda") or n % 4 or k % 4 or u.numel() // k >= 1 << 31:
+        return False
+    if not _matrix_ok(u.reshape(-1, k)):
         return False
     return all(_matrix_ok(w) and w.shape == (n, k) and w.stride(0) == weights[0].stride(0) and w.device == u.device
                for w in weights)
