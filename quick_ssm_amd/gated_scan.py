@@ -79,10 +79,10 @@ def _st(t: Tensor) -> Strides:
 def _launch(plan: Plan, dev: torch.device, fn, *args) -> None:
     with torch.cuda.device(dev):
         stream = hip_scan._raw_stream(dev.index)
-        buf, epoch, capturing = hip_scan._launch_buffers(dev, dev.index, stream, int(plan.control_bytes),
-                                                         int(plan.workspace_bytes))
-        _lib.check(fn(ctypes.byref(plan), *args, buf.ctl_ptr, buf.ctl_size, buf.ws_ptr, buf.ws_size, epoch, stream))
-        hip_scan._after_launch(buf, stream, capturing)
+        taken, epoch, capturing = hip_scan._launch_buffers(dev, dev.index, stream, int(plan.control_bytes),
+                                                           int(plan.workspace_bytes))
+        _lib.check(fn(ctypes.byref(plan), *args, *taken[3:], epoch, stream))
+        hip_scan._after_launch(taken, stream, capturing)
 
 
 def _forward_launch(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype: torch.dtype, train: bool = True):

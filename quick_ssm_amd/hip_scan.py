@@ -223,9 +223,13 @@ def _recover(buf: _Buffers, stream: int) -> int:
     return status
 
 
-def _number_launch(device: torch.device, dev_index: int, stream: int, need_c: int, need_w: int):
-    """Buffers and number of the next launch on (device, stream): (entry, control, workspace, their addresses and
-    sizes, epoch argument, capturing).
+# (entry, control block, workspace, their addresses and sizes in turn): what one launch works with.  The launch holds
+# the two tensors until it is on its stream; the entry may have been given others by then.
+_Taken = Tuple[_Buffers, Tensor, Tensor, int, int, int, int]
+
+
+def _launch_buffers(device: torch.device, dev_index: int, stream: int, need_c: int, need_w: int) -> Tuple[_Taken, int, bool]:
+    """Buffers and epoch argument of the next launch on (device, stream), and whether the stream is capturing.
 
     Both buffers are zero-filled when they are allocated (torch.zeros runs a fill kernel on the
     current stream, ahead of the launch that uses them) and grown on demand.  Every launch leaves
@@ -244,6 +248,7 @@ def _number_launch(device: torch.device, dev_index: int, stream: int, need_c: in
     # the caller's thread and a backward on autograd's thread may launch on one stream at the same time, and two
     # launches with one number would read each other's words as their own.  The addresses are read in the same step:
     # a larger launch on the other thread replaces the tensors, and a number only means something to its own buffers.
+    # Callers pass on these addresses, never the entry's.
     with _ws_lock:
         buf = _buffers.get(key)
         if buf is None or buf.ctl_size < need_c or buf.ws_size < need_w or buf.epoch >= _EPOCH_MAX:
@@ -256,16 +261,10 @@ def _number_launch(device: torch.device, dev_index: int, stream: int, need_c: in
             if not on_device:
                 buf.epoch += 1
                 epoch = buf.epoch
-        taken = (buf, buf.control, buf.workspace, buf.ctl_ptr, buf.ctl_size, buf.ws_ptr, buf.ws_size, epoch, capturing)
+        taken = (buf, buf.control, buf.workspace, buf.ctl_ptr, buf.ctl_size, buf.ws_ptr, buf.ws_size)
     if failed:
         raise ScanLaunchError(_recover(buf, stream), buf.where)
-    return taken
-
-
-def _launch_buffers(device: torch.device, dev_index: int, stream: int, need_c: int, need_w: int) -> Tuple[_Buffers, int, bool]:
-    """Entry, epoch argument and whether the stream is capturing, for the next launch on (device, stream)."""
-    taken = _number_launch(device, dev_index, stream, need_c, need_w)
-    return taken[0], taken[7], taken[8]
+    return taken, epoch, capturing
 
 
 def _status_check_due(buf: _Buffers, capturing: bool) -> bool:
@@ -280,10 +279,11 @@ def _status_check_due(buf: _Buffers, capturing: bool) -> bool:
     return due
 
 
-def _after_launch(buf: _Buffers, stream: int, capturing: bool) -> None:
+def _after_launch(taken: _Taken, stream: int, capturing: bool) -> None:
     """Every `_check_every`-th launch: ask for the status word, to be looked at before a later launch."""
+    buf = taken[0]
     if _status_check_due(buf, capturing):
-        _lib.check(_lib.load().qssm_control_status_async(buf.ctl_ptr, buf.pinned.data_ptr(), stream))
+        _lib.check(_lib.load().qssm_control_status_async(taken[3], buf.pinned.data_ptr(), stream))
 
 
 _devices: Dict[int, torch.device] = {}
@@ -296,7 +296,7 @@ def _take_launch(dev_index: int, stream: int, need_c: int, need_w: int) -> tuple
     device = _devices.get(dev_index)
     if device is None:
         device = _devices[dev_index] = torch.device("cuda", dev_index)
-    buf, control, workspace, cp, cs, wp, ws, epoch, capturing = _number_launch(device, dev_index, stream, need_c, need_w)
+    (buf, control, workspace, cp, cs, wp, ws), epoch, capturing = _launch_buffers(device, dev_index, stream, need_c, need_w)
     status_to = buf.pinned.data_ptr() if _status_check_due(buf, capturing) else 0
     return cp, cs, wp, ws, epoch, status_to, control, workspace
 

@@ -405,6 +405,63 @@ def test_launches_from_several_threads_get_distinct_numbers(monkeypatch):
     assert len(asked) == total // 7 and buf.since_check == total % 7
 
 
+def test_a_gated_launch_uses_the_buffers_its_number_was_taken_for(monkeypatch):
+    # Replacing the buffers of a stream by larger ones restarts the numbers.  A launch whose number and addresses came
+    # from different buffers would meet its own number again in theirs, and one whose buffers nobody holds would write
+    # to freed memory.  Here another thread's larger launch falls between taking the number and launching.
+    import contextlib
+    import weakref
+
+    from quick_ssm_amd import gated_scan
+
+    stream, dev = 0x5678, torch.device("cpu", 0)
+    monkeypatch.setattr(torch._C, "_cuda_isCurrentStreamCapturing", lambda: False, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: stream, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "device", lambda dev: contextlib.nullcontext())
+    asked = []
+    monkeypatch.setattr(hip_scan._lib, "load", lambda: type("L", (), {
+        "qssm_control_status_async": staticmethod(lambda *a: asked.append(a) or 0)})())
+    old_period = hip_scan.set_status_check_period(1)
+    key = (0, stream, False)
+    buf = _FakeBuffers()
+    buf.ctl_size = buf.ws_size = 0
+    buf.pinned = type("P", (), {"data_ptr": staticmethod(lambda: 0)})()
+    hip_scan._buffers[key] = buf
+    real = hip_scan._launch_buffers
+    need = 1 << 17
+    numbered = []
+
+    def interrupted(*args):
+        nonlocal need
+        taken = real(*args)
+        numbered.append((buf.ctl_ptr, buf.ws_ptr, taken[1], weakref.ref(buf.control), weakref.ref(buf.workspace)))
+        need *= 4
+        real(dev, 0, stream, need, need * 8)
+        assert buf.ctl_ptr != numbered[-1][0] and buf.ws_ptr != numbered[-1][1]
+        return taken
+
+    monkeypatch.setattr(hip_scan, "_launch_buffers", interrupted)
+    launched = []
+
+    def fake_launch(plan, cp, cs, wp, ws, epoch, on):
+        control, workspace = numbered[-1][3](), numbered[-1][4]()
+        assert control is not None and control.numel() == cs and workspace is not None and workspace.numel() == ws
+        launched.append((cp, wp, epoch))
+        return 0
+
+    plan = _lib.Plan()
+    plan.control_bytes, plan.workspace_bytes = 64, 1024
+    try:
+        for _ in range(4):
+            gated_scan._launch(plan, dev, fake_launch)
+    finally:
+        hip_scan.set_status_check_period(old_period)
+        hip_scan._buffers.pop(key, None)
+    assert launched == [n[:3] for n in numbered] and len(launched) == 4
+    assert [a[0] for a in asked] == [n[0] for n in numbered]     # and the status of the block it ran with is asked for
+
+
 def test_device_side_launch_count_never_repeats_a_flag_between_wipes(hip_lib):
     # Launches that number themselves (epoch argument 0) use flag count + 1 and the counting kernel stores the
     # next count.  Walk the arithmetic across both wraps: no flag is ever zero, flags grow by one between restarts,
