@@ -17,7 +17,7 @@ namespace qssm {
 
 namespace {
 
-constexpr int kBM = 256, kBN = 128, kBK = 16;
+constexpr int kBM = kSplitTileM, kBN = kSplitTileN, kBK = 16;
 constexpr int kPlaneA = kBM * kBK * 2, kPlaneB = kBN * kBK * 2;   // bytes of one fp16 plane of a stage
 constexpr int kStage = 2 * (kPlaneA + kPlaneB);
 constexpr unsigned kInfBits = 0x7f800000u;

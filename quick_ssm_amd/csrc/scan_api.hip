@@ -1011,6 +1011,9 @@ int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
   if (k->batch < 1 || k->batch > QSSM_SPLIT_MANY || k->segments < 1 || k->segments > QSSM_SPLIT_MANY ||
       (k->batch > 1 && k->segments > 1))
     return fail(QSSM_EINVAL, "1 to %d products, or runs of k of one product", QSSM_SPLIT_MANY);
+  // (the kernel counts rows and columns up to the end of the last tile in 32 bits)
+  if (k->M > 0x7fffffff - kSplitTileM || k->N > 0x7fffffff - kSplitTileN)
+    return fail(QSSM_EINVAL, "M and N must leave room for a tile below 2^31");
   if (k->splits < 1 || k->splits > 64) return fail(QSSM_EINVAL, "splits must be 1 to 64");
   if (k->a_kstrided && !k->b_kstrided) return fail(QSSM_EINVAL, "a k-strided A needs a k-strided B");
   if (k->M == 0 || k->N == 0) return 0;

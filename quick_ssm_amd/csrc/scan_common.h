@@ -570,6 +570,7 @@ bool launch_colsum_any(int dtype, const void* x, int64_t ld, int64_t rows, int S
 
 // ---- fp32 products on the 16-bit matrix cores (gemm_split.hip) -----------------------------------------------------
 constexpr int kSplitGemmMany = 5;   // products (or runs of k) of one launch
+constexpr int kSplitTileM = 256, kSplitTileN = 128;   // rows and columns of a workgroup's tile
 
 struct SplitGemmArgs {
   const float *a[kSplitGemmMany], *b[kSplitGemmMany];  // one pair per product, or per run of k

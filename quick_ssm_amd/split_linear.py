@@ -23,6 +23,9 @@ Tensor = torch.Tensor
 # 660); 2048 rows, 512 x 10240 (1.1e10) a layer step of 705 against 625; 8192 rows, 512 x 5 * 1024 (2.1e10) 1042 against 588.
 MIN_WORK = 1 << 33
 
+# Most rows and outputs: the kernel counts to the end of its last tile of 256 in 32 bits.
+MAX_ROWS = (1 << 31) - 1 - 256
+
 
 class Maxima(NamedTuple):
     """What the backward needs of the operands: bits of the largest magnitude of every column of the input, and of
@@ -42,7 +45,9 @@ def usable(u: Tensor, weights: Sequence[Tensor]) -> bool:
     n, k = weights[0].shape
     if u.dtype is not torch.float32 or u.numel() * n * len(weights) < MIN_WORK:
         return False
-    if not u.is_cuda or torch.is_autocast_enabled("cuda") or n % 4 or k % 4 or u.numel() // k >= 1 << 31:
+    if not u.is_cuda or torch.is_autocast_enabled("cuda") or n % 4 or k % 4:
+        return False
+    if u.numel() // k > MAX_ROWS or n > MAX_ROWS:
         return False
     if not _matrix_ok(u.reshape(-1, k)):
         return False
