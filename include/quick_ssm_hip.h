@@ -486,50 +486,32 @@ QSSM_API int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int
                          int32_t partial_rows, void* out, void* stream);
 
 /*
- * fp32 products on the 16-bit matrix cores: C_i(m, n) = sum over k of A_i(m, k) B_i(n, k) (+ bias_i(n)) for up to
- * QSSM_SPLIT_MANY products of one shape, or the sum of up to QSSM_SPLIT_MANY runs of K k's as one product
- * (`batch` = 1, `segments` > 1; C, bias and the maxima are then entry 0's).  Every operand element is used as the sum
- * of two fp16 values scaled by a power of two per row of A and of B, three products per pair of elements are
- * accumulated in fp32, and the scales leave exactly; error against fp32 products: at or below theirs.  Infinities and
- * NaN reach the result as in fp32 arithmetic.  Results repeat bit for bit.
+ * fp32 products on the bf16 matrix cores: C_i(m, n) = sum over k of A_i(m, k) B_i(n, k) (+ bias_i(n)) for up to
+ * QSSM_GEMM_MANY products of one shape, or the sum of up to QSSM_GEMM_MANY runs of K k's as one product
+ * (`batch` = 1, `segments` > 1; C and bias are then entry 0's).  Every operand element is used as the sum of three bf16
+ * values, which hold all of its bits, six products per pair of elements are accumulated in fp32, and what is left out of
+ * a pair is below 2^-24 of it; sums over k are rounded sixteen times less often than in a chain of fp32 multiply-adds.
+ * Infinities, NaN and overflow reach the result as in fp32 arithmetic.  Results repeat bit for bit.
  *   a, lda   A_i(m, k) = a[m * lda + k], or a[k * lda + m] with `a_kstrided` (then b must be k-strided too)
  *   b, ldb   B_i(n, k) = b[n * ldb + k], or b[k * ldb + n] with `b_kstrided`
- *   amax_a   words of qssm_split_amax over the rows of A_i (over all runs of k), [parts_a][M]; amax_b of B_i, [parts_b][N]
  * N and the leading dimensions are multiples of 4, K too unless both operands are k-strided; a, b and c are 16-byte
- * aligned.  `partial` is fp32 scratch of splits * batch * M * N floats when splits > 1 (qssm_split_gemm_splits names
+ * aligned.  `partial` is fp32 scratch of splits * batch * M * N floats when splits > 1 (qssm_gemm_f32_splits names
  * the number of parts that suits the launch; 1 is always right).
  * These are the layer's projections (quick_ssm/layers.py:76-80,106) and what autograd records for them when the
  * parameters are fp32.
  */
-#define QSSM_SPLIT_MANY 5
+#define QSSM_GEMM_MANY 5
 typedef struct {
-  const float *a[QSSM_SPLIT_MANY], *b[QSSM_SPLIT_MANY];
-  float* c[QSSM_SPLIT_MANY];
-  const float* bias[QSSM_SPLIT_MANY];
-  const uint32_t *amax_a[QSSM_SPLIT_MANY], *amax_b[QSSM_SPLIT_MANY];
+  const float *a[QSSM_GEMM_MANY], *b[QSSM_GEMM_MANY];
+  float* c[QSSM_GEMM_MANY];
+  const float* bias[QSSM_GEMM_MANY];
   int64_t lda, ldb, ldc;
-  int32_t M, N, K, batch, segments, splits, a_kstrided, b_kstrided, parts_a, parts_b;
+  int32_t M, N, K, batch, segments, splits, a_kstrided, b_kstrided;
   float* partial;
   uint64_t partial_floats;
-} qssm_split_gemm_call;
-QSSM_API int qssm_split_gemm(const qssm_split_gemm_call* call, void* stream);
-QSSM_API int qssm_split_gemm_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments);
-
-/*
- * Bits of the largest absolute value in the rows and columns of `count` fp32 matrices (up to QSSM_SPLIT_MANY + 1; row
- * strides and cols multiples of 4, 16-byte aligned), for qssm_split_gemm.  A matrix is taken in blocks, and each writes
- * words of its own: row is [row_parts][rows] and col [col_parts][cols], or NULL, with the numbers of parts that
- * qssm_split_amax_parts gives for the matrix's shape (a row's largest is the largest of its parts).  Parts of several
- * matrices laid one behind the other make the maxima over all of them.
- */
-typedef struct {
-  const float* x;
-  uint32_t *row, *col;
-  int64_t rows, ld;
-  int32_t cols, reserved;
-} qssm_split_amax_matrix;
-QSSM_API int qssm_split_amax(const qssm_split_amax_matrix* matrices, int32_t count, void* stream);
-QSSM_API int qssm_split_amax_parts(int64_t rows, int32_t cols, int32_t* row_parts, int32_t* col_parts);
+} qssm_gemm_f32_call;
+QSSM_API int qssm_gemm_f32(const qssm_gemm_f32_call* call, void* stream);
+QSSM_API int qssm_gemm_f32_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments);
 
 /*
  * Streaming copy of `bytes` bytes (16-byte aligned, multiple of 16) on `stream`.  Not part of

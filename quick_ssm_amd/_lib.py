@@ -50,10 +50,8 @@ EXPORTED_SYMBOLS = (
     "qssm_rmsnorm_forward",
     "qssm_rmsnorm_backward",
     "qssm_colsum",
-    "qssm_split_gemm",
-    "qssm_split_gemm_splits",
-    "qssm_split_amax",
-    "qssm_split_amax_parts",
+    "qssm_gemm_f32",
+    "qssm_gemm_f32_splits",
     "qssm_copy_bytes",
     "qssm_launch_count_step",
 )
@@ -203,8 +201,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.qssm_rmsnorm_backward.argtypes = [vp, i64, vp, i64, vp, vp, vp, vp, vp, i32, i64, i32, ctypes.c_float, i32, vp]
     lib.qssm_colsum.restype = ctypes.c_int
     lib.qssm_colsum.argtypes = [vp, i64, i64, i32, i32, vp, i32, vp, vp]
-    lib.qssm_split_gemm_splits.restype = ctypes.c_int
-    lib.qssm_split_gemm_splits.argtypes = [i32] * 5
+    lib.qssm_gemm_f32_splits.restype = ctypes.c_int
+    lib.qssm_gemm_f32_splits.argtypes = [i32] * 5
     lib.qssm_copy_bytes.restype = ctypes.c_int
     lib.qssm_copy_bytes.argtypes = [vp, vp, u64, vp]
     lib.qssm_launch_count_step.restype = ctypes.c_int

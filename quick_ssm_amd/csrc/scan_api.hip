@@ -92,7 +92,6 @@ static const int kGatedLdsBytes = 80 * 1024;   // the gated backward: half of a 
 static const int kCUs = 256;
 static const uint64_t kKeepBytes = 224ull << 20;  // operand bytes a forward leaves in the caches for its backward
 
-static const double kSplitPartCost = 0.0125;       // stages of the split GEMM that one more MB of partial sums costs
 static const int kSplitStageK = 16;
 
 static const int kLooseColumns = 32;
@@ -988,29 +987,33 @@ int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int32_t dtyp
   return e == hipSuccess ? 0 : hip_fail(e, "colsum kernel launch");
 }
 
-int qssm_split_gemm_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments) {
+int qssm_gemm_f32_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments) {
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || segments <= 0) return 1;
-  // Two workgroups per compute unit run at once.  A launch takes whole rounds of them, each as long as its stages of
-  // 16 k's, and about 24 stages' worth to fill and drain a workgroup (a round of 16 stages takes 36 us where a stage takes
-  // 1.5); every further part writes and reads C once more, at kSplitPartCost stages per MB.
-  const double tiles = (double)split_gemm_tiles(M, N, batch), stages = (double)split_gemm_stages(K, segments);
-  const double out_mb = (double)M * N * batch * 4e-6;
+  // Two workgroups per compute unit run at once, so a launch takes whole rounds of 512 of them, and its last round is
+  // shorter per stage of 16 k's if there is but one for each unit.  Several parts write and read C once more each.  The us
+  // below fit 66 products of 2^30 to 2^36 multiply-adds in 1 to 32 parts to 6 %; the parts chosen by them are the fastest
+  // measured ones for 59 of the products and within 3 % for all.
+  const double kStage = 1.29, kLoneStage = 0.72, kRound = 12.4, kPartMb = 0.087, kParts = 4.7;
+  const double stages = (double)split_gemm_stages(K, segments), out_mb = (double)M * N * batch * 4e-6;
+  const int64_t tiles = split_gemm_tiles(M, N, batch), wave = 2 * kCUs;
   int best = 1;
   double best_cost = 0.0;
   for (int s = 1; s <= 32 && (s == 1 || stages / s >= 16.0); ++s) {
-    const double rounds = (double)(int64_t)((tiles * s + 2 * kCUs - 1) / (2 * kCUs));
-    const double cost = rounds * (stages / s + 24.0) + (s > 1 ? (s + 1) * out_mb * kSplitPartCost : 0.0);
+    const int64_t full = tiles * s / wave, rest = tiles * s % wave;
+    double cost = (double)full * (stages / s * kStage + kRound);
+    if (rest > 0) cost += stages / s * (rest <= kCUs ? kLoneStage : kStage) + kRound;
+    if (s > 1) cost += (2 * s + 1) * out_mb * kPartMb + kParts;
     if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
   }
   return best;
 }
 
-int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
+int qssm_gemm_f32(const qssm_gemm_f32_call* k, void* stream) {
   if (k == nullptr) return fail(QSSM_EINVAL, "call is NULL");
   if (k->M < 0 || k->N < 0 || k->K < 1) return fail(QSSM_EINVAL, "bad dimension");
-  if (k->batch < 1 || k->batch > QSSM_SPLIT_MANY || k->segments < 1 || k->segments > QSSM_SPLIT_MANY ||
+  if (k->batch < 1 || k->batch > QSSM_GEMM_MANY || k->segments < 1 || k->segments > QSSM_GEMM_MANY ||
       (k->batch > 1 && k->segments > 1))
-    return fail(QSSM_EINVAL, "1 to %d products, or runs of k of one product", QSSM_SPLIT_MANY);
+    return fail(QSSM_EINVAL, "1 to %d products, or runs of k of one product", QSSM_GEMM_MANY);
   // (the kernel counts rows and columns up to the end of the last tile in 32 bits)
   if (k->M > 0x7fffffff - kSplitTileM || k->N > 0x7fffffff - kSplitTileN)
     return fail(QSSM_EINVAL, "M and N must leave room for a tile below 2^31");
@@ -1036,19 +1039,15 @@ int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
     p.b[i] = k->b[i];
   }
   for (int i = 0; i < k->batch; ++i) {
-    if (k->c[i] == nullptr || k->amax_a[i] == nullptr || k->amax_b[i] == nullptr) return fail(QSSM_EINVAL, "NULL result or maxima");
+    if (k->c[i] == nullptr) return fail(QSSM_EINVAL, "NULL result");
     if (((uintptr_t)k->c[i]) % 16 != 0) return fail(QSSM_EALIGN, "results must be 16-byte aligned");
     p.c[i] = k->c[i];
     p.bias[i] = k->bias[i];
-    p.amax_a[i] = k->amax_a[i];
-    p.amax_b[i] = k->amax_b[i];
   }
   p.lda = k->lda; p.ldb = k->ldb; p.ldc = k->ldc;
   p.M = k->M; p.N = k->N; p.K = k->K;
   p.batch = k->batch; p.segments = k->segments; p.splits = k->splits;
   p.partial = k->partial;
-  p.parts_a = k->parts_a; p.parts_b = k->parts_b;
-  if (p.parts_a < 1 || p.parts_b < 1) return fail(QSSM_EINVAL, "the maxima have at least one part");
   if (split_gemm_tiles(p.M, p.N, p.batch) * p.splits > 0x7fffffffll || split_gemm_stages(p.K, p.segments) * kSplitStageK > 0x7fffffffll ||
       (int64_t)p.M * p.N / 4 * p.batch > 0x7fffffffll * 128)
     return fail(QSSM_EINVAL, "product too large for one launch");
@@ -1056,36 +1055,6 @@ int qssm_split_gemm(const qssm_split_gemm_call* k, void* stream) {
     return fail(QSSM_EINVAL, "operand layout is not built");
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : hip_fail(e, "split_gemm_kernel launch");
-}
-
-int qssm_split_amax_parts(int64_t rows, int32_t cols, int32_t* row_parts, int32_t* col_parts) {
-  if (row_parts == nullptr || col_parts == nullptr) return fail(QSSM_EINVAL, "NULL argument");
-  if (rows < 1 || cols < 1 || rows > 0x7fffffffll || cols > (1 << 26)) return fail(QSSM_EINVAL, "bad dimension");
-  AmaxMatrix m;
-  amax_shape(rows, cols, &m);
-  *row_parts = m.col_blocks;
-  *col_parts = m.row_blocks;
-  return 0;
-}
-
-int qssm_split_amax(const qssm_split_amax_matrix* matrices, int32_t count, void* stream) {
-  if (matrices == nullptr) return fail(QSSM_EINVAL, "matrices is NULL");
-  if (count < 1 || count > QSSM_SPLIT_MANY + 1) return fail(QSSM_EINVAL, "1 to %d matrices", QSSM_SPLIT_MANY + 1);
-  AmaxArgs p;
-  memset(&p, 0, sizeof(p));
-  for (int i = 0; i < count; ++i) {
-    const qssm_split_amax_matrix& g = matrices[i];
-    if (g.rows < 1 || g.cols < 1 || g.rows > 0x7fffffffll || g.cols > (1 << 26)) return fail(QSSM_EINVAL, "bad dimension");
-    if (g.cols % 4 != 0 || g.ld % 4 != 0 || g.ld < g.cols) return fail(QSSM_EALIGN, "cols and ld must be multiples of 4, ld >= cols");
-    if (g.x == nullptr || ((uintptr_t)g.x) % 16 != 0) return fail(QSSM_EALIGN, "matrices must be there and 16-byte aligned");
-    AmaxMatrix& m = p.m[i];
-    amax_shape(g.rows, g.cols, &m);
-    m.x = g.x; m.row = g.row; m.col = g.col;
-    m.rows = g.rows; m.ld = g.ld; m.cols = g.cols;
-  }
-  launch_amax(p, count, (hipStream_t)stream);
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? 0 : hip_fail(e, "amax_kernel launch");
 }
 
 int qssm_launch_count_step(uint32_t count, int32_t static_scratch, uint32_t* flag, uint32_t* next, int32_t* wipes) {

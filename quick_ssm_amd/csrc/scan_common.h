@@ -568,17 +568,14 @@ bool launch_norm_any(int dtype, const NormFwdArgs* f, const NormBwdArgs* b, int 
 bool launch_colsum_any(int dtype, const void* x, int64_t ld, int64_t rows, int S, int vec, float* partial, int chunks,
                        void* out, hipStream_t stream);
 
-// ---- fp32 products on the 16-bit matrix cores (gemm_split.hip) -----------------------------------------------------
+// ---- fp32 products on the bf16 matrix cores (gemm_split.hip) -----------------------------------------------------
 constexpr int kSplitGemmMany = 5;   // products (or runs of k) of one launch
-constexpr int kSplitTileM = 256, kSplitTileN = 128;   // rows and columns of a workgroup's tile
+constexpr int kSplitTileM = 128, kSplitTileN = 128;   // rows and columns of a workgroup's tile
 
 struct SplitGemmArgs {
   const float *a[kSplitGemmMany], *b[kSplitGemmMany];  // one pair per product, or per run of k
   float* c[kSplitGemmMany];                             // [M, N], row stride ldc
   const float* bias[kSplitGemmMany];                    // [N] or null
-  // bits of the rows' largest magnitudes, [parts_a][M] and [parts_b][N]: a row's is the largest of its parts
-  const unsigned *amax_a[kSplitGemmMany], *amax_b[kSplitGemmMany];
-  int parts_a, parts_b;
   int64_t lda, ldb, ldc;
   int M, N, K;
   int batch;       // products
@@ -587,22 +584,8 @@ struct SplitGemmArgs {
   float* partial;  // [splits][batch][M][N] when there are several
 };
 
-struct AmaxMatrix {
-  const float* x;          // [rows, cols], row stride ld
-  unsigned *row, *col;     // [col_blocks][rows], [row_blocks][cols], or null
-  int64_t rows, ld;
-  int cols;
-  int wide, col_blocks, row_blocks, block_rows, blocks;   // from amax_shape
-};
-
-struct AmaxArgs {
-  AmaxMatrix m[kSplitGemmMany + 1];
-};
-
 int64_t split_gemm_tiles(int64_t M, int64_t N, int64_t batch);
 int64_t split_gemm_stages(int64_t K, int64_t segments);
 bool launch_split_gemm(const SplitGemmArgs& args, bool a_kstrided, bool b_kstrided, hipStream_t stream);
-void amax_shape(int64_t rows, int cols, AmaxMatrix* m);
-void launch_amax(const AmaxArgs& args, int count, hipStream_t stream);
 
 }  // namespace qssm

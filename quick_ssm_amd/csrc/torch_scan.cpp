@@ -368,7 +368,7 @@ struct ScanBackward : public Node {
   }
 };
 
-// ---- linear maps over fp32 parameters (qssm_split_gemm) -----------------------------------------------------------
+// ---- linear maps over fp32 parameters (qssm_gemm_f32) -------------------------------------------------------------
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)t.get_device()).stream(); }
 
@@ -376,65 +376,34 @@ Tensor matrix(int64_t rows, int64_t cols, const Tensor& like) {
   return at::empty({rows, cols}, like.options().memory_format(c10::nullopt).requires_grad(c10::nullopt));
 }
 
-// Maxima of several matrices in one launch; each asks for its rows', its columns' or both.
-struct AmaxList {
-  qssm_split_amax_matrix m[QSSM_SPLIT_MANY + 1];
-  int n = 0;
-
-  // Words for the rows (columns) of `count` matrices of one shape, [count * parts, rows (cols)] int32.
-  static Tensor words(const Tensor& like, bool rows, int count) {
-    int32_t row_parts = 0, col_parts = 0;
-    check_rc(qssm_split_amax_parts(like.size(0), (int32_t)like.size(1), &row_parts, &col_parts));
-    return at::empty({(int64_t)count * (rows ? row_parts : col_parts), like.size(rows ? 0 : 1)},
-                     like.options().dtype(at::kInt).memory_format(c10::nullopt).requires_grad(c10::nullopt));
-  }
-  // `row`, `col`: where matrix i of `count` that share the words finds its parts (undefined: not wanted).
-  void add(const Tensor& t, const Tensor& row, const Tensor& col, int i, int count) {
-    auto at = [&](const Tensor& w) -> uint32_t* {
-      return w.defined() ? (uint32_t*)w.mutable_data_ptr<int32_t>() + w.numel() / count * i : nullptr;
-    };
-    m[n++] = {t.const_data_ptr<float>(), at(row), at(col), t.size(0), t.stride(0), (int32_t)t.size(1), 0};
-  }
-  void launch(const Tensor& like) { check_rc(qssm_split_amax(m, n, stream_of(like))); }
-};
-
-struct Product {
-  qssm_split_gemm_call k{};
+// c[i] = a[i] b[i]^T (+ bias[i]), or c[0] = the sum of them all.
+void product(const std::vector<Tensor>& a, const std::vector<Tensor>& b, const std::vector<Tensor>& c, int64_t K,
+             bool a_kstrided, bool b_kstrided, const std::vector<Tensor>& bias = {}) {
+  qssm_gemm_f32_call k{};
   Tensor partial;
-
-  // c[i] = a[i] b[i]^T (+ bias[i]), or c[0] = the sum of them all.  The words of several products' rows lie one behind
-  // the other in `amax_a` and `amax_b`, or all use the same (`each_*` false).
-  Product(const std::vector<Tensor>& a, const std::vector<Tensor>& b, const std::vector<Tensor>& c, const Tensor& amax_a,
-          bool each_a, const Tensor& amax_b, bool each_b, int64_t K, bool a_kstrided, bool b_kstrided,
-          const std::vector<Tensor>& bias = {}) {
-    const int batch = (int)c.size();
-    for (size_t i = 0; i < a.size(); ++i) {
-      k.a[i] = a[i].const_data_ptr<float>();
-      k.b[i] = b[i].const_data_ptr<float>();
-    }
-    for (int i = 0; i < batch; ++i) {
-      k.c[i] = c[i].mutable_data_ptr<float>();
-      k.amax_a[i] = (const uint32_t*)amax_a.const_data_ptr<int32_t>() + (each_a ? amax_a.numel() / batch * i : 0);
-      k.amax_b[i] = (const uint32_t*)amax_b.const_data_ptr<int32_t>() + (each_b ? amax_b.numel() / batch * i : 0);
-      if ((size_t)i < bias.size()) k.bias[i] = floats_or_null(bias[i]);
-    }
-    k.lda = a[0].stride(0); k.ldb = b[0].stride(0); k.ldc = c[0].stride(0);
-    k.M = (int32_t)c[0].size(0); k.N = (int32_t)c[0].size(1); k.K = (int32_t)K;
-    k.batch = batch;
-    k.segments = batch == 1 ? (int32_t)a.size() : 1;
-    k.a_kstrided = a_kstrided;
-    k.b_kstrided = b_kstrided;
-    k.parts_a = (int32_t)(amax_a.size(0) / (each_a ? batch : 1));
-    k.parts_b = (int32_t)(amax_b.size(0) / (each_b ? batch : 1));
-    k.splits = qssm_split_gemm_splits(k.M, k.N, k.K, batch, k.segments);
-    if (k.splits > 1) {
-      partial = matrix((int64_t)k.splits * batch * k.M, k.N, c[0]);
-      k.partial = partial.mutable_data_ptr<float>();
-      k.partial_floats = (uint64_t)partial.numel();
-    }
-    check_rc(qssm_split_gemm(&k, stream_of(c[0])));
+  const int batch = (int)c.size();
+  for (size_t i = 0; i < a.size(); ++i) {
+    k.a[i] = a[i].const_data_ptr<float>();
+    k.b[i] = b[i].const_data_ptr<float>();
   }
-};
+  for (int i = 0; i < batch; ++i) {
+    k.c[i] = c[i].mutable_data_ptr<float>();
+    if ((size_t)i < bias.size()) k.bias[i] = floats_or_null(bias[i]);
+  }
+  k.lda = a[0].stride(0); k.ldb = b[0].stride(0); k.ldc = c[0].stride(0);
+  k.M = (int32_t)c[0].size(0); k.N = (int32_t)c[0].size(1); k.K = (int32_t)K;
+  k.batch = batch;
+  k.segments = batch == 1 ? (int32_t)a.size() : 1;
+  k.a_kstrided = a_kstrided;
+  k.b_kstrided = b_kstrided;
+  k.splits = qssm_gemm_f32_splits(k.M, k.N, k.K, batch, k.segments);
+  if (k.splits > 1) {
+    partial = matrix((int64_t)k.splits * batch * k.M, k.N, c[0]);
+    k.partial = partial.mutable_data_ptr<float>();
+    k.partial_floats = (uint64_t)partial.numel();
+  }
+  check_rc(qssm_gemm_f32(&k, stream_of(c[0])));
+}
 
 bool matrix_ok(const Tensor& t, int64_t rows, int64_t cols, const Tensor& like) {
   return t.defined() && t.is_cuda() && t.device() == like.device() && t.scalar_type() == at::kFloat && t.dim() == 2 &&
@@ -443,7 +412,7 @@ bool matrix_ok(const Tensor& t, int64_t rows, int64_t cols, const Tensor& like) 
 }
 
 void check_operands(const Tensor& u, const std::vector<Tensor>& w) {
-  TORCH_CHECK_VALUE(!w.empty() && w.size() <= QSSM_SPLIT_MANY && u.defined() && u.dim() == 2 && u.size(0) > 0 &&
+  TORCH_CHECK_VALUE(!w.empty() && w.size() <= QSSM_GEMM_MANY && u.defined() && u.dim() == 2 && u.size(0) > 0 &&
                         matrix_ok(u, u.size(0), u.size(1), u), "split products need a float32 GPU matrix of 16-byte aligned rows");
   for (const Tensor& t : w)
     TORCH_CHECK_VALUE(matrix_ok(t, w[0].size(0), u.size(1), u) && t.stride(0) == w[0].stride(0),
@@ -563,16 +532,14 @@ PyObject* wrap_list(const std::vector<Tensor>& v) {
   return r;
 }
 
-// (u, weights, biases, want: 1 the input's column maxima | 2 the weights') -> (outputs, column maxima of u, of the weights)
+// (u, weights, biases) -> outputs
 PyObject* py_split_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  want_args(n, 4);
+  want_args(n, 3);
   const Tensor& u = tensor_arg(args[0]);
   const std::vector<Tensor> w = tensors_arg(args[1]);
   std::vector<Tensor> bias = tensors_arg(args[2]), out;
-  const int64_t want = int_arg(args[3]);
   check_operands(u, w);
-  Tensor u_col, w_col;
   {
     const c10::AutoGradMode no_grad(false);
     const c10::OptionalDeviceGuard guard(u.device());
@@ -585,34 +552,21 @@ PyObject* py_split_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                           "a bias must be a float32 vector of the outputs' width");
         t = t.contiguous();
       }
-    AmaxList list;
-    const Tensor u_row = AmaxList::words(u, true, 1), w_row = AmaxList::words(w[0], true, count);
-    if (want & 1) u_col = AmaxList::words(u, false, 1);
-    if (want & 2) w_col = AmaxList::words(w[0], false, count);
-    list.add(u, u_row, u_col, 0, 1);
-    for (int i = 0; i < count; ++i) list.add(w[i], w_row, w_col, i, count);
-    list.launch(u);
     for (int i = 0; i < count; ++i) out.push_back(matrix(u.size(0), N, u));
-    Product(std::vector<Tensor>(count, u), w, out, u_row, false, w_row, true, u.size(1), false, false, bias);
+    product(std::vector<Tensor>(count, u), w, out, u.size(1), false, false, bias);
   }
-  PyObject* r = PyTuple_New(3);
-  if (r == nullptr) throw python_error();
-  PyTuple_SET_ITEM(r, 0, wrap_list(out));
-  PyTuple_SET_ITEM(r, 1, wrap_or_none(u_col));
-  PyTuple_SET_ITEM(r, 2, wrap_or_none(w_col));
-  return r;
+  return wrap_list(out);
   END_HANDLE_TH_ERRORS
 }
 
-// (gradients of the outputs, u, weights, column maxima of u, of the weights, want: 1 du | 2 dw) -> (du, [dw])
+// (gradients of the outputs, u, weights, want: 1 du | 2 dw) -> (du, [dw])
 PyObject* py_split_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  want_args(n, 6);
+  want_args(n, 4);
   std::vector<Tensor> g = tensors_arg(args[0]), dw;
   const Tensor& u = tensor_arg(args[1]);
   const std::vector<Tensor> w = tensors_arg(args[2]);
-  const Tensor &u_col = tensor_arg(args[3]), &w_col = tensor_arg(args[4]);
-  const int64_t want = int_arg(args[5]);
+  const int64_t want = int_arg(args[3]);
   check_operands(u, w);
   Tensor du;
   {
@@ -628,21 +582,13 @@ PyObject* py_split_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     if (!whole)
       for (Tensor& t : g) t = matrix(rows, N, u).copy_(t);
-    const bool need_du = want & 1, need_dw = want & 2;
-    TORCH_CHECK_VALUE((!need_du || w_col.defined()) && (!need_dw || u_col.defined()), "the forward saved no maxima for this gradient");
-    Tensor g_row, g_col;
-    if (need_du) g_row = AmaxList::words(g[0], true, count);
-    if (need_dw) g_col = AmaxList::words(g[0], false, count);
-    AmaxList list;
-    for (int i = 0; i < count; ++i) list.add(g[i], g_row, g_col, i, count);
-    if (need_du || need_dw) list.launch(u);
-    if (need_du) {
+    if (want & 1) {
       du = matrix(rows, K, u);
-      Product(g, w, {du}, g_row, false, w_col, false, N, false, true);
+      product(g, w, {du}, N, false, true);
     }
-    if (need_dw) {
+    if (want & 2) {
       for (int i = 0; i < count; ++i) dw.push_back(matrix(N, K, u));
-      Product(g, std::vector<Tensor>(count, u), dw, g_col, true, u_col, false, rows, true, true);
+      product(g, std::vector<Tensor>(count, u), dw, rows, true, true);
     }
   }
   PyObject* r = PyTuple_New(2);

@@ -2,7 +2,7 @@
 
 Same constructor arguments, parameter names (so state dicts interchange) and forward keywords as
 the reference's quick_ssm/layers.py:9-107.  The projections are torch GEMMs, except over fp32
-parameters, where they are split products on the 16-bit matrix cores (quick_ssm_amd/split_linear.py); the gate
+parameters, where they are split products on the bf16 matrix cores (quick_ssm_amd/split_linear.py); the gate
 activations and casts between them and the scan happen inside the scan's own launches when the
 projections are stored as the 16-bit compute dtype (quick_ssm_amd/gated_scan.py) and are one fused HIP
 pass otherwise (quick_ssm_amd/gates.py),
@@ -60,10 +60,10 @@ def column_sum(g2: torch.Tensor) -> torch.Tensor:
 
 
 def _products(ctx, u: torch.Tensor, weights, biases):
-    """u w^T + bias for every weight as split products, inside an autograd function's forward; the maxima the backward
-    wants are saved in `ctx.maxima`."""
+    """u w^T + bias for every weight as split products, inside an autograd function's forward."""
     u2 = u.reshape(-1, u.shape[-1])
-    outs, ctx.maxima = split_linear.forward(u2, weights, biases, ctx.needs_input_grad[0], any(ctx.needs_input_grad[1:]))
+    ctx.split = True
+    outs, _ = split_linear.forward(u2, weights, biases, ctx.needs_input_grad[0], any(ctx.needs_input_grad[1:]))
     return [t.view(*u.shape[:-1], t.shape[-1]) for t in outs]
 
 
@@ -71,9 +71,9 @@ def _product(ctx, u: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor) -> 
     """One of them, as a split product where that applies, else torch's.  (Small layers are bound by the interpreter: a
     16-bit one gets no further than its type.)"""
     if (u.dtype is torch.float32 and u.numel() * weight.shape[0] >= split_linear.MIN_WORK
-            and split_linear.usable(u, (weight,))):
+            and split_linear.usable(u, (weight,), any(ctx.needs_input_grad))):
         return _products(ctx, u, (weight,), (bias,))[0]
-    ctx.maxima = None
+    ctx.split = False
     return torch.nn.functional.linear(u, weight, bias)
 
 
@@ -81,8 +81,8 @@ def _product_gradients(ctx, grads, u: torch.Tensor, weights, need_du: bool, need
     """Gradients of the input and of the weights from the outputs' gradients ([rows, N] each).  A backward that is
     itself recorded (create_graph) takes torch's products, which autograd can follow."""
     u2 = u.reshape(-1, u.shape[-1])
-    if ctx.maxima is not None and not torch.is_grad_enabled():
-        du, dws = split_linear.backward(grads, u2, weights, ctx.maxima, need_du, need_dw)
+    if ctx.split and not torch.is_grad_enabled():
+        du, dws = split_linear.backward(grads, u2, weights, None, need_du, need_dw)
         return (None if du is None else du.view_as(u)), dws
     du = None
     if need_du:
@@ -106,7 +106,7 @@ class _LinearBias(torch.autograd.Function):
         u, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
         g2 = g.reshape(-1, g.shape[-1])
-        if ctx.maxima is not None:
+        if ctx.split:
             du, (dw,) = _product_gradients(ctx, [g2], u, [weight], need[0], need[1])
         else:
             du = (g2 @ weight).view_as(u) if need[0] else None
@@ -133,7 +133,7 @@ class _PackedProjection(torch.autograd.Function):
         S = wide_w.shape[0] // 5
         g2 = g.reshape(-1, g.shape[-1])
         blocks = [None] * 5
-        if ctx.maxima is not None:
+        if ctx.split:
             du, (dw,) = _product_gradients(ctx, [g2], u, [wide_w], need[0], any(need[1:6]))
         else:
             du = (g2 @ wide_w).view_as(u) if need[0] else None
@@ -185,9 +185,8 @@ class _WideProjections(torch.autograd.Function):
 
 
 class _SplitProjections(torch.autograd.Function):
-    """The five projections of a layer with fp32 parameters as one launch: the outputs share the input's maxima, the
-    input's gradient is one product over 5 S k's instead of five products and four additions, and the five weight
-    gradients are one launch."""
+    """The five projections of a layer with fp32 parameters as one launch: the input's gradient is one product over 5 S
+    k's instead of five products and four additions, and the five weight gradients are one launch."""
 
     @staticmethod
     def forward(ctx, u, w_a, w_b, w_ca, w_cb, w_d, bias_a):
@@ -306,7 +305,7 @@ class SSM(nn.Module):
         mods, plain = self._projections()
         if plain and u.is_cuda:
             weights, bias = [m.weight for m in mods], self.A_proj.bias
-            if split_linear.usable(u, weights):
+            if split_linear.usable(u, weights, torch.is_grad_enabled()):
                 return None, _SplitProjections.apply(u, *weights, bias)
             if (u.dtype in (torch.float16, torch.bfloat16) and all(t.dtype == u.dtype for t in (*weights, bias))
                     and 0 < u.numel() // self.hidden_size * self.state_size_dim <= self._WIDE_PRODUCT_LIMIT

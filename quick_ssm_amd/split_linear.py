@@ -1,14 +1,15 @@
-"""Linear maps of the SSM layer over fp32 parameters, on the 16-bit matrix cores (csrc/gemm_split.hip).
+"""Linear maps of the SSM layer over fp32 parameters, on the bf16 matrix cores (csrc/gemm_split.hip).
 
 A layer with fp32 parameters spends nine tenths of its time in its projections (quick_ssm/layers.py:76-80,106): the
-library's fp32 products run at the fp32 MFMA rate, a sixteenth of the fp16 one.  `qssm_split_gemm` takes every element
-as the sum of two scaled fp16 values and accumulates three products in fp32, with an error at or below that of fp32
-products.  Here is the rule for when it is used; maxima, scratch and the calls are in csrc/torch_scan.cpp, the autograd
-functions that use them in quick_ssm_amd/layers.py.
+library's fp32 products run at the fp32 MFMA rate, a sixteenth of the bf16 one.  `qssm_gemm_f32` takes every element as
+the sum of three bf16 values, which hold all of its bits, and accumulates six products in fp32; measured against float64
+it is two to nine times closer than fp32 products (one nonzero product in a sum: 2 % further, 2.6e-8).  Here is the rule
+for when it is used; scratch and the calls are in csrc/torch_scan.cpp, the autograd functions that use them in
+quick_ssm_amd/layers.py.
 """
 from __future__ import annotations
 
-from typing import List, NamedTuple, Optional, Sequence, Tuple
+from typing import List, Optional, Sequence, Tuple
 
 import torch
 
@@ -16,23 +17,19 @@ from . import hip_scan
 
 Tensor = torch.Tensor
 
-# Multiply-adds (over all weights of a launch) below which the library's product stays, because the fixed costs of the
-# maxima, the prologue, the sums over parts and their launches exceed the gain.  us for output, input gradient and weight
-# gradient together, library against these: 4096 rows, 1024 x 256 (1.1e9) 79 against 129; 4096 rows, 256 x 5120 (5.4e9)
-# 335 against 250 on the GPU, but twice the launches, and a layer of that size is bound by its host (617 us a step against
-# 660); 2048 rows, 512 x 10240 (1.1e10) a layer step of 705 against 625; 8192 rows, 512 x 5 * 1024 (2.1e10) 1042 against 588.
-MIN_WORK = 1 << 33
+# Multiply-adds (over all weights of a launch) below which the library's product stays, because filling and draining the
+# launch and the sums over parts exceed the gain.  GPU us for output, input gradient and weight gradient, library against
+# these: 2^31 (2048 rows, 2048 -> 512) 34, 36, 35 against 44, 39, 45; 2^31.3 (2048 rows, 256 -> 5120) 56, 47, 66 against 56,
+# 53, 54; 2^32 (8192 rows, 2048 -> 256) 69, 74, 71 against 69, 70, 69; 2^32.3 (4096 rows, 256 -> 5120) 101, 94, 127 against
+# 95, 82, 85; 2^33.3 (4096 rows, 512 -> 5120) 167, 158, 187 against 144, 139, 144.
+MIN_WORK = 1 << 32
 
-# Most rows and outputs: the kernel counts to the end of its last tile of 256 in 32 bits.
-MAX_ROWS = (1 << 31) - 1 - 256
+# An input narrower than this has few stages to fill a tile's pipeline with before its results are stored: 16384 rows,
+# 128 -> 2560, 105 us against 118, where the gradients gain (83 and 139 against 83 and 85); at 256 columns 174 against 171.
+MIN_INFERENCE_WIDTH = 256
 
-
-class Maxima(NamedTuple):
-    """What the backward needs of the operands: bits of the largest magnitude of every column of the input, and of
-    every column over all weights, in parts (None where no gradient asks for them)."""
-
-    u_col: Optional[Tensor]
-    w_col: Optional[Tensor]
+# Most rows and outputs: the kernel counts to the end of its last tile of 128 in 32 bits.
+MAX_ROWS = (1 << 31) - 1 - 128
 
 
 def _matrix_ok(t: Tensor) -> bool:
@@ -40,14 +37,15 @@ def _matrix_ok(t: Tensor) -> bool:
             and t.stride(0) % 4 == 0 and t.stride(0) < 1 << 20 and t.data_ptr() % 16 == 0)
 
 
-def usable(u: Tensor, weights: Sequence[Tensor]) -> bool:
-    """Whether u [.., K] times the transposes of the weights [N, K] may take the split products."""
+def usable(u: Tensor, weights: Sequence[Tensor], gradients: bool = True) -> bool:
+    """Whether u [.., K] times the transposes of the weights [N, K] may take the split products; `gradients`: theirs will
+    be asked for."""
     n, k = weights[0].shape
     if u.dtype is not torch.float32 or u.numel() * n * len(weights) < MIN_WORK:
         return False
     if not u.is_cuda or torch.is_autocast_enabled("cuda") or n % 4 or k % 4:
         return False
-    if u.numel() // k > MAX_ROWS or n > MAX_ROWS:
+    if u.numel() // k > MAX_ROWS or n > MAX_ROWS or (k < MIN_INFERENCE_WIDTH and not gradients):
         return False
     if not _matrix_ok(u.reshape(-1, k)):
         return False
@@ -55,20 +53,20 @@ def usable(u: Tensor, weights: Sequence[Tensor]) -> bool:
                for w in weights)
 
 
-def forward(u: Tensor, weights: Sequence[Tensor], biases: Sequence[Optional[Tensor]], need_du: bool, need_dw: bool
-            ) -> Tuple[List[Tensor], Maxima]:
-    """u w^T + bias for every weight (call `usable` first), and the maxima a backward wants."""
+def forward(u: Tensor, weights: Sequence[Tensor], biases: Sequence[Optional[Tensor]], need_du: bool = True,
+            need_dw: bool = True) -> Tuple[List[Tensor], None]:
+    """u w^T + bias for every weight (call `usable` first), and what a backward that asks for `need_du` and `need_dw`
+    wants kept besides the operands: nothing, they are split where they are used."""
     native = hip_scan._native or hip_scan._load_native()
-    outs, u_col, w_col = native.split_forward(u, weights, biases, need_dw | need_du << 1)
-    return outs, Maxima(u_col, w_col)
+    return native.split_forward(u, weights, biases), None
 
 
-def backward(grads: Sequence[Tensor], u: Tensor, weights: Sequence[Tensor], saved: Maxima, need_du: bool, need_dw: bool
+def backward(grads: Sequence[Tensor], u: Tensor, weights: Sequence[Tensor], saved: None, need_du: bool, need_dw: bool
              ) -> Tuple[Optional[Tensor], List[Optional[Tensor]]]:
     """Gradients of the input (summed over the weights) and of every weight from the outputs' gradients [rows, N]."""
     native = hip_scan._native or hip_scan._load_native()
-    du, dws = native.split_backward(grads, u, weights, saved.u_col, saved.w_col, need_du | need_dw << 1)
+    du, dws = native.split_backward(grads, u, weights, need_du | need_dw << 1)
     return du, (dws if need_dw else [None] * len(weights))
 
 
-__all__ = ["usable", "forward", "backward", "Maxima"]
+__all__ = ["usable", "forward", "backward"]
