@@ -154,10 +154,12 @@ class _WideProjections(torch.autograd.Function):
 
     What it is for is the backward: one product over 5 S k's for the input's gradient instead of five and four additions,
     and one for all weights, whose five [S, H] products alone leave most of the GPU idle (K is the number of rows).  Unlike
-    `_PackedProjection` the parameters keep their own memory; concatenating them (42 MB at hidden 1024, state 4096) costs
-    a launch of about 20 us.  Layer step, five products -> one, bf16: B=8 L=2048 hidden 512 state 2048 1518 -> 1160 us,
-    B=16 L=1024 hidden 512 state 1024 1171 -> 772, B=2 hidden 1024 state 4096 955 -> 908, B=8 3013 -> 3000; at twice that
-    (B=16, 5718 against 5769) the five products are efficient by themselves (`SSM._WIDE_PRODUCT_LIMIT`)."""
+    `_PackedProjection` the parameters keep their own memory.  They are concatenated by either pass and the copy is not
+    kept between the two (it would hold all projection weights of every layer a second time until the backward: 42 MB at
+    hidden 1024, state 4096); each copy of that size takes 32 us.  Layer step, five products -> one, bf16, at 2^24 and 2^26
+    elements per output: hidden 1024 state 4096 1002 -> 993 and 3164 -> 3049 us, 512 and 2048 928 -> 705 and 2896 -> 2086, 512
+    and 1024 1222 -> 809 and 3411 -> 2414, 256 and 1024 1043 -> 664 and 2824 -> 2034, 2048 and 2048 1578 -> 1409 and 5394 ->
+    5386, where the five are efficient by themselves (`SSM._WIDE_PRODUCT_LIMIT`)."""
 
     @staticmethod
     def forward(ctx, u, w_a, w_b, w_ca, w_cb, w_d, bias_a):
@@ -165,18 +167,16 @@ class _WideProjections(torch.autograd.Function):
         S = w_a.shape[0]
         wide_w = torch.cat(weights)                                                   # [5 S, H]
         wide_b = torch.cat((bias_a, bias_a.new_zeros(4 * S)))
-        ctx.save_for_backward(u, wide_w, *weights)
+        ctx.save_for_backward(u, *weights)
         return torch.nn.functional.linear(u, wide_w, wide_b)
 
     @staticmethod
     def backward(ctx, g):
-        u, wide_w, *weights = ctx.saved_tensors
+        u, *weights = ctx.saved_tensors
         need = ctx.needs_input_grad
-        S = wide_w.shape[0] // 5
+        S = weights[0].shape[0]
         g2 = g.reshape(-1, 5 * S)
-        du = None
-        if need[0]:   # a recorded backward has to see the parameters themselves
-            du = (g2 @ (torch.cat(weights) if torch.is_grad_enabled() else wide_w)).view_as(u)
+        du = (g2 @ torch.cat(weights)).view_as(u) if need[0] else None
         blocks = [None] * 5
         if any(need[1:6]):
             dw = g2.t() @ u.reshape(-1, u.shape[-1])                                  # [5 S, H]

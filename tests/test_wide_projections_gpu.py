@@ -54,3 +54,21 @@ def test_a_weight_changed_before_the_backward_is_an_error_and_second_derivatives
     (dx,) = torch.autograd.grad(layer(x).float().sum(), x, create_graph=True)
     grads = torch.autograd.grad(dx.float().pow(2).sum(), [layer.A_proj.weight, layer.D_proj.weight])
     assert all(bool(g.any()) for g in grads)
+
+
+def test_nothing_is_kept_for_the_backward_that_five_products_would_not_keep(gpu, monkeypatch):
+    monkeypatch.setattr(SSM, "_BATCHED_PROJECTION_LIMIT", 0)
+    layer = SSM(512, 4, dtype=torch.bfloat16, device=gpu, compute_dtype=torch.bfloat16)
+    x = torch.randn(1, 128, 512, device=gpu, dtype=torch.bfloat16, requires_grad=True)
+    kept = {}
+    for name in ("five", "one"):
+        monkeypatch.setattr(SSM, "_WIDE_PRODUCT_LIMIT", 0 if name == "five" else 1 << 26)
+        layer(x).sum().backward()                       # buffers of the launches exist from here on
+        layer.zero_grad()
+        x.grad = None
+        before = torch.cuda.memory_allocated(gpu)
+        y = layer(x)
+        kept[name] = torch.cuda.memory_allocated(gpu) - before
+        del y
+    # (the five weights are 10 MB, what the graph keeps of the activations 3; tensors are rounded up to 512 bytes)
+    assert kept["one"] <= kept["five"] + (1 << 17)
