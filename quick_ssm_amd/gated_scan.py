@@ -58,14 +58,18 @@ def supported(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype: torc
 
 
 def _plan(B: int, L: int, S: int, dtype: torch.dtype, compute_dtype: torch.dtype, out_dtype: torch.dtype,
-          direction: int, ckpt_stride: int, long: bool = False) -> Plan:
-    key = (B, L, S, dtype, compute_dtype, out_dtype, direction, ckpt_stride, long)
+          direction: int, ckpt_stride: int, long: bool = False, keep=True) -> Plan:
+    """`keep`: True for the planner's cache policy, else the most tiles per chain that may leave their operands in the
+    caches (False: none)."""
+    key = (B, L, S, dtype, compute_dtype, out_dtype, direction, ckpt_stride, long, keep, keep is True)
     plan = _plans.get(key)
     if plan is None:
         plan = Plan()
         planner = _lib.load().qssm_plan_scan_gated_long if long else _lib.load().qssm_plan_scan_gated
         _lib.check(planner(B, L, S, _CODES[dtype], _CODES[compute_dtype], _CODES[out_dtype], direction, 8, ckpt_stride,
                            ctypes.byref(plan)))
+        if keep is not True:
+            plan.keep_tiles = min(plan.keep_tiles, int(keep))
         if len(_plans) >= 1024:
             _plans.clear()
         _plans[key] = plan
@@ -77,10 +81,8 @@ def _st(t: Tensor) -> Strides:
 
 
 def _launch(plan: Plan, dev: torch.device, fn, *args) -> None:
-    with torch.cuda.device(dev):
-        stream = hip_scan._raw_stream(dev.index)
-        taken, epoch, capturing = hip_scan._launch_buffers(dev, dev.index, stream, int(plan.control_bytes),
-                                                           int(plan.workspace_bytes))
+    with _lib.launch_stream(dev) as stream:
+        taken, epoch, capturing = hip_scan._launch_buffers(dev, dev.index, stream, plan.control_bytes, plan.workspace_bytes)
         _lib.check(fn(ctypes.byref(plan), *args, *taken[3:], epoch, stream))
         hip_scan._after_launch(taken, stream, capturing)
 
@@ -93,11 +95,8 @@ def _forward_launch(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype
     dev, dtype = A_pre.device, A_pre.dtype
     # the backward's tile length decides how far apart the saved states are; it takes dy stored as the projections are
     stride = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, 0).seg_len
-    plan = _plan(B, L, S, dtype, compute_dtype, out_dtype, _lib.QSSM_FORWARD, stride, True)
-    keep = hip_scan._forward_keep if train else False
-    if keep is not True:
-        plan = Plan.from_buffer_copy(plan)   # cached plans are shared: change a copy
-        plan.keep_tiles = 0 if keep is False else min(int(plan.keep_tiles), int(keep))
+    plan = _plan(B, L, S, dtype, compute_dtype, out_dtype, _lib.QSSM_FORWARD, stride, True,
+                 hip_scan._forward_keep if train else False)
     y = torch.empty((B, L, S), dtype=out_dtype, device=dev)
     ckpt = torch.empty((B, plan.n_ckpt, S), dtype=torch.float32, device=dev)
     _launch(plan, dev, _lib.load().qssm_scan_gated_forward,

@@ -292,24 +292,27 @@ class SSM(nn.Module):
         return _PackedProjection.apply(u, self.A_proj.weight, self.B_proj.weight, self.C_proj_a.weight,
                                        self.C_proj_b.weight, self.D_proj.weight, self.A_proj.bias, wide_w, wide_b)
 
-    def _projections(self):
-        """The five projections in A, B, C_a, C_b, D order, and whether their calls are nothing but products."""
+    def _projections(self, look: bool):
+        """The five projections in A, B, C_a, C_b, D order, and, if asked to look, whether their calls are nothing but
+        products."""
         mods = (self.A_proj, self.B_proj, self.C_proj_a, self.C_proj_b, self.D_proj)
-        plain = (all(_plain_linear(m) for m in mods) and not nn.modules.module._has_any_global_hook()
+        plain = (look and all(_plain_linear(m) for m in mods) and not nn.modules.module._has_any_global_hook()
                  and self.A_proj.bias is not None and all(m.bias is None for m in mods[1:]))
         return mods, plain
 
     def _large_projections(self, u: torch.Tensor):
         """The projection outputs of a layer above `_BATCHED_PROJECTION_LIMIT`: one [.., 5 S] tensor for a 16-bit layer in
         training, or None and the five tensors (blocks in A, B, C_a, C_b, D order)."""
-        mods, plain = self._projections()
+        half = u.dtype in (torch.float16, torch.bfloat16)
+        grad = torch.is_grad_enabled()
+        mods, plain = self._projections(grad or not half)
         if plain and u.is_cuda:
             weights, bias = [m.weight for m in mods], self.A_proj.bias
-            if split_linear.usable(u, weights, torch.is_grad_enabled()):
+            if split_linear.usable(u, weights, grad):
                 return None, _SplitProjections.apply(u, *weights, bias)
-            if (u.dtype in (torch.float16, torch.bfloat16) and all(t.dtype == u.dtype for t in (*weights, bias))
+            if (half and grad and all(t.dtype == u.dtype for t in (*weights, bias))
                     and 0 < u.numel() // self.hidden_size * self.state_size_dim <= self._WIDE_PRODUCT_LIMIT
-                    and torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
+                    and not torch.is_autocast_enabled("cuda")
                     and (u.requires_grad or any(t.requires_grad for t in (*weights, bias)))):
                 return _WideProjections.apply(u, *weights, bias), None
         return None, tuple(m(u) for m in mods)
