@@ -346,7 +346,7 @@ struct ScanBackward : public Node {
     const Tensor ox = x.unpack(), oa = a.unpack(), ob = b.unpack(), oc = c.unpack();
     variable_list out(carry ? 5 : 4);
     const bool have_state = carry && grads[1].defined();
-    if (!grads[0].defined() && !have_state) return out;
+    // (no gradient at all, from a function that returns none for y, stands for zeros, as torch.autograd.Function has it)
     c10::AutoGradMode no_grad(false);
     const at::ScalarType in = scalar_of(k_in), go = scalar_of(k_out);
     const Tensor dy = grads[0].defined() ? in_dtype(grads[0], go) : at::zeros(ox.sizes(), ox.options().dtype(go));

@@ -57,6 +57,25 @@ def test_either_output_of_a_piece_may_go_unused(gpu, used, dtypes):
     assert hip_scan.workspace_status() == 0
 
 
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, t):
+        return t * 2
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+def test_no_gradient_from_a_function_behind_the_scan_is_a_gradient_of_zeros(gpu):
+    x, a, b, c, _ = make_inputs((2, 70, 24), seed=6)
+    leaves = [t.to(gpu).requires_grad_(True) for t in (x, a, b, c, torch.ones(2, 24))]
+    y, h = scan_chunk(*leaves)
+    (_NoGradient.apply(scan(*leaves[:4])).sum() + _NoGradient.apply(y).sum() + _NoGradient.apply(h).sum()).backward()
+    for t in leaves:
+        assert t.grad is not None and not bool(t.grad.any())
+
+
 def test_a_trace_records_the_scan_instead_of_its_result(gpu):
     first, second = ([t.to(gpu) for t in make_inputs((2, 130, 24), seed=s)[:4]] for s in (1, 2))
     state = torch.randn(2, 24, generator=torch.Generator().manual_seed(3)).to(gpu)
