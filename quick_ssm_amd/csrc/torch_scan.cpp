@@ -488,7 +488,8 @@ PyObject* py_scan_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // (y, h, ckpt, stride, x, a, b, c, k_in, k_out, final, state, h_init): makes y (and the final state, when there is
-// one) outputs of a ScanBackward node over the operands (and the incoming state, or None).
+// one) outputs of a ScanBackward node over the operands (and the incoming state, or None).  A y of a type that has no
+// gradients (integers, bool) stays outside.
 PyObject* py_attach_scan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   want_args(n, 13);
@@ -496,6 +497,8 @@ PyObject* py_attach_scan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor &x = tensor_arg(args[4]), &a = tensor_arg(args[5]), &b = tensor_arg(args[6]), &c = tensor_arg(args[7]);
   const Tensor& state = tensor_arg(args[11]);
   TORCH_CHECK_TYPE(y.defined() && x.defined() && a.defined() && b.defined() && c.defined(), "y, x, a, b, c must be tensors");
+  const bool y_has_gradients = torch::autograd::isDifferentiableType(y.scalar_type());
+  if (!y_has_gradients && !final_state.defined()) Py_RETURN_NONE;
   std::shared_ptr<ScanBackward> node(new ScanBackward(), torch::autograd::deleteNode);
   node->carry = final_state.defined();
   node->x = SavedVariable(x, false);
@@ -511,7 +514,8 @@ PyObject* py_attach_scan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (state.defined()) node->state_dtype = state.scalar_type();
   if (node->carry) node->set_next_edges(torch::autograd::collect_next_edges(x, a, b, c, state));
   else node->set_next_edges(torch::autograd::collect_next_edges(x, a, b, c));
-  torch::autograd::set_history(y, node);
+  if (y_has_gradients) torch::autograd::set_history(y, node);
+  else node->add_input_metadata(Node::undefined_input());
   if (node->carry) torch::autograd::set_history(final_state, node);
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS

@@ -76,6 +76,22 @@ def test_no_gradient_from_a_function_behind_the_scan_is_a_gradient_of_zeros(gpu)
         assert t.grad is not None and not bool(t.grad.any())
 
 
+@pytest.mark.parametrize("out", [torch.int32, torch.bool], ids=str)
+def test_an_output_of_a_type_without_gradients_is_returned_without_one(gpu, out):
+    x, a, b, c, _ = make_inputs((2, 70, 24), seed=7)
+    leaves = [(8 * t).to(gpu).requires_grad_(True) for t in (x, a / 8, b, c)]
+    y = scan(*leaves, out_dtype=out)
+    with torch.no_grad():
+        want, final = scan_chunk(*leaves, out_dtype=out)
+    assert y.dtype == out and not y.requires_grad and torch.equal(y, want)
+    y, h = scan_chunk(*leaves, out_dtype=out)
+    assert not y.requires_grad and torch.equal(y, want) and torch.equal(h, final)
+    grads = torch.autograd.grad(h.sum(), leaves[:3])
+    full, h = scan_chunk(*leaves)
+    for got, ref in zip(grads, torch.autograd.grad(h.sum(), leaves[:3])):
+        assert torch.equal(got, ref)
+
+
 def test_a_trace_records_the_scan_instead_of_its_result(gpu):
     first, second = ([t.to(gpu) for t in make_inputs((2, 130, 24), seed=s)[:4]] for s in (1, 2))
     state = torch.randn(2, 24, generator=torch.Generator().manual_seed(3)).to(gpu)
