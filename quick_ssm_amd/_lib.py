@@ -244,6 +244,8 @@ def load_native(take_launch):
     import importlib.machinery
     import importlib.util
 
+    from torch.autograd.graph import Node
+
     load()
     if not NATIVE_PATH.exists():
         raise RuntimeError(f"{NATIVE_PATH} is missing: the native launch path is not built. "
@@ -259,6 +261,7 @@ def load_native(take_launch):
                 raise RuntimeError(f"{NATIVE_PATH} was built for version {module.abi_version} of the C ABI, this package "
                                    f"binds version {QSSM_VERSION}. Rebuild with `python -m quick_ssm_amd.build`.")
             module.set_hooks(take_launch, check)
+            Node.register(module.HipScanBackward)   # torch knows its own node types by name, others by registration
             sys.modules[name] = module
     return module
 

@@ -462,6 +462,10 @@ def test_a_gated_launch_uses_the_buffers_its_number_was_taken_for(monkeypatch):
     assert [a[0] for a in asked] == [n[0] for n in numbered]     # and the status of the block it ran with is asked for
 
 
+def test_the_native_autograd_node_is_one_of_torch_s_nodes():
+    assert issubclass(hip_scan._load_native().HipScanBackward, torch.autograd.graph.Node)
+
+
 def test_device_side_launch_count_never_repeats_a_flag_between_wipes(hip_lib):
     # Launches that number themselves (epoch argument 0) use flag count + 1 and the counting kernel stores the
     # next count.  Walk the arithmetic across both wraps: no flag is ever zero, flags grow by one between restarts,
