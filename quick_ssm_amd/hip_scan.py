@@ -346,22 +346,19 @@ def set_forward_keep(flag):
 
 
 def make_plan(B: int, L: int, D: int, in_dtype: torch.dtype, out_dtype: torch.dtype, direction: int,
-              align_elems: int, ckpt_stride: int = 0, tune: int = 0) -> Plan:
-    """Launch geometry for a shape (qssm_plan_scan; qssm_plan_scan_tuned when a test or sweep overrides single
-    choices with `tune`).  Plans depend on nothing but the arguments, so they are kept: small problems are bound by
-    the host side of a launch.  Callers must not modify the result."""
-    key = (B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune)
+              align_elems: int, ckpt_stride: int = 0, tune: int = 0, loose: bool = False) -> Plan:
+    """Launch geometry for a shape: with `loose` the plan that `scan_forward` and `scan_backward` launch
+    (qssm_plan_scan_loose), without it that of callers whose rows are all aligned to the lanes' width (qssm_plan_scan;
+    the two differ only where they are not).  `tune` overrides single choices, for a test or sweep.  Plans depend on
+    nothing but the arguments, so they are kept.  Callers must not modify the result."""
+    key = (B, L, D, in_dtype, out_dtype, direction, align_elems, ckpt_stride, tune, loose)
     plan = _plans.get(key)
     if plan is None:
         plan = Plan()
         lib = _lib.load()
-        if tune:
-            rc = lib.qssm_plan_scan_tuned(B, L, D, _DTYPE_CODE[in_dtype], _DTYPE_CODE[out_dtype], direction,
-                                          align_elems, ckpt_stride, tune, ctypes.byref(plan))
-        else:
-            rc = lib.qssm_plan_scan(B, L, D, _DTYPE_CODE[in_dtype], _DTYPE_CODE[out_dtype], direction,
-                                    align_elems, ckpt_stride, ctypes.byref(plan))
-        _lib.check(rc)
+        planner = lib.qssm_plan_scan_loose if loose else lib.qssm_plan_scan_tuned
+        _lib.check(planner(B, L, D, _DTYPE_CODE[in_dtype], _DTYPE_CODE[out_dtype], direction, align_elems, ckpt_stride,
+                           tune, ctypes.byref(plan)))
         if len(_plans) >= 4096:
             _plans.clear()
         _plans[key] = plan

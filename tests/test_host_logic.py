@@ -212,6 +212,8 @@ def _tile_accesses(plan, B, L, D):
         bi, strip = divmod(chain, plan.n_strips)
         d = strip * cols + dl
         dok = d < D
+        if plan.element_aligned:   # the last lane of a row ends with it
+            d = np.minimum(d, D - plan.vec)
         for seg in range(plan.n_seg):
             t0 = seg * plan.seg_len + j * plan.steps
             for i in range(plan.steps):

@@ -42,6 +42,60 @@ def test_every_column_is_covered_and_nothing_beyond_the_rows(D):
                     assert (first >= strip).all()
 
 
+def test_loose_plans_describe_launches_that_stay_in_bounds():
+    # What the sweeps over strict plans check, for the plans that scan() launches: geometry, buffer sizes, and every
+    # lane's elements, saved states and words.
+    import random
+
+    from test_host_logic import _tile_accesses
+
+    rng = random.Random(77)
+    pairs = [(torch.float32, torch.float32), (torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+             (torch.float16, torch.float32), (torch.bfloat16, torch.float32)]
+    loose = 0
+    for _ in range(150):
+        B, L = rng.choice([1, 2, 3]), rng.choice([1, 5, 31, 33, 64, 127, 200, 513, 1030])
+        D = rng.choice([1, 3, 31, 32, 33, 34, 47, 63, 65, 77, 130, 255, 258, 333, 514, 777])
+        dt, odt = rng.choice(pairs)
+        align = rng.choice([a for a in (1, 2, 4, 8) if a == 1 or D % a == 0])
+        tune = rng.choice([0, 0, 4, 6, 8]) | (rng.choice([0, 4, 8]) << 8) | (rng.choice([0, 1, 3]) << 28)
+        try:
+            bwd = hip_scan.make_plan(B, L, D, dt, odt, _lib.QSSM_BACKWARD, align, 0, tune, loose=True)
+            fwd = hip_scan.make_plan(B, L, D, dt, odt, _lib.QSSM_FORWARD, align, bwd.seg_len, loose=True)
+        except Exception as exc:   # a forced geometry the planner refuses is fine; anything else is not
+            assert tune and ("LDS" in str(exc) or "ckpt_stride" in str(exc)), (B, L, D, dt, odt, align, tune, str(exc))
+            continue
+        for p in (bwd, fwd):
+            what = (B, L, D, dt, odt, align, tune, p.describe())
+            loose += p.element_aligned
+            assert p.vec <= D and (p.element_aligned or (D % p.vec == 0 and align % p.vec == 0)), what
+            assert p.seg_len == p.steps * (p.threads >> p.g_log2) and p.seg_len % p.ckpt_stride == 0, what
+            assert p.n_strips == -(-D // p.strip_cols) and p.n_seg == -(-L // p.seg_len), what
+            assert 0 < p.lds_bytes <= 64 * 1024, what
+            assert p.ckpt_elems == B * p.n_ckpt * D and p.n_ckpt == -(-L // p.ckpt_stride), what
+            lo, hi, hi_ckpt, hi_word = _tile_accesses(p, B, L, D)
+            assert lo >= 0 and hi == B * L * D - 1, what
+            assert hi_ckpt < p.ckpt_elems and hi_word <= p.workspace_bytes, what
+        assert fwd.ckpt_stride == bwd.ckpt_stride == bwd.seg_len
+    assert loose >= 80
+
+
+def test_a_misaligned_backward_reads_the_states_of_a_gated_forward():
+    # The gated scan's two-pass backward takes y's gradient as autograd hands it over, one element off alignment if it
+    # must be: a loose plan that meets the spacing the gated forward saved its states with.
+    from quick_ssm_amd import gated_scan
+
+    for dtype, compute, out in ((torch.bfloat16, torch.bfloat16, torch.float32), (torch.float16, torch.float16, torch.float32),
+                                (torch.float32, torch.float16, torch.float32), (torch.float32, torch.float32, torch.float32)):
+        for B in (1, 3, 16):
+            for L in (1, 2, 5, 6, 7, 9, 17, 33, 100, 1000, 4096, 65536):
+                for S in (128, 132, 136, 264, 688, 1008, 1024, 4096):
+                    stride = gated_scan._plan(B, L, S, dtype, compute, dtype, _lib.QSSM_BACKWARD, 0).seg_len
+                    for align in (1, 2, 4, 8):
+                        p = hip_scan.make_plan(B, L, S, compute, out, _lib.QSSM_BACKWARD, align, stride, loose=True)
+                        assert p.ckpt_stride == stride and p.seg_len % stride == 0, (B, L, S, dtype, compute, align)
+
+
 SHAPES = [(2, 300, 33), (3, 100, 35), (2, 1100, 257), (1, 700, 258), (2, 513, 777), (1, 5000, 61), (64, 1, 1027)]
 
 

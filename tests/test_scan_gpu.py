@@ -1418,6 +1418,6 @@ def test_seeded_random_shapes_match_the_oracle(gpu):
         for k in ("dx", "da", "db", "dc"):
             assert_close(k, got[k], ref[k], TOL[dtype])
         align = 8 if D % 8 == 0 else 4 if D % 4 == 0 else 2 if D % 2 == 0 else 1
-        plan = hip_scan.make_plan(B, L, D, dtype, out_dtype, _lib.QSSM_BACKWARD, align, 0)
+        plan = hip_scan.make_plan(B, L, D, dtype, out_dtype, _lib.QSSM_BACKWARD, align, 0, loose=True)   # as launched
         seen.add((plan.vec, plan.g_log2, plan.cluster))
     assert len({c for _, _, c in seen}) >= 3, seen     # the draw really covers several cluster sizes
