@@ -72,3 +72,34 @@ def test_nothing_is_kept_for_the_backward_that_five_products_would_not_keep(gpu,
         del y
     # (the five weights are 10 MB, what the graph keeps of the activations 3; tensors are rounded up to 512 bytes)
     assert kept["one"] <= kept["five"] + (1 << 17)
+
+
+@pytest.mark.parametrize("dtype,compute", [(torch.float32, torch.float16), (torch.bfloat16, torch.bfloat16)], ids=["f32", "bf16"])
+def test_autocast_calls_the_projections_themselves(gpu, monkeypatch, dtype, compute):
+    # Under autocast torch decides what type a product runs in: neither the split products nor the one wide product may
+    # stand in for the modules' calls.
+    monkeypatch.setattr(SSM, "_BATCHED_PROJECTION_LIMIT", 0)
+    monkeypatch.setattr(layers.split_linear, "MIN_WORK", 1)
+    torch.manual_seed(2)
+    layer = SSM(256, 2, dtype=dtype, device=gpu, compute_dtype=compute)
+    x = torch.randn(2, 150, 256, device=gpu, dtype=dtype, requires_grad=True)
+    dy = torch.randn_like(x)
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = layer(x)
+            return [y.detach(), *torch.autograd.grad(y, [x, *layer.parameters()], dy.to(y.dtype))]
+
+    def refuse(*a, **k):
+        raise AssertionError("not under autocast")
+
+    calls = []
+    handles = [m.register_forward_hook(lambda *a: calls.append(1)) for m in layer._projections(False)[0]]
+    want = step()
+    for h in handles:
+        h.remove()
+    assert len(calls) == 5
+    monkeypatch.setattr(layers.split_linear, "forward", refuse)
+    monkeypatch.setattr(layers._WideProjections, "apply", refuse)
+    for got, ref in zip(step(), want):
+        assert got.dtype == ref.dtype and torch.equal(got, ref)
