@@ -17,12 +17,13 @@ from . import hip_scan
 
 Tensor = torch.Tensor
 
-# Multiply-adds (over all weights of a launch) below which the library's product stays, because filling and draining the
-# launch and the sums over parts exceed the gain.  GPU us for output, input gradient and weight gradient, library against
-# these: 2^31 (2048 rows, 2048 -> 512) 34, 36, 35 against 44, 39, 45; 2^31.3 (2048 rows, 256 -> 5120) 56, 47, 66 against 56,
-# 53, 54; 2^32 (8192 rows, 2048 -> 256) 69, 74, 71 against 69, 70, 69; 2^32.3 (4096 rows, 256 -> 5120) 101, 94, 127 against
-# 95, 82, 85; 2^33.3 (4096 rows, 512 -> 5120) 167, 158, 187 against 144, 139, 144.
-MIN_WORK = 1 << 32
+# Multiply-adds (over all weights of a launch) below which the library's product stays.  GPU us for output, input gradient
+# and weight gradient, library against these: 2^31 (2048 rows, 2048 -> 512) 34, 36, 35 against 44, 39, 45; 2^32 (8192 rows,
+# 2048 -> 256) 69, 74, 71 against 69, 70, 69; 2^32.3 (4096 rows, 256 -> 5120) 101, 94, 127 against 95, 82, 85; 2^33.3 (4096
+# rows, 512 -> 5120) 167, 158, 187 against 144, 139, 144.  They cross at 2^32; the line is above the copy task's stack
+# (2^32.3 a layer, 8 % of its step), whose six layers in fp16 carry a difference in a product's last bits on to 3e-3 of a
+# gradient: at that size every program's results stay those of the library's products.
+MIN_WORK = 1 << 33
 
 # An input narrower than this has few stages to fill a tile's pipeline with before its results are stored: 16384 rows,
 # 128 -> 2560, 105 us against 118, where the gradients gain (83 and 139 against 83 and 85); at 256 columns 174 against 171.
