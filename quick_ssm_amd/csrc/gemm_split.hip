@@ -110,7 +110,7 @@ constexpr int kPartA[6] = {2, 0, 1, 1, 0, 0}, kPartB[6] = {0, 2, 1, 0, 1, 0};
 // stages of 16 k's in two LDS buffers with one barrier per stage.  A stage's fp32 elements are in flight to registers while
 // the stage before it is multiplied; they are split on their way into LDS, so no 16-bit copy of an operand exists in
 // memory.  48 KB of LDS and under 256 registers: two workgroups per compute unit, one multiplying while the other waits
-// or splits.  The products of a layer with 32768 rows, hidden 1024, state 4096 run at 183, 188 and 184 TFLOP/s (outputs, input
+// or splits.  The products of a layer with 32768 rows, hidden 1024, state 4096 run at 189, 195 and 188 TFLOP/s (outputs, input
 // gradient, weight gradients), six times that on the bf16 units, near the 1.2 PFLOP/s of a large bf16 product of the library
 // on this card; the library's fp32 kernels reach 143 to 152.  Matrix cores busy 59 % of the cycles, at 1.8 GHz; 5.4 other
 // vector instructions per product, most of them conversions, take two thirds of the issue slots beside them.

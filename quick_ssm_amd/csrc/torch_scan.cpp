@@ -1,12 +1,12 @@
 // Native half of the Python package's scan: output tensors, launch plans, the launches and the autograd nodes.
 //
 // A training step over a small tensor is bound by the host: two launches keep the GPU busy for under 20 us, and the
-// interpreter needed 150 us to make them (a Python autograd node runs on autograd's own thread, on a core that has to
+// interpreter needed 114 to 142 us to make them (a Python autograd node runs on autograd's own thread, on a core that has to
 // be woken and under the interpreter lock).  Here a forward is one call from Python, and the backward node runs without
 // the interpreter except for the few bytecodes that number the launch (quick_ssm_amd/hip_scan.py keeps the control
 // block and workspace of every stream and is the only place that numbers launches).  Measured, Python node -> this one:
-// fp32 B=4 L=2048 D=16 forward + backward 150 -> 79 us (of which torch's own hand-over to its thread and back is about
-// 45), fp16 B=2 L=8192 D=512 with a carried state 179 -> 94 us, one token of generation 22.3 -> 10.1 us.
+// fp32 B=4 L=2048 D=16 forward + backward 114-142 -> 78 us (of which torch's own hand-over to its thread and back is
+// about 45), fp16 B=2 L=8192 D=512 with a carried state 170 -> 95 us, one token of generation 21.8 -> 10.5 us.
 //
 // Takes the place of the Python bodies of the reference's `_TritonScanFunction` (quick_ssm/scan_interface.py:49-158).
 #include <Python.h>
