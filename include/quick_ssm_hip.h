@@ -135,7 +135,9 @@ QSSM_API int qssm_plan_scan_tuned(int32_t B, int32_t L, int32_t D, int32_t in_dt
 /*
  * qssm_plan_scan_tuned for tensors whose rows are not all aligned to the lanes' width, or not divided by it: from 32
  * columns on such plans keep 8 or 16 bytes per lane at element alignment (`element_aligned`), where the other planners
- * narrow the lanes to `align_elems` columns.  The same plan as theirs for everything else.
+ * narrow the lanes to `align_elems` columns.  The same plan as theirs for everything else.  With `element_aligned` two
+ * lanes compute and store the columns they share, so results and outgoing states must not share memory with operands or
+ * incoming states.
  */
 QSSM_API int qssm_plan_scan_loose(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype,
                          int32_t direction, int32_t align_elems, int32_t ckpt_stride, int32_t tune,

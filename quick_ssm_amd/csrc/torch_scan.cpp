@@ -195,6 +195,14 @@ void check_state(const Tensor& t, int64_t B, int64_t D, const Tensor& like, cons
                     t.scalar_type(), " ", t.sizes(), " on ", t.device());
 }
 
+// A state that the launch reads, as memory of its own when the launch also writes to it (a state carried in place): where
+// lanes share columns, and where a chain's first tiles read the state that its last one replaces, the order is nobody's.
+Tensor read_state(const Tensor& t, const Tensor& written) {
+  if (!t.defined() || !written.defined() || t.numel() == 0) return t;
+  const char *r = (const char*)t.const_data_ptr(), *w = (const char*)written.const_data_ptr();
+  return r < w + written.nbytes() && w < r + t.nbytes() ? t.clone() : t;
+}
+
 void* data_or_null(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
 const float* floats_or_null(const Tensor& t) { return t.defined() ? t.const_data_ptr<float>() : nullptr; }
 
@@ -258,7 +266,8 @@ ForwardOut scan_forward(const Tensor& x, const Tensor& a, const Tensor& b, const
   k.h_out = (float*)data_or_null(out.h);
   k.sy = k.sh = dense;
   k.ckpt = (float*)data_or_null(out.ckpt);
-  k.h_init = floats_or_null(h_init);
+  const Tensor h0 = read_state(h_init, h_final);
+  k.h_init = floats_or_null(h0);
   k.h_final = (float*)data_or_null(h_final);
   launch(k, plan, x.get_device(), qssm_scan_forward_call);
   return out;
@@ -305,8 +314,9 @@ Grads scan_backward(const Tensor& x, const Tensor& a, const Tensor& b, const Ten
   k.x = ox.p; k.a = oa.p; k.b = ob.p; k.c = oc.p; k.dy = og.p; k.h = (const float*)oh.p;
   k.sx = ox.s; k.sa = oa.s; k.sb = ob.s; k.sc = oc.s; k.sdy = og.s; k.sh = oh.s;
   k.ckpt = floats_or_null(saved);
+  const Tensor g_final = read_state(dh_final, dh_init);
   k.h_init = floats_or_null(h_init);
-  k.dh_final = floats_or_null(dh_final);
+  k.dh_final = floats_or_null(g_final);
   k.dh_init = (float*)data_or_null(dh_init);
   k.dx = data_or_null(out.g[0]); k.da = data_or_null(out.g[1]); k.db = data_or_null(out.g[2]); k.dc = data_or_null(out.g[3]);
   k.sdx = k.sda = k.sdb = k.sdc = dense;

@@ -1,7 +1,7 @@
 """Host side of the HIP scan: workspace, launch numbering, and the two launches.
 
-Everything here and in csrc/torch_scan.cpp (output tensors, plans, the call itself) is plumbing around `qssm_scan_forward` / `qssm_scan_backward`
-(include/quick_ssm_hip.h).  It takes the place of the launch code in the reference's
+Everything here and in csrc/torch_scan.cpp (output tensors, plans, the call itself) is plumbing around
+`qssm_scan_forward` / `qssm_scan_backward` (include/quick_ssm_hip.h).  It takes the place of the launch code in the reference's
 `block_scan_forward_3d` (quick_ssm/triton_forwards.py:134-172) and `block_scan_backward_3d`
 (quick_ssm/triton_backwards.py:168-209): no fp32 upcast copies, no N-sized scratch, one launch per
 direction.

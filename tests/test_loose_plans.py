@@ -141,3 +141,25 @@ def test_states_cross_pieces_of_odd_rows(gpu):
     for got, want in zip((torch.cat(ys, 1), *torch.autograd.grad(torch.cat(ys, 1), parts, dy)),
                          (y, *torch.autograd.grad(y, whole, dy))):
         assert_close("piecewise", got.detach().cpu(), want.detach().cpu().numpy(), 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(64, 1, 1027), (3, 40, 333), (2, 900, 515)], ids=lambda s: "x".join(map(str, s)))
+def test_a_state_carried_in_place_is_read_before_it_is_written(gpu, shape):
+    # Two lanes share columns of a row, and a chain's last tile writes the state that its first ones read.
+    x, a, b, c, dy = (t.to(gpu) for t in make_inputs(shape, seed=9))
+    state = torch.randn(shape[0], shape[2], generator=torch.Generator().manual_seed(1)).to(gpu)
+    want = torch.empty_like(state)
+    y, _, ckpt, stride = hip_scan.scan_forward(x, a, b, c, out_dtype=torch.float32, want_ckpt=True, h_init=state, h_final=want)
+    for _ in range(20):
+        moved = state.clone()
+        again = hip_scan.scan_forward(x, a, b, c, out_dtype=torch.float32, h_init=moved, h_final=moved)[0]
+        assert torch.equal(again, y) and torch.equal(moved, want)
+    grad, out = torch.randn_like(state), torch.empty_like(state)
+    args = dict(ckpt=ckpt, ckpt_stride=stride, h_init=state)
+    want = hip_scan.scan_backward(x, a, b, c, dy, dh_final=grad, dh_init=out, **args)
+    for _ in range(20):
+        moved = grad.clone()
+        got = hip_scan.scan_backward(x, a, b, c, dy, dh_final=moved, dh_init=moved, **args)
+        assert torch.equal(moved, out) and all(torch.equal(g, w) for g, w in zip(got, want))
+    assert hip_scan.workspace_status() == 0
