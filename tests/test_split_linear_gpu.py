@@ -11,13 +11,13 @@ def _error(got, ref):
     return ((got.double() - ref).norm() / ref.norm()).item()
 
 
-# Bound of the relative error (2-norm): 2^-23 for the split (the rounding of lo and the left-out lo*lo are 2^-24 of a
-# product each) plus the fp32 accumulation of up to K / 16 * 3 sums of a part, 2^-24 * sqrt(3 K / 16) and no more.
+# Bound of the relative error (2-norm): 2^-23 for the split (what it leaves out of a pair is below 2^-24 of it) plus the
+# fp32 accumulation of up to K / 16 * 3 sums of a part, 2^-24 * sqrt(3 K / 16) and no more.
 def _bound(k):
     return 2.0 ** -23 + 2.0 ** -24 * (3 * k / 16) ** 0.5
 
 
-# tiles are 256 x 128 and stages 16 long: one below, on and above each edge, several launches' worth, and the
+# tiles are 128 x 128 and stages 16 long: one below, on and above each edge, several launches' worth, and the
 # layer's own ratios
 SHAPES = [(256, 16, 128, 1), (255, 20, 132, 1), (257, 12, 124, 5), (1, 64, 64, 1), (1000, 72, 260, 2), (4096, 256, 1280, 1),
           (2048, 256, 512, 5), (515, 1024, 256, 1), (16384, 36, 64, 3)]
