@@ -3,9 +3,9 @@
 A layer with fp32 parameters spends nine tenths of its time in its projections (quick_ssm/layers.py:76-80,106): the
 library's fp32 products run at the fp32 MFMA rate, a sixteenth of the bf16 one.  `qssm_gemm_f32` takes every element as
 the sum of three bf16 values, which hold all of its bits, and accumulates six products in fp32; measured against float64
-it is two to nine times closer than fp32 products (one nonzero product in a sum: 2 % further, 2.6e-8).  Here is the rule
-for when it is used; scratch and the calls are in csrc/torch_scan.cpp, the autograd functions that use them in
-quick_ssm_amd/layers.py.
+it is 1.2 (rows of two nonzeros) to nine times (long sums) closer than fp32 products, and 2 % further off for a sum of one
+nonzero pair (2.60e-8 against 2.54e-8).  Here is the rule for when it is used; scratch and the calls are in
+csrc/torch_scan.cpp, the autograd functions that use them in quick_ssm_amd/layers.py.
 """
 from __future__ import annotations
 
