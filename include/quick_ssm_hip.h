@@ -516,6 +516,15 @@ QSSM_API int qssm_gemm_f32(const qssm_gemm_f32_call* call, void* stream);
 QSSM_API int qssm_gemm_f32_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments);
 
 /*
+ * The same product with scratch for a copy of its smaller operand in parts (6 bytes per element), which makes large ones a
+ * quarter faster.  qssm_gemm_f32_packed_plan sets `splits` to the number that suits the call and `*bytes` to the scratch
+ * (`packed`, 16-byte aligned) that qssm_gemm_f32_packed then wants; the shapes, the layouts and the operands' addresses are
+ * set before it.  `*bytes` = 0: the call is one for qssm_gemm_f32 (small, or M or N within a tile of 2^31).
+ */
+QSSM_API int qssm_gemm_f32_packed_plan(qssm_gemm_f32_call* call, uint64_t* bytes);
+QSSM_API int qssm_gemm_f32_packed(const qssm_gemm_f32_call* call, void* packed, uint64_t bytes, void* stream);
+
+/*
  * Streaming copy of `bytes` bytes (16-byte aligned, multiple of 16) on `stream`.  Not part of
  * the scan: it is the known-size kernel against which rocprof's FETCH_SIZE / WRITE_SIZE
  * counters and the achievable-bandwidth ceiling are calibrated by the benchmark.

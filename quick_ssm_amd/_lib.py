@@ -52,6 +52,8 @@ EXPORTED_SYMBOLS = (
     "qssm_colsum",
     "qssm_gemm_f32",
     "qssm_gemm_f32_splits",
+    "qssm_gemm_f32_packed_plan",
+    "qssm_gemm_f32_packed",
     "qssm_copy_bytes",
     "qssm_launch_count_step",
 )

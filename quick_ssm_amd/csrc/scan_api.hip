@@ -987,28 +987,34 @@ int qssm_colsum(const void* x, int64_t ld, int64_t rows, int32_t S, int32_t dtyp
   return e == hipSuccess ? 0 : hip_fail(e, "colsum kernel launch");
 }
 
-int qssm_gemm_f32_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments) {
-  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || segments <= 0) return 1;
-  // Two workgroups per compute unit run at once, so a launch takes whole rounds of 512 of them, and its last round is
-  // shorter per stage of 16 k's if there is but one for each unit.  Several parts write and read C once more each.  The us
-  // below fit 66 products of 2^30 to 2^36 multiply-adds in 1 to 32 parts to 6 %; the parts chosen by them are the fastest
-  // measured ones for 59 of the products and within 3 % for all.
-  const double kStage = 1.29, kLoneStage = 0.72, kRound = 12.4, kPartMb = 0.087, kParts = 4.7;
+// Two workgroups per compute unit run at once, so a launch takes whole rounds of 512 of them, and its last round is
+// shorter per stage of 16 k's if there is but one for each unit.  Several parts write and read C once more each.  The us
+// below fit 66 products of 2^30 to 2^36 multiply-adds in 1 to 32 parts to 6 %; the parts chosen by them are the fastest
+// measured ones for 59 of the products and within 3 % for all.
+static const double kPartMb = 0.087, kParts = 4.7;
+static double gemm_cost(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments, int s) {
+  const double kStage = 1.29, kLoneStage = 0.72, kRound = 12.4;
   const double stages = (double)split_gemm_stages(K, segments), out_mb = (double)M * N * batch * 4e-6;
   const int64_t tiles = split_gemm_tiles(M, N, batch), wave = 2 * kCUs;
+  const int64_t full = tiles * s / wave, rest = tiles * s % wave;
+  double cost = (double)full * (stages / s * kStage + kRound);
+  if (rest > 0) cost += stages / s * (rest <= kCUs ? kLoneStage : kStage) + kRound;
+  if (s > 1) cost += (2 * s + 1) * out_mb * kPartMb + kParts;
+  return cost;
+}
+
+int qssm_gemm_f32_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments) {
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || segments <= 0) return 1;
   int best = 1;
   double best_cost = 0.0;
-  for (int s = 1; s <= 32 && (s == 1 || stages / s >= 16.0); ++s) {
-    const int64_t full = tiles * s / wave, rest = tiles * s % wave;
-    double cost = (double)full * (stages / s * kStage + kRound);
-    if (rest > 0) cost += stages / s * (rest <= kCUs ? kLoneStage : kStage) + kRound;
-    if (s > 1) cost += (2 * s + 1) * out_mb * kPartMb + kParts;
+  for (int s = 1; s <= 32 && (s == 1 || (double)split_gemm_stages(K, segments) / s >= 16.0); ++s) {
+    const double cost = gemm_cost(M, N, K, batch, segments, s);
     if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
   }
   return best;
 }
 
-int qssm_gemm_f32(const qssm_gemm_f32_call* k, void* stream) {
+static int check_gemm(const qssm_gemm_f32_call* k) {
   if (k == nullptr) return fail(QSSM_EINVAL, "call is NULL");
   if (k->M < 0 || k->N < 0 || k->K < 1) return fail(QSSM_EINVAL, "bad dimension");
   if (k->batch < 1 || k->batch > QSSM_GEMM_MANY || k->segments < 1 || k->segments > QSSM_GEMM_MANY ||
@@ -1029,32 +1035,127 @@ int qssm_gemm_f32(const qssm_gemm_f32_call* k, void* stream) {
   const uint64_t floats = k->splits > 1 ? (uint64_t)k->splits * k->batch * k->M * k->N : 0;
   if (floats > 0 && (k->partial == nullptr || k->partial_floats < floats || ((uintptr_t)k->partial) % 16 != 0))
     return fail(QSSM_EWORKSPACE, "partial needs %llu floats, 16-byte aligned", (unsigned long long)floats);
-  SplitGemmArgs p;
-  memset(&p, 0, sizeof(p));
   const int pairs = k->batch > k->segments ? k->batch : k->segments;
   for (int i = 0; i < pairs; ++i) {
     if (k->a[i] == nullptr || k->b[i] == nullptr) return fail(QSSM_EINVAL, "NULL operand");
     if (((uintptr_t)k->a[i]) % 16 != 0 || ((uintptr_t)k->b[i]) % 16 != 0) return fail(QSSM_EALIGN, "operands must be 16-byte aligned");
-    p.a[i] = k->a[i];
-    p.b[i] = k->b[i];
   }
   for (int i = 0; i < k->batch; ++i) {
     if (k->c[i] == nullptr) return fail(QSSM_EINVAL, "NULL result");
     if (((uintptr_t)k->c[i]) % 16 != 0) return fail(QSSM_EALIGN, "results must be 16-byte aligned");
-    p.c[i] = k->c[i];
-    p.bias[i] = k->bias[i];
   }
+  if (split_gemm_tiles(k->M, k->N, k->batch) * k->splits > 0x7fffffffll || split_gemm_stages(k->K, k->segments) * kSplitStageK > 0x7fffffffll ||
+      (int64_t)k->M * k->N / 4 * k->batch > 0x7fffffffll * 128)
+    return fail(QSSM_EINVAL, "product too large for one launch");
+  return 0;
+}
+
+int qssm_gemm_f32(const qssm_gemm_f32_call* k, void* stream) {
+  const int rc = check_gemm(k);
+  if (rc != 0 || k->M == 0 || k->N == 0) return rc;
+  SplitGemmArgs p;
+  memset(&p, 0, sizeof(p));
+  for (int i = 0; i < QSSM_GEMM_MANY; ++i) { p.a[i] = k->a[i]; p.b[i] = k->b[i]; p.c[i] = k->c[i]; p.bias[i] = k->bias[i]; }
   p.lda = k->lda; p.ldb = k->ldb; p.ldc = k->ldc;
   p.M = k->M; p.N = k->N; p.K = k->K;
   p.batch = k->batch; p.segments = k->segments; p.splits = k->splits;
   p.partial = k->partial;
-  if (split_gemm_tiles(p.M, p.N, p.batch) * p.splits > 0x7fffffffll || split_gemm_stages(p.K, p.segments) * kSplitStageK > 0x7fffffffll ||
-      (int64_t)p.M * p.N / 4 * p.batch > 0x7fffffffll * 128)
-    return fail(QSSM_EINVAL, "product too large for one launch");
   if (!launch_split_gemm(p, k->a_kstrided != 0, k->b_kstrided != 0, (hipStream_t)stream))
     return fail(QSSM_EINVAL, "operand layout is not built");
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : hip_fail(e, "split_gemm_kernel launch");
+}
+
+static int distinct(const float* const* v, int n) {
+  for (int i = 1; i < n; ++i)
+    if (v[i] != v[0]) return n;
+  return 1;
+}
+
+// Which operand of a call is packed, into how many parts its k's are dealt and how many bytes the packed operand takes.
+// One workgroup per compute unit: us of a stage of 32 k's, of a tile's start and end, of 2^20 packed elements and of the
+// parts' way through memory.  (600 rows, gradient of five 1024 -> 4096: the rows fill their tiles of 128 to 94 % and tiles of
+// 256 to 78 %, so the weights are packed although they are more.)
+struct PackedChoice {
+  bool swap;
+  int many, splits;
+  uint64_t bytes;
+  double cost;
+};
+static PackedChoice packed_choice(const qssm_gemm_f32_call* k) {
+  const double kStage = 1.95, kRound = 12.0, kPack = 2.24;
+  const int pairs = k->batch > k->segments ? k->batch : k->segments;
+  const double stages = (double)packed_gemm_stages(k->K, k->segments), out_mb = (double)k->M * k->N * k->batch * 4e-6;
+  // Never fewer parts than the other kernel takes: shorter sums are rounded less often.
+  const int least = qssm_gemm_f32_splits(k->M, k->N, k->K, k->batch, k->segments);
+  PackedChoice best = {false, 0, least, 0, 0.0};
+  for (int swap = 0; swap < 2; ++swap) {
+    const int32_t rows = swap ? k->M : k->N;
+    const int many = k->segments > 1 ? pairs : distinct(swap ? k->a : k->b, pairs);
+    const int64_t tiles = swap ? packed_gemm_tiles(k->N, k->M, k->batch) : packed_gemm_tiles(k->M, k->N, k->batch);
+    const double pack = (double)rows * k->K * many * (kPack / (1 << 20)) + 3.0;
+    for (int s = least; s <= 64 && (s == least || stages / s >= 8.0); ++s) {
+      double cost = pack + (double)((tiles * s + kCUs - 1) / kCUs) * (stages / s * kStage + kRound);
+      if (s > 1) cost += (2 * s + 1) * out_mb * kPartMb + kParts;
+      if (best.many == 0 || cost < best.cost) best = {swap != 0, many, s, packed_bytes(rows, k->K, many), cost};
+    }
+  }
+  return best;
+}
+
+// Whether the packed kernel's counts stay within 32 bits.
+static bool packed_fits(const qssm_gemm_f32_call* k, const PackedChoice& c) {
+  return k->M <= 0x7fffffff - kPackedTileN && k->N <= 0x7fffffff - kPackedTileN && c.bytes / kPackedPiece <= 0x7fffffffull;
+}
+
+int qssm_gemm_f32_packed_plan(qssm_gemm_f32_call* k, uint64_t* bytes) {
+  if (k == nullptr || bytes == nullptr) return fail(QSSM_EINVAL, "NULL argument");
+  *bytes = 0;
+  k->splits = 1;
+  if (k->M <= 0 || k->N <= 0 || k->K <= 0 || k->batch < 1 || k->batch > QSSM_GEMM_MANY || k->segments < 1 ||
+      k->segments > QSSM_GEMM_MANY)
+    return 0;
+  const PackedChoice c = packed_choice(k);
+  const int plain = qssm_gemm_f32_splits(k->M, k->N, k->K, k->batch, k->segments);
+  if (!packed_fits(k, c) || gemm_cost(k->M, k->N, k->K, k->batch, k->segments, plain) <= c.cost) {
+    k->splits = plain;
+    return 0;
+  }
+  k->splits = c.splits;
+  *bytes = c.bytes;
+  return 0;
+}
+
+int qssm_gemm_f32_packed(const qssm_gemm_f32_call* k, void* packed, uint64_t bytes, void* stream) {
+  const int rc = check_gemm(k);
+  if (rc != 0 || k->M == 0 || k->N == 0) return rc;
+  const PackedChoice c = packed_choice(k);
+  if (packed == nullptr || bytes < c.bytes || ((uintptr_t)packed) % 16 != 0)
+    return fail(QSSM_EWORKSPACE, "packed needs %llu bytes, 16-byte aligned", (unsigned long long)c.bytes);
+  if (!packed_fits(k, c) || (c.swap ? packed_gemm_tiles(k->N, k->M, k->batch) : packed_gemm_tiles(k->M, k->N, k->batch)) * k->splits > 0x7fffffffll)
+    return fail(QSSM_EINVAL, "product too large for one launch");
+  PackedGemmArgs p;
+  memset(&p, 0, sizeof(p));
+  for (int i = 0; i < QSSM_GEMM_MANY; ++i) {
+    p.a[i] = c.swap ? k->b[i] : k->a[i];
+    p.b[i] = c.swap ? k->a[i] : k->b[i];
+    p.c[i] = k->c[i];
+    p.bias[i] = k->bias[i];
+  }
+  p.lda = c.swap ? k->ldb : k->lda;
+  p.ldb = c.swap ? k->lda : k->ldb;
+  p.ldc = k->ldc;
+  p.M = c.swap ? k->N : k->M;
+  p.N = c.swap ? k->M : k->N;
+  p.K = k->K;
+  p.batch = k->batch; p.segments = k->segments; p.splits = k->splits;
+  p.b_kstrided = c.swap ? k->a_kstrided : k->b_kstrided;
+  p.packed_each = c.many > 1;
+  p.packed = (char*)packed;
+  p.partial = k->partial;
+  launch_packed_gemm(p, (c.swap ? k->b_kstrided : k->a_kstrided) != 0, c.swap, (hipStream_t)stream);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : hip_fail(e, "packed_gemm_kernel launch");
 }
 
 int qssm_launch_count_step(uint32_t count, int32_t static_scratch, uint32_t* flag, uint32_t* next, int32_t* wipes) {

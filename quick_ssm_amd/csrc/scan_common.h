@@ -588,4 +588,33 @@ int64_t split_gemm_tiles(int64_t M, int64_t N, int64_t batch);
 int64_t split_gemm_stages(int64_t K, int64_t segments);
 bool launch_split_gemm(const SplitGemmArgs& args, bool a_kstrided, bool b_kstrided, hipStream_t stream);
 
+// The same with B taken from a copy in parts, which the launch makes first.
+constexpr int kPackedTileM = 128, kPackedTileN = 256, kPackedStageK = 32;
+constexpr int kPackedPiece = 3 * kPackedTileN * kPackedStageK * 2;   // bytes of a tile's stage of B in parts
+
+struct PackArgs {
+  const float* src[kSplitGemmMany];   // one matrix per product or run
+  char* dst;
+  int64_t ld;
+  int rows, K, segments, stages_per, tiles_per;
+};
+
+struct PackedGemmArgs {
+  const float *a[kSplitGemmMany], *b[kSplitGemmMany];
+  float* c[kSplitGemmMany];
+  const float* bias[kSplitGemmMany];
+  int64_t lda, ldb, ldc;
+  int M, N, K;
+  int batch, segments, splits;
+  int b_kstrided;
+  int packed_each;   // products with a B of their own each (0: one B for all)
+  char* packed;
+  float* partial;
+};
+
+int64_t packed_gemm_tiles(int64_t M, int64_t N, int64_t batch);
+int64_t packed_gemm_stages(int64_t K, int64_t segments);
+uint64_t packed_bytes(int64_t N, int64_t K, int64_t many);
+void launch_packed_gemm(const PackedGemmArgs& args, bool a_kstrided, bool trans, hipStream_t stream);
+
 }  // namespace qssm

@@ -406,13 +406,16 @@ void product(const std::vector<Tensor>& a, const std::vector<Tensor>& b, const s
   k.segments = batch == 1 ? (int32_t)a.size() : 1;
   k.a_kstrided = a_kstrided;
   k.b_kstrided = b_kstrided;
-  k.splits = qssm_gemm_f32_splits(k.M, k.N, k.K, batch, k.segments);
+  uint64_t bytes = 0;
+  check_rc(qssm_gemm_f32_packed_plan(&k, &bytes));
+  const Tensor packed = at::empty({(int64_t)bytes}, c[0].options().dtype(at::kByte));
   if (k.splits > 1) {
     partial = matrix((int64_t)k.splits * batch * k.M, k.N, c[0]);
     k.partial = partial.mutable_data_ptr<float>();
     k.partial_floats = (uint64_t)partial.numel();
   }
-  check_rc(qssm_gemm_f32(&k, stream_of(c[0])));
+  if (bytes == 0) check_rc(qssm_gemm_f32(&k, stream_of(c[0])));
+  else check_rc(qssm_gemm_f32_packed(&k, packed.mutable_data_ptr(), bytes, stream_of(c[0])));
 }
 
 bool matrix_ok(const Tensor& t, int64_t rows, int64_t cols, const Tensor& like) {

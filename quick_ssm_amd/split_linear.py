@@ -18,16 +18,15 @@ from . import hip_scan
 Tensor = torch.Tensor
 
 # Multiply-adds (over all weights of a launch) below which the library's product stays.  GPU us for output, input gradient
-# and weight gradient, library against these: 2^31 (2048 rows, 2048 -> 512) 34, 36, 35 against 44, 39, 45; 2^32 (8192 rows,
-# 2048 -> 256) 69, 74, 71 against 69, 70, 69; 2^32.3 (4096 rows, 256 -> 5120) 101, 94, 127 against 95, 82, 85; 2^33.3 (4096
-# rows, 512 -> 5120) 167, 158, 187 against 144, 139, 144.  They cross at 2^32; the line is above the copy task's stack
-# (2^32.3 a layer, 8 % of its step), whose six layers in fp16 carry a difference in a product's last bits on to 3e-3 of a
-# gradient: at that size every program's results stay those of the library's products.
+# and weight gradient, library against these: 2^30 (4096 rows, 1024 -> 256) 24, 25, 30 against 41, 33, 42; 2^32.3 (4096 rows,
+# 256 -> 5120) 103, 95, 133 against 83, 66, 69; 2^33.3 (4096 rows, 512 -> 5120) 168, 154, 171 against 130, 113, 115.  They
+# cross near 2^31; the line is above the copy task's stack (2^32.3 a layer), whose six layers in fp16 carry a difference in a
+# product's last bits on to 3e-3 of a gradient: at that size every program's results stay those of the library's products.
 MIN_WORK = 1 << 33
 
 # An input narrower than this has few stages to fill a tile's pipeline with before its results are stored: 16384 rows,
-# 128 -> 2560, 105 us against 118, where the gradients gain (83 and 139 against 83 and 85); at 256 columns 174 against 171.
-MIN_INFERENCE_WIDTH = 256
+# 64 -> 2560 would be two.  At 128 columns the library's 109 us stand against 97, at 208 -> 4160 357 against 244.
+MIN_INFERENCE_WIDTH = 128
 
 # Most rows and outputs: the kernel counts to the end of its last tile of 128 in 32 bits.
 MAX_ROWS = (1 << 31) - 1 - 128
