@@ -525,6 +525,18 @@ QSSM_API int qssm_gemm_f32_packed_plan(qssm_gemm_f32_call* call, uint64_t* bytes
 QSSM_API int qssm_gemm_f32_packed(const qssm_gemm_f32_call* call, void* packed, uint64_t bytes, void* stream);
 
 /*
+ * A weight gradient in one 16-bit storage type: c [M, N] = sum over k of a [K, M]^T b [K, N], row strides ldc, lda, ldb in
+ * elements; a: the outputs' gradient, b: the inputs, K: their rows.  fp32 accumulation, one rounding; results repeat bit for
+ * bit.  M and N are multiples of 8 and all rows 16-byte aligned; `partial` is fp32 scratch of
+ * qssm_weight_gradient_floats(M, N, K) floats, 16-byte aligned (none: 0 floats).
+ * This is what autograd records for the weights of the layer's projections (quick_ssm/layers.py:76-80,106).
+ */
+QSSM_API int qssm_weight_gradient(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int32_t M,
+                                  int32_t N, int32_t K, int32_t dtype, float* partial, uint64_t partial_floats, void* stream);
+QSSM_API uint64_t qssm_weight_gradient_floats(int32_t M, int32_t N, int32_t K);
+QSSM_API int qssm_weight_gradient_suits(int32_t M, int32_t N, int32_t K);   /* 1: faster than the library's product */
+
+/*
  * Streaming copy of `bytes` bytes (16-byte aligned, multiple of 16) on `stream`.  Not part of
  * the scan: it is the known-size kernel against which rocprof's FETCH_SIZE / WRITE_SIZE
  * counters and the achievable-bandwidth ceiling are calibrated by the benchmark.

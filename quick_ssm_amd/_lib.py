@@ -54,6 +54,9 @@ EXPORTED_SYMBOLS = (
     "qssm_gemm_f32_splits",
     "qssm_gemm_f32_packed_plan",
     "qssm_gemm_f32_packed",
+    "qssm_weight_gradient",
+    "qssm_weight_gradient_floats",
+    "qssm_weight_gradient_suits",
     "qssm_copy_bytes",
     "qssm_launch_count_step",
 )

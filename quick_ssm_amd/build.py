@@ -19,7 +19,8 @@ PKG_DIR = Path(__file__).resolve().parent
 SRC_DIR = PKG_DIR / "csrc"
 OBJ_DIR = SRC_DIR / "build"
 LIB_PATH = PKG_DIR / "libquick_ssm_hip.so"
-SOURCES = ("scan_fwd.hip", "scan_bwd.hip", "gates.hip", "rmsnorm.hip", "colsum.hip", "gemm_split.hip", "scan_api.hip")
+SOURCES = ("scan_fwd.hip", "scan_bwd.hip", "gates.hip", "rmsnorm.hip", "colsum.hip", "gemm_split.hip", "gemm_half.hip",
+           "scan_api.hip")
 
 NATIVE_SOURCE = "torch_scan.cpp"
 NATIVE_PATH = PKG_DIR / "_qssm_torch.so"

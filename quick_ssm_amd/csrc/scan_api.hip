@@ -1158,6 +1158,78 @@ int qssm_gemm_f32_packed(const qssm_gemm_f32_call* k, void* packed, uint64_t byt
   return e == hipSuccess ? 0 : hip_fail(e, "packed_gemm_kernel launch");
 }
 
+// How a weight gradient's tiles are dealt out: `whole` workgroups with a tile each, in full rounds of one workgroup per
+// compute unit, and the tiles after them in `splits` parts, so that the last round is full as well.
+static int64_t half_tiles(int64_t M, int64_t N) {
+  return ((M + kHalfTile - 1) / kHalfTile) * ((N + kHalfTile - 1) / kHalfTile);
+}
+static void half_deal(int64_t M, int64_t N, int64_t K, int64_t* whole, int* splits) {
+  // us of a stage of 64 k's, of a tile's start and end, of a part's way through memory and of the launch that sums them
+  const double kStage = 1.6, kRound = 9.0, kPart = 0.1, kReduce = 5.0;
+  const int64_t tiles = half_tiles(M, N), rest = tiles % kCUs;
+  const double stages = (double)((K + kHalfStageK - 1) / kHalfStageK);
+  double best = 0.0;
+  *splits = 1;
+  for (int s = 1; s <= 64 && (s == 1 || stages / s >= 4.0); ++s) {
+    double cost = (double)((rest * s + kCUs - 1) / kCUs) * (stages / s * kStage + kRound);
+    if (s > 1) cost += (double)(rest * s) * kPart + kReduce;
+    if (s == 1 || cost < best) { *splits = s; best = cost; }
+  }
+  *whole = *splits > 1 ? tiles - rest : tiles;
+}
+
+// us here against the library's product, bf16: 16384 rows 128 x 128 26 / 121, 256 x 1024 34 / 98, 640 x 128 29 / 111, 5120 x
+// 256 62 / 123, 5120 x 512 95 / 166, 1024 x 4096 131 / 174, 20480 x 1024 683 / 868; 8192 rows 128 x 128 22 / 63, 512 x 512
+// 28 / 53, 2560 x 512 44 / 65, 5120 x 1024 89 / 121; 4096 rows 256 x 1024 29 / 28, 2560 x 512 35 / 36, 10240 x 1024 100 / 88;
+// 2048 rows 1024 x 1024 28 / 20.  With few rows the library's shorter tiles fill the GPU without parts.  Where the last
+// round of tiles is neither full nor can be dealt out (10240 x 1024: 160 tiles) its product stays: 8192 rows 191 / 164.
+int qssm_weight_gradient_suits(int32_t M, int32_t N, int32_t K) {
+  if (M <= 0 || N <= 0 || K < 8192) return 0;
+  int64_t whole;
+  int splits;
+  half_deal(M, N, K, &whole, &splits);
+  const int64_t tiles = half_tiles(M, N), rest = tiles - whole;
+  const double rounds = (double)((whole + kCUs - 1) / kCUs) + (double)((rest * splits + kCUs - 1) / kCUs) / splits;
+  return tiles <= kCUs / 2 || (double)tiles >= 0.75 * kCUs * rounds;
+}
+
+uint64_t qssm_weight_gradient_floats(int32_t M, int32_t N, int32_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  int64_t whole;
+  int splits;
+  half_deal(M, N, K, &whole, &splits);
+  return (uint64_t)(half_tiles(M, N) - whole) * splits * kHalfTile * kHalfTile;
+}
+
+int qssm_weight_gradient(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int32_t M, int32_t N,
+                         int32_t K, int32_t dtype, float* partial, uint64_t partial_floats, void* stream) {
+  if (dtype != QSSM_F16 && dtype != QSSM_BF16) return fail(QSSM_EINVAL, "a 16-bit storage type is needed");
+  if (M < 0 || N < 0 || K < 1) return fail(QSSM_EINVAL, "bad dimension");
+  if (M == 0 || N == 0) return 0;
+  if (a == nullptr || b == nullptr || c == nullptr) return fail(QSSM_EINVAL, "NULL tensor");
+  if (lda < M || ldb < N || ldc < N) return fail(QSSM_EINVAL, "a leading dimension is below its row");
+  if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) % 16 != 0 || M % 8 != 0 || N % 8 != 0 || lda % 8 != 0 || ldb % 8 != 0 || ldc % 8 != 0)
+    return fail(QSSM_EALIGN, "operands and results need 16-byte aligned rows of a multiple of 8 columns");
+  if (lda >= (1 << 24) || ldb >= (1 << 24)) return fail(QSSM_EINVAL, "a leading dimension is too large for 32-bit tile offsets");
+  const int64_t tiles = half_tiles(M, N);
+  if (K > 0x7fffffff - kHalfStageK || tiles > 0x1fffffffll) return fail(QSSM_EINVAL, "product too large for one launch");
+  int64_t whole;
+  HalfGemmArgs p;
+  memset(&p, 0, sizeof(p));
+  half_deal(M, N, K, &whole, &p.splits);
+  const uint64_t floats = (uint64_t)(tiles - whole) * p.splits * kHalfTile * kHalfTile;
+  if (floats > 0 && p.splits > 1 && (partial == nullptr || partial_floats < floats || ((uintptr_t)partial) % 16 != 0))
+    return fail(QSSM_EWORKSPACE, "partial needs %llu floats, 16-byte aligned", (unsigned long long)floats);
+  p.a = a; p.b = b; p.c = c;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.M = M; p.N = N; p.K = K;
+  p.whole = (int)whole;
+  p.partial = partial;
+  launch_half_gemm(dtype, p, (hipStream_t)stream);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : hip_fail(e, "half_gemm_kernel launch");
+}
+
 int qssm_launch_count_step(uint32_t count, int32_t static_scratch, uint32_t* flag, uint32_t* next, int32_t* wipes) {
   if (flag == nullptr || next == nullptr || wipes == nullptr) return fail(QSSM_EINVAL, "NULL argument");
   const unsigned reset_at = static_scratch ? kScratchWipeAt : kCountWrapAt;

@@ -617,4 +617,19 @@ int64_t packed_gemm_stages(int64_t K, int64_t segments);
 uint64_t packed_bytes(int64_t N, int64_t K, int64_t many);
 void launch_packed_gemm(const PackedGemmArgs& args, bool a_kstrided, bool trans, hipStream_t stream);
 
+// ---- weight gradients in 16 bits (gemm_half.hip) -----------------------------------------------------------------
+constexpr int kHalfTile = 256, kHalfStageK = 64;
+
+struct HalfGemmArgs {
+  const void *a, *b;    // [K, M] and [K, N]
+  void* c;              // [M, N]
+  int64_t lda, ldb, ldc;
+  int M, N, K;
+  int whole;            // tiles that are one workgroup's each; the ones after them are dealt out
+  int splits;           // in this many parts of their k's
+  float* partial;       // [tiles dealt out][splits][tile]
+};
+
+void launch_half_gemm(int dtype, const HalfGemmArgs& args, hipStream_t stream);
+
 }  // namespace qssm

@@ -616,6 +616,47 @@ PyObject* py_split_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Rows of 16-byte pieces next to each other, in one of the storage types of qssm_weight_gradient.
+bool rows_of_16_bytes(const Tensor& t) {
+  return t.defined() && t.is_cuda() && t.dim() == 2 && t.size(0) > 0 && t.size(1) > 0 &&
+         t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.size(1) % 8 == 0 && t.stride(0) % 8 == 0 && t.stride(0) < (1 << 24) &&
+         t.size(0) < (1 << 30) && t.size(1) < (1 << 30) && (uintptr_t)t.const_data_ptr() % 16 == 0;
+}
+
+// (gradient of a linear map's outputs [rows, N], its inputs [rows, K]) -> the weight's gradient [N, K], or None where the
+// library's product is the faster one or this has no kernel for the operands.
+PyObject* py_weight_gradient(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  want_args(n, 2);
+  const Tensor &g = tensor_arg(args[0]), &u = tensor_arg(args[1]);
+  Tensor dw;
+  if (g.defined() && u.defined() && g.dim() == 2 && u.dim() == 2 && g.size(0) == u.size(0) && g.device() == u.device() &&
+      g.scalar_type() == u.scalar_type()) {
+    const c10::AutoGradMode no_grad(false);
+    const c10::OptionalDeviceGuard guard(g.device());
+    const at::ScalarType type = g.scalar_type();
+    const int64_t rows = g.size(0), N = g.size(1), K = u.size(1);
+    if (type == at::kFloat) {
+      if (rows > 0 && matrix_ok(g, rows, N, u) && matrix_ok(u, rows, K, g) && N % 4 == 0 && K % 4 == 0 && N > 0 && K > 0 &&
+          N < (1 << 30) && K < (1 << 30) && rows < (1 << 30)) {
+        dw = matrix(N, K, u);
+        product({g}, {u}, {dw}, rows, true, true);
+      }
+    } else if ((type == at::kHalf || type == at::kBFloat16) && rows_of_16_bytes(g) && rows_of_16_bytes(u) &&
+               qssm_weight_gradient_suits((int32_t)N, (int32_t)K, (int32_t)rows) != 0) {
+      dw = matrix(N, K, u);
+      const uint64_t floats = qssm_weight_gradient_floats((int32_t)N, (int32_t)K, (int32_t)rows);
+      Tensor partial;
+      if (floats > 0) partial = at::empty({(int64_t)floats}, u.options().dtype(at::kFloat).requires_grad(c10::nullopt));
+      check_rc(qssm_weight_gradient(g.const_data_ptr(), g.stride(0), u.const_data_ptr(), u.stride(0), dw.mutable_data_ptr(),
+                                    dw.stride(0), (int32_t)N, (int32_t)K, (int32_t)rows, type == at::kHalf ? QSSM_F16 : QSSM_BF16,
+                                    floats > 0 ? partial.mutable_data_ptr<float>() : nullptr, floats, stream_of(dw)));
+    }
+  }
+  return wrap_or_none(dw);
+  END_HANDLE_TH_ERRORS
+}
+
 PyObject* node_h_saved(PyObject* self, void*) {
   HANDLE_TH_ERRORS
   auto* node = static_cast<ScanBackward*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get());
@@ -653,6 +694,7 @@ PyObject* py_set_hooks(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef g_methods[] = {QSSM_METHOD("set_hooks", py_set_hooks), QSSM_METHOD("scan_forward", py_scan_forward),
                            QSSM_METHOD("scan_backward", py_scan_backward), QSSM_METHOD("attach_scan", py_attach_scan),
                            QSSM_METHOD("split_forward", py_split_forward), QSSM_METHOD("split_backward", py_split_backward),
+                           QSSM_METHOD("weight_gradient", py_weight_gradient),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_qssm_torch", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -19,6 +19,7 @@ import torch.nn as nn
 
 from . import _lib
 from . import gated_scan as _gated
+from . import hip_scan
 from . import scan_interface as _scan_interface
 from . import split_linear
 from .gates import gate_prologue, gate_prologue_wide
@@ -57,6 +58,27 @@ def column_sum(g2: torch.Tensor) -> torch.Tensor:
         _lib.check(_lib.load().qssm_colsum(g2.data_ptr(), g2.stride(0), rows, S, _CODES[g2.dtype], partial.data_ptr(),
                                            _COLSUM_PARTIAL_ROWS, out.data_ptr(), stream))
     return out
+
+
+# Rows, or multiply-adds in fp32, from which a weight gradient is this package's own product.  Its sums are as long as there
+# are rows, and the library gives a tile of it to one workgroup, most of the GPU idle.  16 bits: the measured line is at
+# qssm_weight_gradient_suits.  fp32, us for the library's product and the packed one (csrc/gemm_split.hip): 2^32.3 (4096 rows,
+# 5120 x 256) 120 and 68, (1024 rows, 5120 x 1024) 88 and 74, (512 rows, 10240 x 1024) 89 and 86; 2^32 (4096 rows, 1024 x 1024)
+# 63 and 67; with many rows earlier: 8192 rows, 256 x 1024 55 and 46, 128 x 128 45 and 36, 16384 rows, 128 x 512 99 and 47.
+# (No result of a step but the gradient itself depends on its last bits, as those of split_linear.MIN_WORK do.)
+_GRADIENT_ROWS, _GRADIENT_WORK = 8192, 1 << 32
+
+
+def _weight_gradient(g2: torch.Tensor, u2: torch.Tensor) -> torch.Tensor:
+    """The gradient of a linear map's weight from its outputs' gradient and its inputs ([rows, N], [rows, K])."""
+    rows, n = g2.shape
+    if ((rows >= _GRADIENT_ROWS or (g2.dtype is torch.float32 and rows * n * u2.shape[1] > _GRADIENT_WORK)) and g2.is_cuda
+            and not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or _scan_interface._followed_by_torch())):
+        native = hip_scan._native or hip_scan._load_native()
+        dw = native.weight_gradient(g2, u2)
+        if dw is not None:
+            return dw
+    return g2.t() @ u2
 
 
 def _products(ctx, u: torch.Tensor, weights, biases):
@@ -110,7 +132,7 @@ class _LinearBias(torch.autograd.Function):
             du, (dw,) = _product_gradients(ctx, [g2], u, [weight], need[0], need[1])
         else:
             du = (g2 @ weight).view_as(u) if need[0] else None
-            dw = g2.t() @ u.reshape(-1, u.shape[-1]) if need[1] else None
+            dw = _weight_gradient(g2, u.reshape(-1, u.shape[-1])) if need[1] else None
         db = column_sum(g2) if need[2] else None
         return du, dw, db
 
@@ -137,7 +159,7 @@ class _PackedProjection(torch.autograd.Function):
             du, (dw,) = _product_gradients(ctx, [g2], u, [wide_w], need[0], any(need[1:6]))
         else:
             du = (g2 @ wide_w).view_as(u) if need[0] else None
-            dw = g2.t() @ u.reshape(-1, u.shape[-1]) if any(need[1:6]) else None              # [5 S, H]
+            dw = _weight_gradient(g2, u.reshape(-1, u.shape[-1])) if any(need[1:6]) else None   # [5 S, H]
         if dw is not None:
             blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
         dbias = column_sum(g2[:, :S]) if need[6] else None
@@ -179,7 +201,7 @@ class _WideProjections(torch.autograd.Function):
         du = (g2 @ torch.cat(weights)).view_as(u) if need[0] else None
         blocks = [None] * 5
         if any(need[1:6]):
-            dw = g2.t() @ u.reshape(-1, u.shape[-1])                                  # [5 S, H]
+            dw = _weight_gradient(g2, u.reshape(-1, u.shape[-1]))                     # [5 S, H]
             blocks = [dw[k * S:(k + 1) * S] if need[1 + k] else None for k in range(5)]
         return (du, *blocks, _bias_gradient(g2[:, :S]) if need[6] else None)
 
