@@ -406,6 +406,44 @@ static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t 
       const int64_t seg = (int64_t)steps * (threads / g);
       if ((int64_t)B * strips < 32 && L >= 256 * seg) g >>= 1;
     }
+    // Rows of 256 bytes instead of 512 for launches that are not large enough for the wider pieces' higher rate to pay.  They
+    // come in tiles twice as long, i.e. with half the hand-overs along a chain, and fill a width that is no multiple of a
+    // 512-byte strip better.  `padded`: what the tiles cover, beyond the end of rows and sequences as well.  Measured with rows
+    // of 64 lanes against 32, forward and backward, 16-bit storage:
+    //   less padding     bf16 B=6 L=7480 D=384 48 -> 42 us and 95 -> 75, B=12 L=3000 D=192 28 -> 23 and 48 -> 37, B=3 L=6000
+    //                    D=640 37 -> 32 and 70 -> 55; rows that end anywhere only gain forward, and with much less of it
+    //                    (B=13 L=1125 D=361 28 -> 21 and 43 -> 45, B=7 L=3000 D=1100 66 -> 61, B=34 L=3335 D=152 57 -> 59 and
+    //                    100 -> 138)
+    //   a chain that takes 0.6 of the stream's time or more   fp16 B=2 L=8192 D=512 33 -> 23, bf16 B=1 L=4096 D=1280 39 -> 29
+    //                    backward, B=1 L=9000 D=2304 50 -> 44; at 0.57 bf16 B=2 L=4096 D=2048 34 -> 32 and 67 -> 67; below: B=8
+    //                    L=2048 D=1024 63 -> 63 backward, the headline shape 217 -> 227
+    // and fp32, where the strips are half as many columns and only less padding counts: B=1 L=20000 D=320 37 -> 33 and 70 ->
+    // 57, L=8192 D=1728 57 -> 55 and 106 -> 101; B=11 L=1024 D=3968 306 -> 318 without it.
+    const double hop_us = direction == QSSM_FORWARD ? 2.1 : 1.8;
+    const double stream_us = (double)B * L * D * (direction == QSSM_FORWARD ? 4 * es + os : 8 * es + os) / 5.7e6;
+    auto padded = [&](int gg) -> double {
+      const int64_t cols = (int64_t)gg * vec, seg = (int64_t)steps * (threads / gg);
+      return (double)((D + cols - 1) / cols * cols) * (double)((L + seg - 1) / seg * seg);
+    };
+    auto chain_us = [&](int gg) -> double {   // with clusters of eight
+      const int64_t seg = (int64_t)steps * (threads / gg);
+      return (double)((L + seg - 1) / seg) * hop_us / 8.0;
+    };
+    const bool whole_rows = (int64_t)D * es % 32 == 0;
+    if (!fixed_g && vec < 8 && g * vec * es == 512 && g > 1 && stream_us <= 110.0 && (direction == QSSM_BACKWARD || L >= 256)) {
+      const double ratio = padded(g / 2) / padded(g);
+      bool narrow;
+      if (!whole_rows) narrow = direction == QSSM_FORWARD && es == 2 && ratio <= 0.95;
+      else if (ratio <= 0.985) narrow = true;
+      else narrow = es == 2 && ratio <= 1.05 && stream_us <= 64.0 && chain_us(g) >= 0.6 * stream_us;
+      if (narrow) g >>= 1;
+    }
+    // And of 128 bytes where the chain would still set the pace of a backward: bf16 B=1 L=21625 D=256 51 -> 35 us, L=17098 42
+    // -> 32, L=16384 D=640 58 -> 56; forward they lose (L=16384 D=640 33 -> 37), and so do rows off 128-byte lines (L=10729
+    // D=880 59 -> 73).
+    if (!fixed_g && es == 2 && vec < 8 && direction == QSSM_BACKWARD && g * vec * es == 256 && g > 1 && (int64_t)D * es % 128 == 0 &&
+        chain_us(g) > 1.2 * stream_us)
+      g >>= 1;
     // Very short sequences: widen the rows instead of idling most time groups of a workgroup.
     if (!fixed_g)
       while (g < cap && g < threads && (int64_t)steps * (threads / g) / 2 >= lp2) g <<= 1;
