@@ -226,6 +226,17 @@ void launch(Call& k, const qssm_plan& plan, int index, Fn fn) {
   if (buf.status_to != nullptr) check_rc(qssm_control_status_async(buf.control, buf.status_to, stream));
 }
 
+// A call of the library that makes launches, with the other threads running beside it.
+template <typename Fn>
+void unlocked(Fn fn) {
+  int rc;
+  {
+    const Unlocked other_threads_may_run;
+    rc = fn();
+  }
+  check_rc(rc);
+}
+
 struct ForwardOut {
   Tensor y, h, ckpt;
   int64_t stride = 0;
@@ -414,8 +425,8 @@ void product(const std::vector<Tensor>& a, const std::vector<Tensor>& b, const s
     k.partial = partial.mutable_data_ptr<float>();
     k.partial_floats = (uint64_t)partial.numel();
   }
-  if (bytes == 0) check_rc(qssm_gemm_f32(&k, stream_of(c[0])));
-  else check_rc(qssm_gemm_f32_packed(&k, packed.mutable_data_ptr(), bytes, stream_of(c[0])));
+  void* const stream = stream_of(c[0]);
+  unlocked([&] { return bytes == 0 ? qssm_gemm_f32(&k, stream) : qssm_gemm_f32_packed(&k, packed.mutable_data_ptr(), bytes, stream); });
 }
 
 bool matrix_ok(const Tensor& t, int64_t rows, int64_t cols, const Tensor& like) {
@@ -648,12 +659,216 @@ PyObject* py_weight_gradient(PyObject*, PyObject* const* args, Py_ssize_t n) {
       const uint64_t floats = qssm_weight_gradient_floats((int32_t)N, (int32_t)K, (int32_t)rows);
       Tensor partial;
       if (floats > 0) partial = at::empty({(int64_t)floats}, u.options().dtype(at::kFloat).requires_grad(c10::nullopt));
-      check_rc(qssm_weight_gradient(g.const_data_ptr(), g.stride(0), u.const_data_ptr(), u.stride(0), dw.mutable_data_ptr(),
+      unlocked([&] {
+        return qssm_weight_gradient(g.const_data_ptr(), g.stride(0), u.const_data_ptr(), u.stride(0), dw.mutable_data_ptr(),
                                     dw.stride(0), (int32_t)N, (int32_t)K, (int32_t)rows, type == at::kHalf ? QSSM_F16 : QSSM_BF16,
-                                    floats > 0 ? partial.mutable_data_ptr<float>() : nullptr, floats, stream_of(dw)));
+                                    floats > 0 ? partial.mutable_data_ptr<float>() : nullptr, floats, stream_of(dw));
+      });
     }
   }
   return wrap_or_none(dw);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- the layer's other launches ------------------------------------------------------------------------------------
+//
+// Called inside the layer's autograd functions, which stay in Python; here are the outputs, the scratch and the arguments of
+// their launches.  Through ctypes a layer's forward and backward spent about 110 us of the interpreter's time on these.
+
+// Five tensors, or the five column blocks of one.
+struct FiveBlocks {
+  std::vector<Tensor> t;
+  const char* p[5];
+  qssm_strides s[5];
+};
+
+FiveBlocks blocks_arg(PyObject* o, bool written) {
+  FiveBlocks b;
+  if (THPVariable_Check(o)) {
+    const Tensor& wide = THPVariable_Unpack(o);
+    TORCH_CHECK_VALUE(wide.dim() == 3 && wide.size(2) % 5 == 0, "expected a [B, L, 5 S] tensor");
+    b.t.push_back(wide);
+    const int64_t step = wide.size(2) / 5 * wide.element_size();
+    for (int k = 0; k < 5; ++k) {
+      b.p[k] = (const char*)(written ? wide.mutable_data_ptr() : wide.const_data_ptr()) + k * step;
+      b.s[k] = {wide.stride(0), wide.stride(1)};
+    }
+    return b;
+  }
+  b.t = tensors_arg(o);
+  TORCH_CHECK_VALUE(b.t.size() == 5, "expected five tensors");
+  for (int k = 0; k < 5; ++k) {
+    TORCH_CHECK_VALUE(b.t[k].defined() && b.t[k].dim() == 3, "expected five tensors [B, L, S]");
+    b.p[k] = (const char*)(written ? b.t[k].mutable_data_ptr() : b.t[k].const_data_ptr());
+    b.s[k] = {b.t[k].stride(0), b.t[k].stride(1)};
+  }
+  return b;
+}
+
+qssm_strides strides3(const Tensor& t) {
+  TORCH_CHECK_VALUE(t.defined() && t.dim() == 3, "expected a tensor [B, L, S]");
+  return {t.stride(0), t.stride(1)};
+}
+
+// What gated_scan._launch hands on behind a launch's own arguments: control block, workspace, epoch and stream.
+struct Taken {
+  void* control;
+  uint64_t control_size;
+  void* workspace;
+  uint64_t workspace_size;
+  uint32_t epoch;
+  void* stream;
+  explicit Taken(PyObject* const* a) {
+    unsigned long long v[6];
+    for (int k = 0; k < 6; ++k) {
+      v[k] = PyLong_AsUnsignedLongLong(a[k]);
+      if (v[k] == (unsigned long long)-1 && PyErr_Occurred() != nullptr) throw python_error();
+    }
+    control = (void*)(uintptr_t)v[0];
+    control_size = v[1];
+    workspace = (void*)(uintptr_t)v[2];
+    workspace_size = v[3];
+    epoch = (uint32_t)v[4];
+    stream = (void*)(uintptr_t)v[5];
+  }
+};
+
+const qssm_plan* plan_arg(PyObject* o) {
+  const unsigned long long v = PyLong_AsUnsignedLongLong(o);
+  if (v == (unsigned long long)-1 && PyErr_Occurred() != nullptr) throw python_error();
+  return (const qssm_plan*)(uintptr_t)v;
+}
+
+// (unused, plan's address, projection outputs: five or one wide, y, ckpt, control ...) -> return code
+PyObject* py_gated_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  want_args(n, 11);
+  const qssm_plan* plan = plan_arg(args[1]);
+  const FiveBlocks pre = blocks_arg(args[2], false);
+  const Tensor &y = tensor_arg(args[3]), &ckpt = tensor_arg(args[4]);
+  const Taken to(args + 5);
+  const qssm_strides sy = strides3(y);
+  void* yp = y.mutable_data_ptr();
+  float* cp = ckpt.mutable_data_ptr<float>();
+  int rc;
+  {
+    const Unlocked other_threads_may_run;
+    rc = qssm_scan_gated_forward(plan, pre.p[0], pre.s[0], pre.p[1], pre.s[1], pre.p[2], pre.s[2], pre.p[3], pre.s[3], pre.p[4],
+                                 pre.s[4], yp, sy, cp, to.control, to.control_size, to.workspace, to.workspace_size, to.epoch,
+                                 to.stream);
+  }
+  return PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+// (unused, plan's address, projection outputs, dy, ckpt, gradients: five or one wide, control ...) -> return code
+PyObject* py_gated_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  want_args(n, 12);
+  const qssm_plan* plan = plan_arg(args[1]);
+  const FiveBlocks pre = blocks_arg(args[2], false), grad = blocks_arg(args[5], true);
+  const Tensor &dy = tensor_arg(args[3]), &ckpt = tensor_arg(args[4]);
+  const Taken to(args + 6);
+  const qssm_strides sdy = strides3(dy);
+  const void* dyp = dy.const_data_ptr();
+  const float* cp = ckpt.const_data_ptr<float>();
+  void* g[5];
+  for (int k = 0; k < 5; ++k) g[k] = const_cast<char*>(grad.p[k]);
+  int rc;
+  {
+    const Unlocked other_threads_may_run;
+    rc = qssm_scan_gated_backward(plan, pre.p[0], pre.s[0], pre.p[1], pre.s[1], pre.p[2], pre.s[2], pre.p[3], pre.s[3], pre.p[4],
+                                  pre.s[4], dyp, sdy, cp, g[0], grad.s[0], g[1], grad.s[1], g[2], grad.s[2], g[3], grad.s[3],
+                                  g[4], grad.s[4], to.control, to.control_size, to.workspace, to.workspace_size, to.epoch,
+                                  to.stream);
+  }
+  return PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+Tensor like_of(std::initializer_list<int64_t> sizes, const Tensor& like, at::ScalarType type) {
+  return at::empty(at::IntArrayRef(sizes), like.options().dtype(type).memory_format(c10::nullopt).requires_grad(c10::nullopt));
+}
+
+int64_t row_stride(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : t.size(1); }
+
+// (x [rows, H], weight, eps) -> (y, rstd)
+PyObject* py_rmsnorm_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  want_args(n, 3);
+  const Tensor &x = tensor_arg(args[0]), &w = tensor_arg(args[1]);
+  const double eps = PyFloat_AsDouble(args[2]);
+  if (eps == -1.0 && PyErr_Occurred() != nullptr) throw python_error();
+  TORCH_CHECK_VALUE(x.defined() && w.defined() && x.dim() == 2, "expected a [rows, H] matrix and its weight");
+  Tensor y, rstd;
+  {
+    const c10::AutoGradMode no_grad(false);
+    const c10::OptionalDeviceGuard guard(x.device());
+    const int64_t rows = x.size(0), H = x.size(1);
+    TORCH_CHECK_VALUE(H <= INT32_MAX, "a row does not fit 32 bits");
+    y = like_of({rows, H}, x, x.scalar_type());
+    rstd = like_of({rows}, x, at::kFloat);
+    const int type = code_of(x.scalar_type());
+    unlocked([&] {
+      return qssm_rmsnorm_forward(x.const_data_ptr(), row_stride(x), w.const_data_ptr(), y.mutable_data_ptr(),
+                                  rstd.mutable_data_ptr<float>(), rows, (int32_t)H, (float)eps, type, stream_of(x));
+    });
+  }
+  return Py_BuildValue("(NN)", THPVariable_Wrap(y), THPVariable_Wrap(rstd));
+  END_HANDLE_TH_ERRORS
+}
+
+// (dy [rows, H], x [rows, H], weight, rstd, eps, rows of scratch) -> (dx, dweight)
+PyObject* py_rmsnorm_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  want_args(n, 6);
+  const Tensor &dy = tensor_arg(args[0]), &x = tensor_arg(args[1]), &w = tensor_arg(args[2]), &rstd = tensor_arg(args[3]);
+  const double eps = PyFloat_AsDouble(args[4]);
+  if (eps == -1.0 && PyErr_Occurred() != nullptr) throw python_error();
+  const int64_t scratch = int_arg(args[5]);
+  TORCH_CHECK_VALUE(dy.defined() && x.defined() && w.defined() && rstd.defined() && x.dim() == 2 && dy.sizes() == x.sizes(),
+                    "expected two [rows, H] matrices, the weight and what the forward saved");
+  Tensor dx, dw;
+  {
+    const c10::AutoGradMode no_grad(false);
+    const c10::OptionalDeviceGuard guard(x.device());
+    const int64_t rows = x.size(0), H = x.size(1);
+    TORCH_CHECK_VALUE(H <= INT32_MAX && scratch <= INT32_MAX, "a row does not fit 32 bits");
+    dx = like_of({rows, H}, x, x.scalar_type());
+    dw = like_of({H}, x, w.scalar_type());
+    const Tensor partial = like_of({scratch, H}, x, at::kFloat);
+    const int type = code_of(x.scalar_type());
+    unlocked([&] {
+      return qssm_rmsnorm_backward(dy.const_data_ptr(), row_stride(dy), x.const_data_ptr(), row_stride(x), w.const_data_ptr(),
+                                   rstd.const_data_ptr<float>(), dx.mutable_data_ptr(), dw.mutable_data_ptr(),
+                                   partial.mutable_data_ptr<float>(), (int32_t)scratch, rows, (int32_t)H, (float)eps, type,
+                                   stream_of(x));
+    });
+  }
+  return Py_BuildValue("(NN)", THPVariable_Wrap(dx), THPVariable_Wrap(dw));
+  END_HANDLE_TH_ERRORS
+}
+
+// ([rows, S] matrix, rows of scratch) -> its column sums
+PyObject* py_column_sum(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  want_args(n, 2);
+  const Tensor& g = tensor_arg(args[0]);
+  const int64_t scratch = int_arg(args[1]);
+  TORCH_CHECK_VALUE(g.defined() && g.dim() == 2 && g.size(1) <= INT32_MAX && scratch <= INT32_MAX, "expected a [rows, S] matrix");
+  Tensor out;
+  {
+    const c10::AutoGradMode no_grad(false);
+    const c10::OptionalDeviceGuard guard(g.device());
+    out = like_of({g.size(1)}, g, g.scalar_type());
+    const Tensor partial = like_of({scratch, g.size(1)}, g, at::kFloat);
+    const int type = code_of(g.scalar_type());
+    unlocked([&] {
+      return qssm_colsum(g.const_data_ptr(), g.stride(0), g.size(0), (int32_t)g.size(1), type, partial.mutable_data_ptr<float>(),
+                         (int32_t)scratch, out.mutable_data_ptr(), stream_of(g));
+    });
+  }
+  return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -694,7 +909,9 @@ PyObject* py_set_hooks(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef g_methods[] = {QSSM_METHOD("set_hooks", py_set_hooks), QSSM_METHOD("scan_forward", py_scan_forward),
                            QSSM_METHOD("scan_backward", py_scan_backward), QSSM_METHOD("attach_scan", py_attach_scan),
                            QSSM_METHOD("split_forward", py_split_forward), QSSM_METHOD("split_backward", py_split_backward),
-                           QSSM_METHOD("weight_gradient", py_weight_gradient),
+                           QSSM_METHOD("weight_gradient", py_weight_gradient), QSSM_METHOD("gated_forward", py_gated_forward),
+                           QSSM_METHOD("gated_backward", py_gated_backward), QSSM_METHOD("rmsnorm_forward", py_rmsnorm_forward),
+                           QSSM_METHOD("rmsnorm_backward", py_rmsnorm_backward), QSSM_METHOD("column_sum", py_column_sum),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_qssm_torch", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

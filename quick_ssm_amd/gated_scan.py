@@ -18,12 +18,12 @@ call qualifies, and the layer takes the two-pass route (quick_ssm_amd/gates.py +
 from __future__ import annotations
 
 import ctypes
-from typing import Optional, Sequence, Tuple
+from typing import Optional, Sequence, Tuple, Union
 
 import torch
 
 from . import _lib, hip_scan
-from ._lib import Plan, Strides
+from ._lib import Plan
 from .gates import gate_prologue, gate_prologue_wide
 
 Tensor = torch.Tensor
@@ -32,18 +32,30 @@ _CODES = {torch.float32: _lib.QSSM_F32, torch.float16: _lib.QSSM_F16, torch.bflo
 _plans: dict = {}
 
 
+def _built(t: Tensor, compute_dtype: torch.dtype, out_dtype: torch.dtype, checkpoint: bool) -> bool:
+    if t.device.type != "cuda" or not checkpoint:
+        return False
+    if t.dtype in (torch.float16, torch.bfloat16):
+        return compute_dtype == t.dtype and out_dtype in (t.dtype, torch.float32)
+    return t.dtype == torch.float32 and compute_dtype in _CODES and out_dtype == torch.float32
+
+
+def supported_wide(wide: Tensor, compute_dtype: torch.dtype, out_dtype: torch.dtype, checkpoint: bool = True) -> bool:
+    """`supported` for the five column blocks of one [B, L, 5 S] tensor, without cutting it up."""
+    if wide.dim() != 3 or not _built(wide, compute_dtype, out_dtype, checkpoint):
+        return False
+    B, L, W = wide.shape
+    es = wide.element_size()
+    sb, sl, one = wide.stride()
+    # (every block starts where 16 bytes do: the first one, and S elements are a multiple of that)
+    return (B > 0 and L > 0 and W >= 640 and W % 20 == 0 and one == 1 and wide.data_ptr() % 16 == 0 and (W // 5 * es) % 16 == 0
+            and (sb * es) % 16 == 0 and (sl * es) % 16 == 0)
+
+
 def supported(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype: torch.dtype, checkpoint: bool = True) -> bool:
     """Whether the five projection outputs can take the gated launches."""
     t0 = pre[0]
-    if t0.device.type != "cuda" or t0.dim() != 3 or not checkpoint:
-        return False
-    if t0.dtype in (torch.float16, torch.bfloat16):
-        if compute_dtype != t0.dtype or out_dtype not in (t0.dtype, torch.float32):
-            return False
-    elif t0.dtype == torch.float32:
-        if compute_dtype not in _CODES or out_dtype != torch.float32:
-            return False
-    else:
+    if t0.dim() != 3 or not _built(t0, compute_dtype, out_dtype, checkpoint):
         return False
     B, L, S = t0.shape
     if B == 0 or L == 0 or S < 128 or S % 4 != 0:
@@ -76,10 +88,6 @@ def _plan(B: int, L: int, S: int, dtype: torch.dtype, compute_dtype: torch.dtype
     return plan
 
 
-def _st(t: Tensor) -> Strides:
-    return Strides(t.stride(0), t.stride(1))
-
-
 def _launch(plan: Plan, dev: torch.device, fn, *args) -> None:
     with _lib.launch_stream(dev) as stream:
         taken, epoch, capturing = hip_scan._launch_buffers(dev, dev.index, stream, plan.control_bytes, plan.workspace_bytes)
@@ -87,21 +95,29 @@ def _launch(plan: Plan, dev: torch.device, fn, *args) -> None:
         hip_scan._after_launch(taken, stream, capturing)
 
 
-def _forward_launch(pre: Sequence[Tensor], compute_dtype: torch.dtype, out_dtype: torch.dtype, train: bool = True):
+# The projection outputs (and their gradients) of a launch: five tensors, or one whose column blocks they are.
+_Blocks = Union[Sequence[Tensor], Tensor]
+
+
+def _shape(pre: _Blocks) -> Tuple[int, int, int, Tensor]:
+    if isinstance(pre, Tensor):
+        return pre.shape[0], pre.shape[1], pre.shape[2] // 5, pre
+    return (*pre[0].shape, pre[0])
+
+
+def _forward_launch(pre: _Blocks, compute_dtype: torch.dtype, out_dtype: torch.dtype, train: bool = True):
     """y, the saved states and their spacing for the five projection outputs.  `train`: a backward will follow, so
     the last tiles of every chain may leave their operands in the caches for it (`hip_scan.set_forward_keep`)."""
-    A_pre, B_in, Ca, Cb, D_pre = pre
-    B, L, S = A_pre.shape
-    dev, dtype = A_pre.device, A_pre.dtype
+    B, L, S, t0 = _shape(pre)
+    dev, dtype = t0.device, t0.dtype
     # the backward's tile length decides how far apart the saved states are; it takes dy stored as the projections are
     stride = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, 0).seg_len
     plan = _plan(B, L, S, dtype, compute_dtype, out_dtype, _lib.QSSM_FORWARD, stride, True,
                  hip_scan._forward_keep if train else False)
     y = torch.empty((B, L, S), dtype=out_dtype, device=dev)
     ckpt = torch.empty((B, plan.n_ckpt, S), dtype=torch.float32, device=dev)
-    _launch(plan, dev, _lib.load().qssm_scan_gated_forward,
-            A_pre.data_ptr(), _st(A_pre), B_in.data_ptr(), _st(B_in), Ca.data_ptr(), _st(Ca), Cb.data_ptr(), _st(Cb),
-            D_pre.data_ptr(), _st(D_pre), y.data_ptr(), _st(y), ckpt.data_ptr())
+    native = hip_scan._native or hip_scan._load_native()
+    _launch(plan, dev, native.gated_forward, ctypes.addressof(plan), pre, y, ckpt)
     return y, ckpt, int(plan.ckpt_stride)
 
 
@@ -111,19 +127,14 @@ def _fits_fused_backward(grad_y: Tensor, dtype: torch.dtype) -> bool:
                 or (grad_y.stride(1) * es) % 16)
 
 
-def _backward_launch(pre: Sequence[Tensor], compute_dtype: torch.dtype, grad_y: Tensor, ckpt: Tensor, stride: int,
-                     grads: Sequence[Tensor]) -> None:
+def _backward_launch(pre: _Blocks, compute_dtype: torch.dtype, grad_y: Tensor, ckpt: Tensor, stride: int,
+                     grads: _Blocks) -> None:
     """The five projection gradients, written into `grads` (any batch and time strides)."""
-    A_pre, B_in, Ca, Cb, D_pre = pre
-    dA, dB, dCa, dCb, dD = grads
-    B, L, S = A_pre.shape
-    dtype = A_pre.dtype
+    B, L, S, t0 = _shape(pre)
+    dtype = t0.dtype
     plan = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, stride, True)
-    _launch(plan, A_pre.device, _lib.load().qssm_scan_gated_backward,
-            A_pre.data_ptr(), _st(A_pre), B_in.data_ptr(), _st(B_in), Ca.data_ptr(), _st(Ca), Cb.data_ptr(), _st(Cb),
-            D_pre.data_ptr(), _st(D_pre), grad_y.data_ptr(), _st(grad_y), ckpt.data_ptr(),
-            dA.data_ptr(), _st(dA), dB.data_ptr(), _st(dB), dCa.data_ptr(), _st(dCa), dCb.data_ptr(), _st(dCb),
-            dD.data_ptr(), _st(dD))
+    native = hip_scan._native or hip_scan._load_native()
+    _launch(plan, t0.device, native.gated_backward, ctypes.addressof(plan), pre, grad_y, ckpt, grads)
 
 
 class _GatedScanFunction(torch.autograd.Function):
@@ -153,18 +164,13 @@ class _GatedScanFunction(torch.autograd.Function):
         return (*grads, None, None)
 
 
-def _blocks(wide: Tensor) -> Tuple[Tensor, ...]:
-    S = wide.shape[-1] // 5
-    return tuple(wide[..., k * S:(k + 1) * S] for k in range(5))
-
-
 class _GatedScanWide(torch.autograd.Function):
     """The same on one wide [B, L, 5 S] tensor whose column blocks are the five projection outputs (one GEMM over the
     stacked weights): the gradients are written into the blocks of one wide gradient."""
 
     @staticmethod
     def forward(ctx, wide: Tensor, out_dtype: torch.dtype, compute_dtype: torch.dtype) -> Tensor:
-        y, ckpt, stride = _forward_launch(_blocks(wide), compute_dtype, out_dtype, ctx.needs_input_grad[0])
+        y, ckpt, stride = _forward_launch(wide, compute_dtype, out_dtype, ctx.needs_input_grad[0])
         ctx.save_for_backward(wide, ckpt)
         ctx.stride, ctx.out_dtype, ctx.compute_dtype = stride, out_dtype, compute_dtype
         return y
@@ -187,7 +193,7 @@ class _GatedScanWide(torch.autograd.Function):
                 (dwide,) = torch.autograd.grad((a, x, c, b), (leaf,), (da, dx, dc, db))
                 return dwide, None, None
         dwide = torch.empty_like(wide, memory_format=torch.contiguous_format)
-        _backward_launch(_blocks(wide), ctx.compute_dtype, grad_y, ckpt, ctx.stride, _blocks(dwide))
+        _backward_launch(wide, ctx.compute_dtype, grad_y, ckpt, ctx.stride, dwide)
         return dwide, None, None
 
 
@@ -223,4 +229,4 @@ def gated_scan_wide(wide: Tensor, *, out_dtype: Optional[torch.dtype] = None,
     return _GatedScanWide.apply(wide, out_dtype or wide.dtype, compute_dtype or wide.dtype)
 
 
-__all__ = ["gated_scan", "gated_scan_wide", "supported"]
+__all__ = ["gated_scan", "gated_scan_wide", "supported", "supported_wide"]

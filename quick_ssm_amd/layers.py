@@ -52,12 +52,7 @@ def column_sum(g2: torch.Tensor) -> torch.Tensor:
     rows, S = g2.shape
     if not (g2.is_cuda and g2.dtype in _CODES and S > 0 and rows > 0 and g2.stride(1) == 1 and g2.stride(0) >= S):
         return g2.sum(0)
-    out = torch.empty((S,), dtype=g2.dtype, device=g2.device)
-    partial = torch.empty((_COLSUM_PARTIAL_ROWS, S), dtype=torch.float32, device=g2.device)
-    with _lib.launch_stream(g2.device) as stream:
-        _lib.check(_lib.load().qssm_colsum(g2.data_ptr(), g2.stride(0), rows, S, _CODES[g2.dtype], partial.data_ptr(),
-                                           _COLSUM_PARTIAL_ROWS, out.data_ptr(), stream))
-    return out
+    return (hip_scan._native or hip_scan._load_native()).column_sum(g2, _COLSUM_PARTIAL_ROWS)
 
 
 # Rows, or multiply-adds in fp32, from which a weight gradient is this package's own product.  Its sums are as long as there
@@ -374,12 +369,9 @@ class SSM(nn.Module):
             wide = self._wide_projection(u)
             if wide is None:
                 wide, pre = self._large_projections(u)
-            if wide is not None:
-                S = self.state_size_dim
-                pre = tuple(wide[..., k * S:(k + 1) * S] for k in range(5))
-            if wide is not None and wide.dim() == 3 and _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
+            if wide is not None and _gated.supported_wide(wide, self.compute_dtype, out_dtype, checkpoint):
                 y = _gated.gated_scan_wide(wide, out_dtype=out_dtype, compute_dtype=self.compute_dtype)
-            elif _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
+            elif wide is None and _gated.supported(pre, self.compute_dtype, out_dtype, checkpoint):
                 y = _gated.gated_scan(*pre, out_dtype=out_dtype, compute_dtype=self.compute_dtype)
             else:
                 if wide is not None:

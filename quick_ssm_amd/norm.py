@@ -11,7 +11,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _lib
+from . import _lib, hip_scan
 
 Tensor = torch.Tensor
 
@@ -25,10 +25,6 @@ def _rows(t: Tensor, H: int) -> Tensor:
     return t2 if t2.stride(1) == 1 or t2.shape[0] == 0 else t2.contiguous()
 
 
-def _ld(t2: Tensor, H: int) -> int:
-    return t2.stride(0) if t2.shape[0] > 1 else H
-
-
 def rms_norm_reference(x: Tensor, weight: Tensor, eps: float) -> Tensor:
     """The reference's own order of operations (quick_ssm/layers.py:15-17)."""
     rms = torch.sqrt(x.pow(2).mean(dim=-1, keepdim=True) + eps)
@@ -40,14 +36,8 @@ class _RmsNorm(torch.autograd.Function):
     def forward(ctx, x: Tensor, weight: Tensor, eps: float):
         H = x.shape[-1]
         x2 = _rows(x, H)
-        rows = x2.shape[0]
         w = weight.contiguous()
-        y = torch.empty((rows, H), dtype=x.dtype, device=x.device)
-        rstd = torch.empty((rows,), dtype=torch.float32, device=x.device)
-        with _lib.launch_stream(x.device) as stream:
-            _lib.check(_lib.load().qssm_rmsnorm_forward(
-                x2.data_ptr(), _ld(x2, H), w.data_ptr(), y.data_ptr(), rstd.data_ptr(), rows, H, float(eps),
-                _CODES[x.dtype], stream))
+        y, rstd = (hip_scan._native or hip_scan._load_native()).rmsnorm_forward(x2, w, float(eps))
         ctx.save_for_backward(x2, w, rstd)
         ctx.shape, ctx.eps = x.shape, float(eps)
         return y.view(x.shape)
@@ -56,20 +46,13 @@ class _RmsNorm(torch.autograd.Function):
     def backward(ctx, dy: Tensor):
         x2, w, rstd = ctx.saved_tensors
         rows, H = x2.shape
-        dev = x2.device
         g = dy.reshape(rows, H)
         if g.dtype != x2.dtype:
             g = g.to(x2.dtype)
         if rows > 0 and g.stride(1) != 1:
             g = g.contiguous()
-        dx = torch.empty((rows, H), dtype=x2.dtype, device=dev)
-        dw = torch.empty((H,), dtype=w.dtype, device=dev)
         n_part = max(_lib.QSSM_RMSNORM_MIN_PARTIAL_ROWS, min(PARTIAL_ROWS, (rows + 7) // 8))
-        partial = torch.empty((n_part, H), dtype=torch.float32, device=dev)
-        with _lib.launch_stream(dev) as stream:
-            _lib.check(_lib.load().qssm_rmsnorm_backward(
-                g.data_ptr(), _ld(g, H), x2.data_ptr(), _ld(x2, H), w.data_ptr(), rstd.data_ptr(), dx.data_ptr(),
-                dw.data_ptr(), partial.data_ptr(), n_part, rows, H, ctx.eps, _CODES[x2.dtype], stream))
+        dx, dw = (hip_scan._native or hip_scan._load_native()).rmsnorm_backward(g, x2, w, rstd, ctx.eps, n_part)
         return dx.view(ctx.shape), dw, None
 
 

@@ -114,3 +114,25 @@ def test_what_the_node_cannot_do_is_refused(gpu):
         with pytest.raises(RuntimeError):
             torch.func.vmap(fn)(torch.stack([x, x]))
         assert torch.isfinite(fn(x)).all()
+
+
+@pytest.mark.parametrize("dtype,compute", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float16)], ids=str)
+def test_a_wide_tensor_and_its_five_blocks_are_the_same_launch(gpu, dtype, compute):
+    from quick_ssm_amd import gated_scan
+
+    gen = torch.Generator(device=gpu).manual_seed(1)
+    wide = torch.empty(2, 70, 5 * 136, device=gpu).normal_(generator=gen).to(dtype).requires_grad_(True)
+    dy = torch.empty(2, 70, 136, device=gpu).normal_(generator=gen).to(dtype)
+    blocks = [t.detach().contiguous().requires_grad_(True) for t in wide.split(136, 2)]
+    assert gated_scan.supported_wide(wide, compute, dtype) and gated_scan.supported(blocks, compute, dtype)
+    got = gated_scan.gated_scan_wide(wide, compute_dtype=compute)
+    want = gated_scan.gated_scan(*blocks, compute_dtype=compute)
+    assert torch.equal(got, want)
+    (dwide,) = torch.autograd.grad(got, wide, dy)
+    for a, b in zip(dwide.split(136, 2), torch.autograd.grad(want, blocks, dy)):
+        assert torch.equal(a, b)
+    # the two rules agree, block by block, on widths and rows that 16 bytes do not divide
+    for width, at in ((128, 0), (132, 0), (136, 4), (136, 8), (124, 0)):
+        odd = torch.empty(2, 5, 5 * width + 16, device=gpu, dtype=dtype)[..., at:at + 5 * width]
+        five = [odd[..., k * width:(k + 1) * width] for k in range(5)]
+        assert gated_scan.supported_wide(odd, compute, dtype) == gated_scan.supported(five, compute, dtype), (width, at)
