@@ -62,6 +62,8 @@ __global__ void __launch_bounds__(256) colsum_final_kernel(const float* __restri
   float sum = 0.0f;
   if (col < S) {
     const int lo = grp * per, hi = n < lo + per ? n : lo + per;
+    // eight rows in flight, added in order (one at a time: 5.4 us for 64 rows of 256 columns)
+#pragma unroll 8
     for (int i = lo; i < hi; ++i) sum += partial[(int64_t)i * S + col];
   }
   part[grp][cl] = sum;

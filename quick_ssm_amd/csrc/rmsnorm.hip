@@ -273,6 +273,8 @@ __global__ void __launch_bounds__(1024) rmsnorm_dw_kernel(const float* partial, 
   float sum = 0.0f;
   if (col < H) {
     const int lo = grp * per, hi = min(n, lo + per);
+    // eight rows in flight: one at a time, the launch was a chain of 32 round trips (512 rows, H = 256 9.3 us)
+#pragma unroll 8
     for (int i = lo; i < hi; ++i) sum += partial[(int64_t)i * H + col];
   }
   part[grp][cl] = sum;
