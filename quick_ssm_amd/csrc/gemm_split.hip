@@ -354,7 +354,7 @@ __device__ __forceinline__ void split8(const float* v, Parts& t) {
 
 // The parts of a matrix in the order the product's tiles take them: [tile of 256 rows][run][stage of 32 k's][part][16 rows]
 // in pieces of kFrag, zeros past the ends.  One workgroup per tile and stage: 4 bytes read and 6 written per element, once,
-// where the tiles of the other operand would each convert it again (20480 x 1024 weights: 47 us before a product of 6.1 ms).
+// where the tiles of the other operand would each convert it again (20480 x 1024 weights: 39 us before a product of 6.1 ms).
 template <bool KSTRIDED>
 __global__ void __launch_bounds__(256) pack_parts_kernel(const PackArgs p) {
   const int stages = p.segments * p.stages_per;
@@ -488,6 +488,8 @@ __global__ void __launch_bounds__(512, 2) packed_gemm_kernel(const PackedGemmArg
           v[i] = 0.0f;
           if (aoct * 8 + i < left) v[i] = *(const __attribute__((address_space(1))) float*)(base + (AKS ? (int64_t)i * p.lda * 4 : i * 4) + aoff);
         }
+        // (how many loads that were depends on the lanes, and the waits below count: none is left open here)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
     };
     int next = s_begin;   // the stage the next load takes; after the last one it is taken again, and never used

@@ -2,7 +2,8 @@
 
 Same constructor arguments, parameter names (so state dicts interchange) and forward keywords as
 the reference's quick_ssm/layers.py:9-107.  The projections are torch GEMMs, except over fp32
-parameters, where they are split products on the bf16 matrix cores (quick_ssm_amd/split_linear.py); the gate
+parameters, where they are split products on the bf16 matrix cores (quick_ssm_amd/split_linear.py), and
+except weight gradients over many rows (`_weight_gradient`); the gate
 activations and casts between them and the scan happen inside the scan's own launches when the
 projections are stored as the 16-bit compute dtype (quick_ssm_amd/gated_scan.py) and are one fused HIP
 pass otherwise (quick_ssm_amd/gates.py),
