@@ -210,7 +210,7 @@ static int backward_launch(const qssm_plan* plan, const void* x, qssm_strides sx
                            void* stream, const GateExtras* gate = nullptr);
 
 static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
-                     int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan);
+                     int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan, bool gated = false);
 
 static int plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32_t compute_dtype, int32_t out_dtype,
                            int32_t direction, int32_t align_elems, int32_t ckpt_stride, int most, qssm_plan* plan);
@@ -269,10 +269,11 @@ static int plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32
   if (D % 4 != 0 || (align_elems * es) % 16 != 0 || D < 128)
     return fail(QSSM_EALIGN, "the gated scan needs D >= 128, a multiple of 4, and 16-byte aligned rows");
   const int32_t kGatedTune = (8 << 8) | (vec << 16) | (1 << 24);
-  // The row width comes from a plan without a given spacing of saved states, so that the forward (which is handed
-  // the backward's tile length as that spacing) and the backward (which is handed it back) agree on it; the gated
-  // kernels exist for rows of 32 and 64 lanes.
-  int rc = qssm_plan_scan_tuned(B, L, D, dtype, out_dtype, direction, align_elems, 0, kGatedTune, plan);
+  // The row width of either direction comes from its plan without a given spacing of saved states, so that a backward
+  // planned for the spacing and the one that saves of it are the same launch.  The two directions need not agree: a forward
+  // of narrower rows has tiles of twice the backward's length and saves two states in each, and one that is handed a
+  // spacing longer than its tiles takes the narrower rows (plan_scan).  The kernels exist for rows of 32 and 64 lanes.
+  int rc = plan_scan(B, L, D, dtype, out_dtype, direction, align_elems, 0, kGatedTune, false, plan, true);
   if (rc != 0) return rc;
   if (B == 0 || L == 0) {
     rc = qssm_plan_scan_tuned(B, L, D, dtype, out_dtype, direction, align_elems, ckpt_stride, kGatedTune, plan);
@@ -295,7 +296,7 @@ static int plan_scan_gated(int32_t B, int32_t L, int32_t D, int32_t dtype, int32
 }
 
 static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t out_dtype, int32_t direction,
-                     int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan) {
+                     int32_t align_elems, int32_t ckpt_stride, int32_t tune, bool loose, qssm_plan* plan, bool gated) {
   if (plan == nullptr) return fail(QSSM_EINVAL, "plan is NULL");
   if (B < 0 || L < 0 || D < 0) return fail(QSSM_EINVAL, "negative dimension");
   if (direction != QSSM_FORWARD && direction != QSSM_BACKWARD) return fail(QSSM_EINVAL, "bad direction");
@@ -374,6 +375,9 @@ static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t 
   if (fixed_t) threads = 256 << (tune_t - 1);
   if (vec == 1 && threads != 256) threads = 256;
   if (g > threads) g = threads;
+  // us of one hand-over along a chain, and of the operands' way through memory by itself
+  const double hop_us = direction == QSSM_FORWARD ? 2.1 : 1.8;
+  const double stream_us = (double)B * L * D * (direction == QSSM_FORWARD ? 4 * es + os : 8 * es + os) / 5.6e6;
   auto tiles = [&](int gg, int tt) -> int64_t {
     const int64_t strips = (D + (int64_t)gg * vec - 1) / ((int64_t)gg * vec);
     const int64_t seg = (int64_t)steps * (tt / gg);
@@ -411,16 +415,23 @@ static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t 
     // 512-byte strip better.  `padded`: what the tiles cover, beyond the end of rows and sequences as well.  Measured with rows
     // of 64 lanes against 32, forward and backward, 16-bit storage:
     //   less padding     bf16 B=6 L=7480 D=384 48 -> 42 us and 95 -> 75, B=12 L=3000 D=192 28 -> 23 and 48 -> 37, B=3 L=6000
-    //                    D=640 37 -> 32 and 70 -> 55; rows that end anywhere only gain forward, and with much less of it
-    //                    (B=13 L=1125 D=361 28 -> 21 and 43 -> 45, B=7 L=3000 D=1100 66 -> 61, B=34 L=3335 D=152 57 -> 59 and
-    //                    100 -> 138)
+    //                    D=640 37 -> 32 and 70 -> 55
     //   a chain that takes 0.6 of the stream's time or more   fp16 B=2 L=8192 D=512 33 -> 23, bf16 B=1 L=4096 D=1280 39 -> 29
-    //                    backward, B=1 L=9000 D=2304 50 -> 44; at 0.57 bf16 B=2 L=4096 D=2048 34 -> 32 and 67 -> 67; below: B=8
-    //                    L=2048 D=1024 63 -> 63 backward, the headline shape 217 -> 227
-    // and fp32, where the strips are half as many columns and only less padding counts: B=1 L=20000 D=320 37 -> 33 and 70 ->
-    // 57, L=8192 D=1728 57 -> 55 and 106 -> 101; B=11 L=1024 D=3968 306 -> 318 without it.
-    const double hop_us = direction == QSSM_FORWARD ? 2.1 : 1.8;
-    const double stream_us = (double)B * L * D * (direction == QSSM_FORWARD ? 4 * es + os : 8 * es + os) / 5.7e6;
+    //                    backward, B=1 L=9000 D=2304 50 -> 44; at 0.57 only the forward gains (B=2
+    //                    L=4096 D=2048 34 -> 32 and 67 -> 67), far below neither (B=8 L=2048 D=1024 63 -> 63 backward, the
+    //                    headline shape 217 -> 227)
+    // and fp32, where the strips are half as many columns and only less padding counts, beside a chain of 0.4 of the stream:
+    // B=1 L=20000 D=320 37 -> 33 and 70 -> 57, L=8192 D=1728 57 -> 55 and 106 -> 101; B=11 L=1024 D=3968 306 -> 318 without
+    // less padding, B=5 L=418 D=928 17 -> 19 backward with a chain of 0.2.
+    // All that holds for rows that start on 128-byte lines.  Elsewhere both ends of every row piece share their lines with
+    // the neighbours, which half the width doubles, and only a chain longer than the stream pays for it: fp32 B=4 L=1019
+    // D=1976 69 -> 91 backward, bf16 B=19 L=638 D=1616 92 -> 109, fp16 B=4 L=7540 D=1384 89 -> 99 forward; with such a chain
+    // bf16 B=13 L=1125 D=361 28 -> 21 forward.  fp32 rows off half a line lose some even then (backward 0.89 to 1.2 times
+    // the speed), and so does the backward of rows that end anywhere (B=13 L=1125 D=361 43 -> 45).
+    // 1150 launches of drawn shapes that this narrows: 1.15 times the speed in the mean, 14 of them slower by 3 to 8 %.
+    // Gated launches move a fifth more than `stream_us` says, and their forward's chains weigh more: off 128-byte lines it
+    // gains with a chain as long as the stream, of any storage; their backward stays as it is (B=1 L=4852 S=1840 65 -> 73).
+    // 420 of them that this narrows: 1.23 times the speed in the mean, none slower by more than 3 %.
     auto padded = [&](int gg) -> double {
       const int64_t cols = (int64_t)gg * vec, seg = (int64_t)steps * (threads / gg);
       return (double)((D + cols - 1) / cols * cols) * (double)((L + seg - 1) / seg * seg);
@@ -429,19 +440,22 @@ static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t 
       const int64_t seg = (int64_t)steps * (threads / gg);
       return (double)((L + seg - 1) / seg) * hop_us / 8.0;
     };
-    const bool whole_rows = (int64_t)D * es % 32 == 0;
+    const int64_t row_bytes = (int64_t)D * es;
     if (!fixed_g && vec < 8 && g * vec * es == 512 && g > 1 && stream_us <= 110.0 && (direction == QSSM_BACKWARD || L >= 256)) {
-      const double ratio = padded(g / 2) / padded(g);
+      const double ratio = padded(g / 2) / padded(g), chain = chain_us(g) / stream_us;
+      const bool less = ratio <= (row_bytes % 32 == 0 ? 0.985 : 0.95);
+      const bool held_up = es == 2 && row_bytes % 32 == 0 && ratio <= 1.05 && stream_us <= 64.0 && chain >= 0.6;
       bool narrow;
-      if (!whole_rows) narrow = direction == QSSM_FORWARD && es == 2 && ratio <= 0.95;
-      else if (ratio <= 0.985) narrow = true;
-      else narrow = es == 2 && ratio <= 1.05 && stream_us <= 64.0 && chain_us(g) >= 0.6 * stream_us;
+      if (row_bytes % 128 == 0) narrow = es == 2 ? less || held_up : less && chain >= 0.4;
+      else if (gated) narrow = direction == QSSM_FORWARD && (less || held_up) && chain >= 1.0;
+      else if (row_bytes % 32 == 0) narrow = less && chain >= 1.2 && (es == 2 || row_bytes % 64 == 0);
+      else narrow = less && chain >= 1.0 && es == 2 && direction == QSSM_FORWARD;
       if (narrow) g >>= 1;
     }
     // And of 128 bytes where the chain would still set the pace of a backward: bf16 B=1 L=21625 D=256 51 -> 35 us, L=17098 42
     // -> 32, L=16384 D=640 58 -> 56; forward they lose (L=16384 D=640 33 -> 37), and so do rows off 128-byte lines (L=10729
     // D=880 59 -> 73).
-    if (!fixed_g && es == 2 && vec < 8 && direction == QSSM_BACKWARD && g * vec * es == 256 && g > 1 && (int64_t)D * es % 128 == 0 &&
+    if (!fixed_g && es == 2 && vec < 8 && direction == QSSM_BACKWARD && g * vec * es == 256 && g > 1 && row_bytes % 128 == 0 &&
         chain_us(g) > 1.2 * stream_us)
       g >>= 1;
     // Very short sequences: widen the rows instead of idling most time groups of a workgroup.
@@ -507,8 +521,6 @@ static int plan_scan(int32_t B, int32_t L, int32_t D, int32_t in_dtype, int32_t 
     cluster = 1 << (tune_r - 1);
   } else if (plan->n_seg > 1) {
     static const double kMapCost[2][6] = {{-0.02, 0.0, 0.02, 0.035, 0.15, 0.40}, {-0.02, 0.0, -0.005, 0.14, 0.30, 0.35}};
-    const double hop_us = direction == QSSM_FORWARD ? 2.1 : 1.8;
-    const double stream_us = (double)B * L * D * (direction == QSSM_FORWARD ? 4 * es + os : 8 * es + os) / 5.6e6;
     double best = 0.0;
     cluster = 0;
     // what the kernels that load operands straight into LDS need on top (16-bit storage): clusters beyond 8 must
