@@ -516,10 +516,11 @@ QSSM_API int qssm_gemm_f32(const qssm_gemm_f32_call* call, void* stream);
 QSSM_API int qssm_gemm_f32_splits(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t segments);
 
 /*
- * The same product with scratch for a copy of its smaller operand in parts (6 bytes per element), which makes large ones a
- * quarter faster.  qssm_gemm_f32_packed_plan sets `splits` to the number that suits the call and `*bytes` to the scratch
- * (`packed`, 16-byte aligned) that qssm_gemm_f32_packed then wants; the shapes, the layouts and the operands' addresses are
- * set before it.  `*bytes` = 0: the call is one for qssm_gemm_f32 (small, or M or N within a tile of 2^31).
+ * The same product with scratch for a copy of its smaller operand in parts (6 bytes per element, rows rounded up to 256 and
+ * k's to 32), which makes large ones a quarter faster.  qssm_gemm_f32_packed_plan sets `splits` to the number that suits the
+ * call and `*bytes` to the scratch (`packed`, 16-byte aligned) that qssm_gemm_f32_packed then wants, at most twice what the
+ * operands take; the shapes, the layouts and the operands' addresses are set before it.  `*bytes` = 0: the call is one for
+ * qssm_gemm_f32 (small, narrow, or M or N within a tile of 2^31).
  */
 QSSM_API int qssm_gemm_f32_packed_plan(qssm_gemm_f32_call* call, uint64_t* bytes);
 QSSM_API int qssm_gemm_f32_packed(const qssm_gemm_f32_call* call, void* packed, uint64_t bytes, void* stream);

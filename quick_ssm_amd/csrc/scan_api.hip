@@ -1125,7 +1125,9 @@ static int distinct(const float* const* v, int n) {
 // Which operand of a call is packed, into how many parts its k's are dealt and how many bytes the packed operand takes.
 // One workgroup per compute unit: us of a stage of 32 k's, of a tile's start and end, of 2^20 packed elements and of the
 // parts' way through memory.  (600 rows, gradient of five 1024 -> 4096: the rows fill their tiles of 128 to 94 % and tiles of
-// 256 to 78 %, so the weights are packed although they are more.)
+// 256 to 78 %, so the weights are packed although they are more.)  The rows that pad a narrow operand to 256 are not counted:
+// a few columns in few parts leave the other kernel's GPU emptier than this estimate of it says (131072 rows, 40 x 200 180 us
+// packed and 199 not; 16384 rows 51 and 43).
 struct PackedChoice {
   bool swap;
   int many, splits;
@@ -1167,7 +1169,12 @@ int qssm_gemm_f32_packed_plan(qssm_gemm_f32_call* k, uint64_t* bytes) {
     return 0;
   const PackedChoice c = packed_choice(k);
   const int plain = qssm_gemm_f32_splits(k->M, k->N, k->K, k->batch, k->segments);
-  if (!packed_fits(k, c) || gemm_cost(k->M, k->N, k->K, k->batch, k->segments, plain) <= c.cost) {
+  // No more scratch than twice the operands: narrow ones are padded to 256 rows (64 x 64 over 262144 rows 403 MB for operands
+  // of 134 MB, to gain 380 -> 347 us); whole rows take 1.5 times the packed operand.
+  const int pairs = k->batch > k->segments ? k->batch : k->segments;
+  const int a_many = k->segments > 1 ? pairs : distinct(k->a, pairs), b_many = k->segments > 1 ? pairs : distinct(k->b, pairs);
+  const uint64_t operands = ((uint64_t)k->M * a_many + (uint64_t)k->N * b_many) * k->K * sizeof(float);
+  if (c.bytes > 2 * operands || !packed_fits(k, c) || gemm_cost(k->M, k->N, k->K, k->batch, k->segments, plain) <= c.cost) {
     k->splits = plain;
     return 0;
   }

@@ -60,3 +60,17 @@ def test_three_bf16_parts_hold_every_bit_and_six_products_all_but_the_last():
     kept = sum(pa[i].double() * pb[j].double() for i, j in ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1), (0, 0)))
     exact = a.double() * b.double()
     assert bool(((kept - exact).abs() <= 2.0 ** -24 * exact.abs()).all())
+
+
+@pytest.mark.parametrize("n,k,many", [(8, 8, 1), (64, 64, 1), (80, 16, 1), (320, 64, 1), (64, 64, 5), (128, 128, 1), (640, 128, 1), (96, 96, 5)])
+def test_scratch_for_a_packed_operand_is_bounded_by_the_operands(n, k, many):
+    # Weight gradients [n, k] over many rows: an operand is packed in whole tiles of 256 columns, however narrow it is.
+    lib = _lib.load()
+    nbytes = ctypes.c_uint64()
+    for rows in (8192, 32768, 262144, 1 << 20, 1 << 24):
+        call = _Call(M=n, N=k, K=rows, lda=n, ldb=k, ldc=k, batch=many, segments=1, splits=1, a_kstrided=1, b_kstrided=1)
+        for i in range(many):
+            call.a[i], call.b[i], call.c[i] = 4096 * (2 + i), 4096, 8192
+        _lib.check(lib.qssm_gemm_f32_packed_plan(ctypes.byref(call), ctypes.byref(nbytes)))
+        assert nbytes.value <= 2 * 4 * rows * (n * many + k)
+        assert 1 <= call.splits <= 64 and call.splits * n * k * many * 4 <= max(1 << 22, 4 * rows * (n * many + k))

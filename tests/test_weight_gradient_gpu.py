@@ -85,3 +85,19 @@ def test_a_layer_takes_them_and_nothing_else_changes(gpu, monkeypatch, params, c
     assert native.weight_gradient(g, u.double()) is None
     if params != torch.float32:
         assert native.weight_gradient(g[:4096], u[:4096]) is None
+
+
+@pytest.mark.parametrize("n,k,taken", [(16, 16, False), (400, 16, False), (16, 400, False), (20, 20, True), (100, 20, True), (64, 64, True)])
+def test_narrow_fp32_gradients(gpu, n, k, taken):
+    native = hip_scan._native or hip_scan._load_native()
+    gen = torch.Generator(device=gpu).manual_seed(n)
+    rows = 40000
+    g, u = (torch.empty(rows, c, device=gpu).normal_(generator=gen) for c in (n, k))
+    assert (native.weight_gradient(g, u) is not None) == taken
+    free = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = layers._weight_gradient(g, u).double()
+    if taken:   # the operand's copy (twice the operands at most) and sums of up to 64 parts
+        assert torch.cuda.max_memory_allocated() - free <= 2 * 4 * rows * (n + k) + 65 * 4 * n * k + (1 << 20)
+    ref, size = g.double().t().contiguous() @ u.double(), g.double().abs().t().contiguous() @ u.double().abs()
+    assert bool(((got - ref).abs() <= 2.0 ** -24 * (2 * rows + 8) * size).all())
