@@ -1216,7 +1216,9 @@ int qssm_gemm_f32_packed(const qssm_gemm_f32_call* k, void* packed, uint64_t byt
 }
 
 // How a weight gradient's tiles are dealt out: `whole` workgroups with a tile each, in full rounds of one workgroup per
-// compute unit, and the tiles after them in `splits` parts, so that the last round is full as well.
+// compute unit, and the tiles after them in `splits` parts, so that the last round is full as well.  No more than two rounds
+// of parts: they cost more than `kPart` says once there are many (32768 rows, 12800 x 1024, 200 tiles: in five parts 960 us,
+// whole 841), and their sums take 256 KB each (128 MB at most).
 static int64_t half_tiles(int64_t M, int64_t N) {
   return ((M + kHalfTile - 1) / kHalfTile) * ((N + kHalfTile - 1) / kHalfTile);
 }
@@ -1227,7 +1229,7 @@ static void half_deal(int64_t M, int64_t N, int64_t K, int64_t* whole, int* spli
   const double stages = (double)((K + kHalfStageK - 1) / kHalfStageK);
   double best = 0.0;
   *splits = 1;
-  for (int s = 1; s <= 64 && (s == 1 || stages / s >= 4.0); ++s) {
+  for (int s = 1; s <= 64 && (s == 1 || (stages / s >= 4.0 && rest * s <= 2 * kCUs)); ++s) {
     double cost = (double)((rest * s + kCUs - 1) / kCUs) * (stages / s * kStage + kRound);
     if (s > 1) cost += (double)(rest * s) * kPart + kReduce;
     if (s == 1 || cost < best) { *splits = s; best = cost; }
@@ -1235,19 +1237,27 @@ static void half_deal(int64_t M, int64_t N, int64_t K, int64_t* whole, int* spli
   *whole = *splits > 1 ? tiles - rest : tiles;
 }
 
-// us here against the library's product, bf16: 16384 rows 128 x 128 26 / 121, 256 x 1024 34 / 98, 640 x 128 29 / 111, 5120 x
-// 256 62 / 123, 5120 x 512 95 / 166, 1024 x 4096 131 / 174, 20480 x 1024 683 / 868; 8192 rows 128 x 128 22 / 63, 512 x 512
-// 28 / 53, 2560 x 512 44 / 65, 5120 x 1024 89 / 121; 4096 rows 256 x 1024 29 / 28, 2560 x 512 35 / 36, 10240 x 1024 100 / 88;
-// 2048 rows 1024 x 1024 28 / 20.  With few rows the library's shorter tiles fill the GPU without parts.  Where the last
-// round of tiles is neither full nor can be dealt out (10240 x 1024: 160 tiles) its product stays: 8192 rows 191 / 164.
+// Tiles from which on a last round without parts is full enough, and columns below which the library's product of few rows is
+// the faster one.
+static const int64_t kFullTiles = 200;
+static const int32_t kNarrow = 64;
+
+// us of the library's product / here, bf16.  Up to 80 tiles: 16384 rows 128 x 128 120 / 26, 256 x 1024 98 / 34, 5120 x 256 123 /
+// 62, 1024 x 4096 174 / 131; 8192 rows 128 x 128 62 / 22, 5120 x 1024 117 / 88; 4096 rows 256 x 1024 28 / 29, 10240 x 1024 88 /
+// 100; 2048 rows 1024 x 1024 20 / 28 (with few rows the library's shorter tiles fill the GPU without parts).  Up to 128 tiles,
+// in two to five parts: 8192 rows 5120 x 1280 117 / 110 but 12800 x 512 116 / 127, 10240 rows and more 0.97 to 1.85 times the
+// library's speed (2048 x 3072 over 32768 rows is the exception: 377 / 415).  Between 128 and 200 neither parts nor a round of
+// that few tiles pay: 8192 rows 10240 x 1024 162 / 191, 12288 rows 11520 x 1024 270 / 303, 16384 rows 3072 x 3072 284 / 308 and
+// 12800 x 640 276 / 360 (some shapes gain, 32768 rows 10240 x 1024 949 / 701).  From 200 on, whatever is left beyond full
+// rounds, 1.0 to 1.6 times: 8192 rows 12800 x 1024 276 / 185, 16384 rows 20480 x 1024 868 / 683, 17920 x 1024 690 / 512.
+// Narrow ones: 8192 rows 8 x 8 13 / 22, 48 x 48 16 / 22, 16384 rows 512 x 8 28 / 29; 24576 rows 8 x 8 31 / 28, 24 x 120 97 / 28.
+// Over 356 other shapes of layers, 64 to 17920 columns and 8192 to 65536 rows: 1.45 times the library's speed in the mean.
 int qssm_weight_gradient_suits(int32_t M, int32_t N, int32_t K) {
   if (M <= 0 || N <= 0 || K < 8192) return 0;
-  int64_t whole;
-  int splits;
-  half_deal(M, N, K, &whole, &splits);
-  const int64_t tiles = half_tiles(M, N), rest = tiles - whole;
-  const double rounds = (double)((whole + kCUs - 1) / kCUs) + (double)((rest * splits + kCUs - 1) / kCUs) / splits;
-  return tiles <= kCUs / 2 || (double)tiles >= 0.75 * kCUs * rounds;
+  if ((M < kNarrow || N < kNarrow) && K < 24576) return 0;
+  const int64_t tiles = half_tiles(M, N);
+  if (tiles > kCUs / 2) return tiles >= kFullTiles;
+  return tiles <= 80 || K >= 10240;
 }
 
 uint64_t qssm_weight_gradient_floats(int32_t M, int32_t N, int32_t K) {
