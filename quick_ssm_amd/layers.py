@@ -58,18 +58,21 @@ def column_sum(g2: torch.Tensor) -> torch.Tensor:
 
 # Rows, or multiply-adds in fp32, from which a weight gradient is this package's own product.  Its sums are as long as there
 # are rows, and the library gives a tile of it to one workgroup, most of the GPU idle.  16 bits: the measured line is at
-# qssm_weight_gradient_suits.  fp32, us for the library's product and the packed one (csrc/gemm_split.hip): 2^32.3 (4096 rows,
-# 5120 x 256) 120 and 68, (1024 rows, 5120 x 1024) 88 and 74, (512 rows, 10240 x 1024) 89 and 86; 2^32 (4096 rows, 1024 x 1024)
-# 63 and 67; with many rows earlier: 8192 rows, 256 x 1024 55 and 46, 128 x 128 45 and 36, 16384 rows, 128 x 512 99 and 47.
+# qssm_weight_gradient_suits.  fp32, us for the library's product and for these (csrc/gemm_split.hip): 2^32.3 (4096 rows, 5120 x
+# 256) 120 and 68, (1024 rows, 5120 x 1024) 88 and 74, (512 rows, 10240 x 1024) 86 and 84; 2^32 (4096 rows, 1024 x 1024) 63 and
+# 67; with few rows a tile is all start and end and only memory counts: (128 rows, 8192 x 8192) 155 and 144, but (64 rows, 8192
+# x 16384) 193 and 213, (16 rows, 40960 x 8192) 248 and 508; with many rows earlier: 8192 rows, 256 x 1024 55 and 46, 128 x 128
+# 45 and 36, 16384 rows, 128 x 512 99 and 47 (and never below 20 columns, csrc/torch_scan.cpp).
 # (No result of a step but the gradient itself depends on its last bits, as those of split_linear.MIN_WORK do.)
-_GRADIENT_ROWS, _GRADIENT_WORK = 8192, 1 << 32
+_GRADIENT_ROWS, _GRADIENT_WORK, _GRADIENT_FEW_ROWS = 8192, 1 << 32, 128
 
 
 def _weight_gradient(g2: torch.Tensor, u2: torch.Tensor) -> torch.Tensor:
     """The gradient of a linear map's weight from its outputs' gradient and its inputs ([rows, N], [rows, K])."""
     rows, n = g2.shape
-    if ((rows >= _GRADIENT_ROWS or (g2.dtype is torch.float32 and rows * n * u2.shape[1] > _GRADIENT_WORK)) and g2.is_cuda
-            and not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or _scan_interface._followed_by_torch())):
+    if ((rows >= _GRADIENT_ROWS
+         or (rows >= _GRADIENT_FEW_ROWS and g2.dtype is torch.float32 and rows * n * u2.shape[1] > _GRADIENT_WORK))
+            and g2.is_cuda and not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or _scan_interface._followed_by_torch())):
         native = hip_scan._native or hip_scan._load_native()
         dw = native.weight_gradient(g2, u2)
         if dw is not None:

@@ -9,6 +9,21 @@ from quick_ssm_amd import SSM, _lib, hip_scan, layers
 pytestmark = pytest.mark.gpu
 
 
+class _Counted:
+    """The native module, with the weight gradients counted that it computes."""
+
+    def __init__(self, native):
+        self.native, self.taken = native, 0
+
+    def __getattr__(self, name):
+        return getattr(self.native, name)
+
+    def weight_gradient(self, g, u):
+        dw = self.native.weight_gradient(g, u)
+        self.taken += dw is not None
+        return dw
+
+
 def _launch(a, b, pad=0):
     (K, M), N = a.shape, b.shape[1]
     lib = _lib.load()
@@ -88,16 +103,32 @@ def test_a_layer_takes_them_and_nothing_else_changes(gpu, monkeypatch, params, c
 
 
 @pytest.mark.parametrize("n,k,taken", [(16, 16, False), (400, 16, False), (16, 400, False), (20, 20, True), (100, 20, True), (64, 64, True)])
-def test_narrow_fp32_gradients(gpu, n, k, taken):
-    native = hip_scan._native or hip_scan._load_native()
+def test_narrow_fp32_gradients(gpu, monkeypatch, n, k, taken):
+    counted = _Counted(hip_scan._native or hip_scan._load_native())
+    monkeypatch.setattr(hip_scan, "_native", counted)
     gen = torch.Generator(device=gpu).manual_seed(n)
     rows = 40000
     g, u = (torch.empty(rows, c, device=gpu).normal_(generator=gen) for c in (n, k))
-    assert (native.weight_gradient(g, u) is not None) == taken
-    free = torch.cuda.memory_allocated()
+    before = torch.cuda.memory_allocated()
     torch.cuda.reset_peak_memory_stats()
-    got = layers._weight_gradient(g, u).double()
+    with torch.no_grad():
+        got = layers._weight_gradient(g, u)
+    assert counted.taken == taken
     if taken:   # the operand's copy (twice the operands at most) and sums of up to 64 parts
-        assert torch.cuda.max_memory_allocated() - free <= 2 * 4 * rows * (n + k) + 65 * 4 * n * k + (1 << 20)
+        assert torch.cuda.max_memory_allocated() - before <= 2 * 4 * rows * (n + k) + 65 * 4 * n * k + (1 << 20)
     ref, size = g.double().t().contiguous() @ u.double(), g.double().abs().t().contiguous() @ u.double().abs()
-    assert bool(((got - ref).abs() <= 2.0 ** -24 * (2 * rows + 8) * size).all())
+    assert bool(((got.double() - ref).abs() <= 2.0 ** -24 * (2 * rows + 8) * size).all())
+
+
+@pytest.mark.parametrize("rows,n,k,taken", [(64, 8200, 8200, 0), (120, 6400, 6400, 0), (128, 6144, 6144, 1), (512, 4096, 2048, 0),
+                                            (512, 4096, 2052, 1)])
+def test_fp32_gradients_of_few_rows(gpu, monkeypatch, rows, n, k, taken):
+    counted = _Counted(hip_scan._native or hip_scan._load_native())
+    monkeypatch.setattr(hip_scan, "_native", counted)
+    gen = torch.Generator(device=gpu).manual_seed(rows)
+    g, u = (torch.empty(rows, c, device=gpu).normal_(generator=gen) for c in (n, k))
+    with torch.no_grad():
+        got = layers._weight_gradient(g, u)
+    assert counted.taken == taken and got.shape == (n, k)
+    ref, size = g[:, :64].double().t() @ u.double(), g[:, :64].double().abs().t() @ u.double().abs()
+    assert bool(((got[:64].double() - ref).abs() <= 2.0 ** -24 * (2 * rows + 8) * size).all())
