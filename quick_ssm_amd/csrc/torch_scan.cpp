@@ -689,7 +689,7 @@ FiveBlocks blocks_arg(PyObject* o, bool written) {
   FiveBlocks b;
   if (THPVariable_Check(o)) {
     const Tensor& wide = THPVariable_Unpack(o);
-    TORCH_CHECK_VALUE(wide.dim() == 3 && wide.size(2) % 5 == 0, "expected a [B, L, 5 S] tensor");
+    TORCH_CHECK_VALUE(wide.dim() == 3, "expected a [B, L, 5 S] tensor");   // (columns behind the last block are not touched)
     b.t.push_back(wide);
     const int64_t step = wide.size(2) / 5 * wide.element_size();
     for (int k = 0; k < 5; ++k) {

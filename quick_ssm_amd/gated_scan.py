@@ -101,7 +101,8 @@ _Blocks = Union[Sequence[Tensor], Tensor]
 
 def _shape(pre: _Blocks) -> Tuple[int, int, int, Tensor]:
     if isinstance(pre, Tensor):
-        return pre.shape[0], pre.shape[1], pre.shape[2] // 5, pre
+        B, L, W = pre.shape
+        return B, L, W // 5, pre
     return (*pre[0].shape, pre[0])
 
 
@@ -193,6 +194,8 @@ class _GatedScanWide(torch.autograd.Function):
                 (dwide,) = torch.autograd.grad((a, x, c, b), (leaf,), (da, dx, dc, db))
                 return dwide, None, None
         dwide = torch.empty_like(wide, memory_format=torch.contiguous_format)
+        if wide.shape[2] % 5:   # columns behind the last block are nobody's
+            dwide[..., wide.shape[2] // 5 * 5:].zero_()
         _backward_launch(wide, ctx.compute_dtype, grad_y, ckpt, ctx.stride, dwide)
         return dwide, None, None
 

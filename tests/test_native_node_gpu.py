@@ -136,3 +136,18 @@ def test_a_wide_tensor_and_its_five_blocks_are_the_same_launch(gpu, dtype, compu
         odd = torch.empty(2, 5, 5 * width + 16, device=gpu, dtype=dtype)[..., at:at + 5 * width]
         five = [odd[..., k * width:(k + 1) * width] for k in range(5)]
         assert gated_scan.supported_wide(odd, compute, dtype) == gated_scan.supported(five, compute, dtype), (width, at)
+
+
+def test_a_wide_tensor_that_is_more_than_five_blocks(gpu):
+    # four columns behind the last block
+    from quick_ssm_amd import gated_scan
+
+    gen = torch.Generator(device=gpu).manual_seed(2)
+    rows = torch.empty(2, 70, 684, device=gpu).normal_(generator=gen)
+    wide, five = (rows[..., :n].detach().requires_grad_(True) for n in (684, 680))
+    got, want = (gated_scan.gated_scan_wide(t, compute_dtype=torch.float16) for t in (wide, five))
+    assert torch.equal(got, want)
+    (dwide,), (dfive,) = torch.autograd.grad(got.sum(), wide), torch.autograd.grad(want.sum(), five)
+    assert dwide.shape == wide.shape and torch.equal(dwide[..., :680], dfive) and not dwide[..., 680:].any()
+    with pytest.raises(ValueError):
+        gated_scan.gated_scan_wide(rows[0])
