@@ -188,6 +188,21 @@ def is_built() -> bool:
     return LIB_PATH.exists() and NATIVE_PATH.exists()
 
 
+# What the extension module offers (csrc/torch_scan.cpp).
+NATIVE_FUNCTIONS = (
+    "set_hooks", "scan_forward", "scan_backward", "attach_scan", "split_forward", "split_backward", "weight_gradient",
+    "gated_forward", "gated_backward", "rmsnorm_forward", "rmsnorm_backward", "column_sum",
+)
+
+
+def _require_all(built, names, path) -> None:
+    """The version says whether argument lists agree, not whether everything added since is there."""
+    missing = [name for name in names if not hasattr(built, name)]
+    if missing:
+        raise RuntimeError(f"{path} is older than this package: it lacks {', '.join(missing)}. "
+                           "Rebuild with `python -m quick_ssm_amd.build`.")
+
+
 def load() -> ctypes.CDLL:
     """Load the shared library (once).  Raises RuntimeError if it has not been built."""
     global _lib
@@ -207,6 +222,7 @@ def load() -> ctypes.CDLL:
                 raise RuntimeError(
                     f"{LIB_PATH} was built from version {built} of the C ABI, this package binds version "
                     f"{QSSM_VERSION}: the argument lists differ. Rebuild with `python -m quick_ssm_amd.build`.")
+            _require_all(lib, EXPORTED_SYMBOLS, LIB_PATH)
             _declare(lib)
             _lib = lib
     return _lib
@@ -234,6 +250,7 @@ def load_native(take_launch):
             if module.abi_version // 100 != QSSM_VERSION // 100:
                 raise RuntimeError(f"{NATIVE_PATH} was built for version {module.abi_version} of the C ABI, this package "
                                    f"binds version {QSSM_VERSION}. Rebuild with `python -m quick_ssm_amd.build`.")
+            _require_all(module, NATIVE_FUNCTIONS, NATIVE_PATH)
             module.set_hooks(take_launch, check)
             Node.register(module.HipScanBackward)   # torch knows its own node types by name, others by registration
             sys.modules[name] = module

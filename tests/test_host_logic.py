@@ -546,3 +546,19 @@ def test_packed_projection_parameters_stay_the_reference_parameters():
     g = torch.randn_like(out)
     for got, want in zip(torch.autograd.grad(out, wrt, g), torch.autograd.grad(ref, wrt, g)):
         assert torch.allclose(got, want, rtol=1e-12, atol=1e-12)
+
+
+def test_a_build_without_the_newer_functions_is_refused(hip_lib):
+    # same minor version, so only what is missing tells that the file is stale
+    class Stale:
+        abi_version = _lib.QSSM_VERSION
+
+    for name in _lib.NATIVE_FUNCTIONS[:6]:
+        setattr(Stale, name, None)
+    with pytest.raises(RuntimeError, match="weight_gradient.*column_sum.*Rebuild"):
+        _lib._require_all(Stale, _lib.NATIVE_FUNCTIONS, _lib.NATIVE_PATH)
+    _lib._require_all(hip_lib, _lib.EXPORTED_SYMBOLS, _lib.LIB_PATH)
+    native = hip_scan._native or hip_scan._load_native()
+    _lib._require_all(native, _lib.NATIVE_FUNCTIONS, _lib.NATIVE_PATH)
+    offered = {n for n in dir(native) if callable(getattr(native, n)) and n[0].islower()}
+    assert offered == set(_lib.NATIVE_FUNCTIONS)
