@@ -74,18 +74,23 @@ def test_infinities_and_nan_stay_where_they_belong(gpu):
                                                  (torch.float32, torch.bfloat16, 8192)], ids=str)
 def test_a_layer_takes_them_and_nothing_else_changes(gpu, monkeypatch, params, compute, rows):
     native = hip_scan._native or hip_scan._load_native()
+    counted = _Counted(native)
+    monkeypatch.setattr(hip_scan, "_native", counted)
     torch.manual_seed(0)
     layer = SSM(128, 2, device=gpu, dtype=params, compute_dtype=compute)
     x = torch.randn(8, rows // 8, 128, device=gpu, dtype=params, requires_grad=True)
     dy = torch.randn_like(x)
 
     def step():
+        counted.taken = 0
         return torch.autograd.grad(layer(x), [x, *layer.parameters()], dy)
 
     got = step()
+    assert counted.taken == 2   # the five projections' and out_proj's
     monkeypatch.setattr(layers, "_GRADIENT_ROWS", 1 << 40)
     monkeypatch.setattr(layers, "_GRADIENT_WORK", 1 << 60)
     want = step()
+    assert counted.taken == 0
     for (name, _), g, w in zip([("x", x), *layer.named_parameters()], got, want):
         if name.endswith("weight") and "norm" not in name:
             assert g.dtype == w.dtype and (g.double() - w.double()).norm() <= (2e-6 if params == torch.float32 else 4e-3) * w.double().norm()
