@@ -42,8 +42,10 @@ def _run(call, packed, splits, gpu):
     torch.cuda.synchronize()
 
 
-# tiles of 128 x 256 and stages of 32: one below, on and above the edges; N > M packs A instead of B
-SHAPES = [(128, 256, 32), (129, 260, 36), (127, 252, 28), (384, 64, 64), (64, 384, 96), (1, 4, 4), (300, 1024, 260), (260, 512, 31)]
+# tiles of 128 x 256 and stages of 32: one below, on and above the edges; N > M packs A instead of B (each with whole and with
+# ragged stages)
+SHAPES = [(128, 256, 32), (129, 260, 36), (127, 252, 28), (384, 64, 64), (64, 384, 96), (1, 4, 4), (300, 1024, 260), (260, 512, 31),
+          (384, 64, 44), (640, 260, 99)]
 
 
 @pytest.mark.parametrize("packed", [True, False])
@@ -84,7 +86,7 @@ def test_edges_match_float64(gpu, M, N, K, kind, packed):
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 3e38])
 def test_what_bf16_does_not_hold_ends_as_fp32_does_in_either_operand(gpu, value):
     gen = torch.Generator(device=gpu).manual_seed(1)
-    for M, N in ((300, 520), (520, 300)):   # B packed, A packed
+    for M, N in ((300, 520), (520, 300)):   # A packed, B packed
         for which in range(2):
             a, b = (torch.empty(n, 64, device=gpu).normal_(generator=gen) for n in (M, N))
             (a, b)[which][70, 9] = value
