@@ -393,9 +393,11 @@ struct ScanBackward : public Node {
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)t.get_device()).stream(); }
 
-Tensor matrix(int64_t rows, int64_t cols, const Tensor& like) {
-  return at::empty({rows, cols}, like.options().memory_format(c10::nullopt).requires_grad(c10::nullopt));
+Tensor like_of(std::initializer_list<int64_t> sizes, const Tensor& like, at::ScalarType type) {
+  return at::empty(at::IntArrayRef(sizes), like.options().dtype(type).memory_format(c10::nullopt).requires_grad(c10::nullopt));
 }
+
+Tensor matrix(int64_t rows, int64_t cols, const Tensor& like) { return like_of({rows, cols}, like, like.scalar_type()); }
 
 // c[i] = a[i] b[i]^T (+ bias[i]), or c[0] = the sum of them all.
 void product(const std::vector<Tensor>& a, const std::vector<Tensor>& b, const std::vector<Tensor>& c, int64_t K,
@@ -419,7 +421,7 @@ void product(const std::vector<Tensor>& a, const std::vector<Tensor>& b, const s
   k.b_kstrided = b_kstrided;
   uint64_t bytes = 0;
   check_rc(qssm_gemm_f32_packed_plan(&k, &bytes));
-  const Tensor packed = at::empty({(int64_t)bytes}, c[0].options().dtype(at::kByte));
+  const Tensor packed = like_of({(int64_t)bytes}, c[0], at::kByte);
   if (k.splits > 1) {
     partial = matrix((int64_t)k.splits * batch * k.M, k.N, c[0]);
     k.partial = partial.mutable_data_ptr<float>();
@@ -661,7 +663,7 @@ PyObject* py_weight_gradient(PyObject*, PyObject* const* args, Py_ssize_t n) {
       dw = matrix(N, K, u);
       const uint64_t floats = qssm_weight_gradient_floats((int32_t)N, (int32_t)K, (int32_t)rows);
       Tensor partial;
-      if (floats > 0) partial = at::empty({(int64_t)floats}, u.options().dtype(at::kFloat).requires_grad(c10::nullopt));
+      if (floats > 0) partial = like_of({(int64_t)floats}, u, at::kFloat);
       unlocked([&] {
         return qssm_weight_gradient(g.const_data_ptr(), g.stride(0), u.const_data_ptr(), u.stride(0), dw.mutable_data_ptr(),
                                     dw.stride(0), (int32_t)N, (int32_t)K, (int32_t)rows, type == at::kHalf ? QSSM_F16 : QSSM_BF16,
@@ -742,14 +744,14 @@ const qssm_plan* plan_arg(PyObject* o) {
   return (const qssm_plan*)(uintptr_t)v;
 }
 
-// (unused, plan's address, projection outputs: five or one wide, y, ckpt, control ...) -> return code
+// (plan's address, projection outputs: five or one wide, y, ckpt, control ...) -> return code
 PyObject* py_gated_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  want_args(n, 11);
-  const qssm_plan* plan = plan_arg(args[1]);
-  const FiveBlocks pre = blocks_arg(args[2], false);
-  const Tensor &y = tensor_arg(args[3]), &ckpt = tensor_arg(args[4]);
-  const Taken to(args + 5);
+  want_args(n, 10);
+  const qssm_plan* plan = plan_arg(args[0]);
+  const FiveBlocks pre = blocks_arg(args[1], false);
+  const Tensor &y = tensor_arg(args[2]), &ckpt = tensor_arg(args[3]);
+  const Taken to(args + 4);
   const qssm_strides sy = strides3(y);
   void* yp = y.mutable_data_ptr();
   float* cp = ckpt.mutable_data_ptr<float>();
@@ -764,14 +766,14 @@ PyObject* py_gated_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// (unused, plan's address, projection outputs, dy, ckpt, gradients: five or one wide, control ...) -> return code
+// (plan's address, projection outputs, dy, ckpt, gradients: five or one wide, control ...) -> return code
 PyObject* py_gated_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  want_args(n, 12);
-  const qssm_plan* plan = plan_arg(args[1]);
-  const FiveBlocks pre = blocks_arg(args[2], false), grad = blocks_arg(args[5], true);
-  const Tensor &dy = tensor_arg(args[3]), &ckpt = tensor_arg(args[4]);
-  const Taken to(args + 6);
+  want_args(n, 11);
+  const qssm_plan* plan = plan_arg(args[0]);
+  const FiveBlocks pre = blocks_arg(args[1], false), grad = blocks_arg(args[4], true);
+  const Tensor &dy = tensor_arg(args[2]), &ckpt = tensor_arg(args[3]);
+  const Taken to(args + 5);
   const qssm_strides sdy = strides3(dy);
   const void* dyp = dy.const_data_ptr();
   const float* cp = ckpt.const_data_ptr<float>();
@@ -787,10 +789,6 @@ PyObject* py_gated_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   return PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
-}
-
-Tensor like_of(std::initializer_list<int64_t> sizes, const Tensor& like, at::ScalarType type) {
-  return at::empty(at::IntArrayRef(sizes), like.options().dtype(type).memory_format(c10::nullopt).requires_grad(c10::nullopt));
 }
 
 int64_t row_stride(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : t.size(1); }

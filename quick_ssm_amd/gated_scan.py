@@ -91,7 +91,7 @@ def _plan(B: int, L: int, S: int, dtype: torch.dtype, compute_dtype: torch.dtype
 def _launch(plan: Plan, dev: torch.device, fn, *args) -> None:
     with _lib.launch_stream(dev) as stream:
         taken, epoch, capturing = hip_scan._launch_buffers(dev, dev.index, stream, plan.control_bytes, plan.workspace_bytes)
-        _lib.check(fn(ctypes.byref(plan), *args, *taken[3:], epoch, stream))
+        _lib.check(fn(ctypes.addressof(plan), *args, *taken[3:], epoch, stream))
         hip_scan._after_launch(taken, stream, capturing)
 
 
@@ -118,7 +118,7 @@ def _forward_launch(pre: _Blocks, compute_dtype: torch.dtype, out_dtype: torch.d
     y = torch.empty((B, L, S), dtype=out_dtype, device=dev)
     ckpt = torch.empty((B, plan.n_ckpt, S), dtype=torch.float32, device=dev)
     native = hip_scan._native or hip_scan._load_native()
-    _launch(plan, dev, native.gated_forward, ctypes.addressof(plan), pre, y, ckpt)
+    _launch(plan, dev, native.gated_forward, pre, y, ckpt)
     return y, ckpt, int(plan.ckpt_stride)
 
 
@@ -135,7 +135,7 @@ def _backward_launch(pre: _Blocks, compute_dtype: torch.dtype, grad_y: Tensor, c
     dtype = t0.dtype
     plan = _plan(B, L, S, dtype, compute_dtype, dtype, _lib.QSSM_BACKWARD, stride, True)
     native = hip_scan._native or hip_scan._load_native()
-    _launch(plan, t0.device, native.gated_backward, ctypes.addressof(plan), pre, grad_y, ckpt, grads)
+    _launch(plan, t0.device, native.gated_backward, pre, grad_y, ckpt, grads)
 
 
 class _GatedScanFunction(torch.autograd.Function):
@@ -227,8 +227,8 @@ def gated_scan(A_pre: Tensor, B_in: Tensor, Ca: Tensor, Cb: Tensor, D_pre: Tenso
 
 def gated_scan_wide(wide: Tensor, *, out_dtype: Optional[torch.dtype] = None,
                     compute_dtype: Optional[torch.dtype] = None) -> Tensor:
-    """`gated_scan` on one [B, L, 5 S] tensor holding A_pre, B_in, Ca, Cb, D_pre side by side; call `supported()` on
-    its five blocks first."""
+    """`gated_scan` on one [B, L, 5 S] tensor holding A_pre, B_in, Ca, Cb, D_pre side by side; call `supported_wide()`
+    first."""
     return _GatedScanWide.apply(wide, out_dtype or wide.dtype, compute_dtype or wide.dtype)
 
 
