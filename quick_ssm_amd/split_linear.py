@@ -28,6 +28,11 @@ MIN_WORK = 1 << 33
 # 64 -> 2560 would be two.  At 128 columns the library's 109 us stand against 97, at 208 -> 4160 357 against 244.
 MIN_INFERENCE_WIDTH = 128
 
+# Below 256 columns the outputs (of all weights) have to fill their tiles as well: 1572869 rows, 128 -> 128 546 against 587,
+# 2139100 rows, 128 -> 32 338 against 558, 118843 rows, 144 -> 512 176 against 183; from 1024 outputs on 1.0 to 2.2 times the
+# library's speed.
+_NARROW, _NARROW_OUTPUTS = 256, 1024
+
 # Most rows and outputs: the kernel counts to the end of its last tile of 128 in 32 bits.
 MAX_ROWS = (1 << 31) - 1 - 128
 
@@ -45,7 +50,9 @@ def usable(u: Tensor, weights: Sequence[Tensor], gradients: bool = True) -> bool
         return False
     if not u.is_cuda or torch.is_autocast_enabled("cuda") or n % 4 or k % 4:
         return False
-    if u.numel() // k > MAX_ROWS or n > MAX_ROWS or (k < MIN_INFERENCE_WIDTH and not gradients):
+    if u.numel() // k > MAX_ROWS or n > MAX_ROWS:
+        return False
+    if not gradients and (k < MIN_INFERENCE_WIDTH or (k < _NARROW and n * len(weights) < _NARROW_OUTPUTS)):
         return False
     if not _matrix_ok(u.reshape(-1, k)):
         return False

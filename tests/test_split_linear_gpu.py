@@ -100,3 +100,13 @@ def test_a_layer_takes_them_and_repeats_bit_for_bit(gpu, monkeypatch):
     for got, want in zip(first, step()):
         # the gates round to fp16, so a product's last bit may move an operand by 2^-11
         assert _error(got, want.double()) < 2e-3
+
+
+@pytest.mark.parametrize("k,n,count,gradients,taken", [
+    (128, 32, 1, False, False), (144, 192, 5, False, False), (128, 256, 5, False, True), (144, 1024, 1, False, True),
+    (124, 4096, 5, False, False), (256, 32, 1, False, True), (128, 32, 1, True, True), (124, 64, 5, True, True)])
+def test_narrow_inputs_and_outputs_stay_with_the_library_in_inference(gpu, k, n, count, gradients, taken):
+    rows = split_linear.MIN_WORK // (k * n * count) + 1
+    u, ws = torch.empty(rows, k, device=gpu), [torch.empty(n, k, device=gpu) for _ in range(count)]
+    assert split_linear.usable(u, ws, gradients) == taken
+    assert not split_linear.usable(u[:rows // 2], ws, gradients)
