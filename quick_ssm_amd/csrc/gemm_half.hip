@@ -69,7 +69,7 @@ __device__ __forceinline__ Place place(const HalfGemmArgs& p, int tile) {
 //
 // What it is for are long sums into few tiles: the rows of a batch are k here, and a weight has 4 to 320 tiles.  The tiles
 // beyond full rounds of one workgroup per compute unit are dealt out in parts of their k's (qssm_weight_gradient).  16384
-// rows, library -> here: 20480 x 1024 868 -> 683 us, 1024 x 4096 174 -> 131, 5120 x 256 121 -> 59, 256 x 1024 97 -> 33.
+// rows, library -> here: 20480 x 1024 866 -> 566 us, 1024 x 4096 165 -> 121, 5120 x 256 120 -> 58, 256 x 1024 95 -> 32.
 template <typename T, bool RAGGED>
 __global__ void __launch_bounds__(512, 2) half_gemm_kernel(const HalfGemmArgs p) {
   __shared__ __align__(16) char lds[2 * kStage];

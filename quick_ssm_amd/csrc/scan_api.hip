@@ -1249,7 +1249,7 @@ static const int32_t kNarrow = 64;
 // library's speed (2048 x 3072 over 32768 rows is the exception: 377 / 415).  Between 128 and 200 neither parts nor a round of
 // that few tiles pay: 8192 rows 10240 x 1024 162 / 191, 12288 rows 11520 x 1024 270 / 303, 16384 rows 3072 x 3072 284 / 308 and
 // 12800 x 640 276 / 360 (some shapes gain, 32768 rows 10240 x 1024 949 / 701).  From 200 on, whatever is left beyond full
-// rounds, 1.0 to 1.6 times: 8192 rows 12800 x 1024 276 / 185, 16384 rows 20480 x 1024 868 / 683, 17920 x 1024 690 / 512.
+// rounds, 1.0 to 1.6 times: 8192 rows 12800 x 1024 276 / 185, 16384 rows 20480 x 1024 866 / 566, 17920 x 1024 690 / 512.
 // Narrow ones: 8192 rows 8 x 8 13 / 22, 48 x 48 16 / 22, 16384 rows 512 x 8 28 / 29; 24576 rows 8 x 8 31 / 28, 24 x 120 97 / 28.
 // Over 356 other shapes of layers, 64 to 17920 columns and 8192 to 65536 rows: 1.45 times the library's speed in the mean.
 int qssm_weight_gradient_suits(int32_t M, int32_t N, int32_t K) {

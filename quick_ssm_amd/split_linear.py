@@ -21,7 +21,8 @@ Tensor = torch.Tensor
 # and weight gradient, library against these: 2^30 (4096 rows, 1024 -> 256) 24, 25, 30 against 41, 33, 42; 2^32.3 (4096 rows,
 # 256 -> 5120) 103, 95, 133 against 83, 66, 69; 2^33.3 (4096 rows, 512 -> 5120) 168, 154, 171 against 130, 113, 115.  They
 # cross near 2^31; the line is above the copy task's stack (2^32.3 a layer), whose six layers in fp16 carry a difference in a
-# product's last bits on to 3e-3 of a gradient: at that size every program's results stay those of the library's products.
+# product's last bits on to 3e-3 of a gradient: at that size outputs and input gradients stay the library's products.  (Weight
+# gradients, on which nothing else in a step depends, are this package's from layers._GRADIENT_WORK on.)
 MIN_WORK = 1 << 33
 
 # An input narrower than this has few stages to fill a tile's pipeline with before its results are stored: 16384 rows,
